@@ -243,7 +243,7 @@ size_t fg_sample_workspace(int rows);
  * greedy or temperature == 0: argmax (first maximum). top_k <= 0: off.
  * top_p_fixed = floor(top_p * 2^32), 0 = off. workspace (optional, >= fg_sample_workspace(rows)
  * bytes): unrestricted and greedy draws then run split over several workgroups per row;
- * results are identical either way. */
+ * results are identical either way (greedy, unrestricted, top-p and top-k up to 4096). */
 int fg_sample_tokens(const void* logits, int dtype, int64_t row_stride, int rows, int vocab,
                      const int32_t* row_index, const int32_t* forced, const uint32_t* noise, int noise_stride,
                      int noise_col, uint64_t seed, uint64_t step, const int32_t* seq_ids, int draw,
@@ -253,7 +253,7 @@ int fg_sample_tokens(const void* logits, int dtype, int64_t row_stride, int rows
 /* fg_sample_tokens without a workspace argument and without any allocation. No
  * counterpart in the reference: it is for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * The split partials live in a static device array of the library (9.1 MB per GPU,
+ * The split partials live in a static device array of the library (17.5 MB per GPU,
  * held until the process ends) that holds rows <= fg_sample_tokens_noalloc_max_rows()
  * (256); more rows are rejected with an error. Same arguments, rule and tokens as
  * fg_sample_tokens with a large enough workspace. Every call on one GPU shares that
@@ -289,9 +289,8 @@ int fg_accept_walk(const void* tree_logits, int dtype, int64_t row_stride, int v
  *                     (noise column noise_col0 + walk_step, counter draw draw0 + walk_step).
  * After the walk, state[2*batch + b] is the step whose logits row b last sampled (-1: none).
  * fg_walk_step's workspace is optional, as for fg_sample_tokens (rows = batch). With a
- * workspace, an unrestricted or greedy step whose row maxima parts are given (part_max /
- * part_key [batch, nparts], as fg_lm_head_topk writes them with the step's logits) skips
- * the chunk-maxima launch. next_row_index / next_row_active (optional): the step also writes the next
+ * workspace, a step whose row maxima parts are given (part_max / part_key [batch, nparts],
+ * as fg_lm_head_topk writes them with the step's logits) skips the chunk-maxima launch. next_row_index / next_row_active (optional): the step also writes the next
  * step's rows, as fg_walk_rows would (rows that are already inactive keep their entries). */
 int fg_walk_begin(const int32_t* tree_tokens, const int32_t* parents, const int32_t* n_nodes, int nmax, int batch,
                   int32_t* acc_tokens, int32_t* acc_nodes, int acc_stride, int32_t* acc_len, int32_t* last_node,

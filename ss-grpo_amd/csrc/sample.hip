@@ -22,6 +22,7 @@
 // 16-byte loads) per step. Top-k / top-p use an MSB-first 4 x 8-bit radix
 // select over the keys with count or q-weighted histograms in LDS.
 #include <mutex>
+#include <type_traits>
 
 #include "fg_common.h"
 
@@ -468,19 +469,15 @@ struct SplitArgs {
   const uint64_t* src_key;
   int src_parts;
   int64_t src_stride;
-  // split top-p (see "split top-p")
+  // restricted draws (see "split top-k / top-p")
+  int top_k;
   uint32_t tp32;
-  uint64_t* hist;            // [rows, kSplitChunks, 256] chunk histograms of one radix level
-  struct SelState* sel;      // [rows, 2] select state, double-buffered across levels
-  uint64_t* part_a;          // [rows, kSplitChunks] q-mass of keys above the cut key
-  uint64_t* part_t;          // [rows, kSplitChunks] q-mass of keys equal to it
-};
-
-// Radix select state of one row: the selected key bits so far, the q-mass of
-// keys above them, and the top-p target mass.
-struct SelState {
-  uint32_t prefix, pmask;
-  uint64_t above, target;
+  uint64_t* hist;            // [rows, kSplitChunks, 256] chunk histograms (q-mass or counts)
+  struct SelState* sel;      // [rows]
+  uint64_t* part_a;          // [rows, kSplitChunks] q-mass above the cut's bin
+  int32_t* part_nan;         // [rows, kSplitChunks] NaN count
+  uint32_t* list;            // [rows, kSelList] indices of the elements around the cut
+  int32_t* list_n;           // [rows] listed elements (may exceed kSelList: then not all are there)
 };
 
 template <int DT>
@@ -586,13 +583,6 @@ __global__ void __launch_bounds__(kSplitThreads) split_max_kernel(SplitArgs a) {
     a.part_max[r * kSplitChunks + c] = fmaxf(smax[0], mx);
     a.part_key[r * kSplitChunks + c] = skey[0] > best ? skey[0] : best;
   }
-}
-
-// Row maximum from the chunk maxima.
-FG_DEVICE float split_row_max(const SplitArgs& a, int r) {
-  float mx = -INFINITY;
-  for (int c = 0; c < kSplitChunks; ++c) mx = fmaxf(mx, a.part_max[r * kSplitChunks + c]);
-  return mx;
 }
 
 FG_DEVICE float split_kt(const SplitArgs& a) { return fg::weight_kt(a.scale != 0, a.temperature); }
@@ -846,170 +836,340 @@ __global__ void __launch_bounds__(kSplitThreads) split_pick_kernel(SplitArgs a, 
   }
 }
 
-// ------------------------------------------------------------------ split top-p
-// Top-p draws (no top-k) over kSplitChunks workgroups per row, the same integer
-// rule as block_sample / radix_select: (1) chunk maxima (split_max_kernel);
-// (2) four launches of one 8-bit radix level each over the scaled-logit keys: every
-// chunk workgroup first merges the previous level's 16 chunk histograms (all of a
-// row's workgroups reach the same digit; chunk 0 records the state) and then
-// histograms its chunk's q-mass under the new prefix -- the first merge also yields
-// the row's q total and the target floor(total * tp32 / 2^32); (3) the last merge
-// fixes the cut key; each chunk sums the q-mass above it and tied with it;
-// (4) one workgroup per row resolves the ties in index order, then locates the
-// draw among the kept tokens in vocabulary order (chunk by chunk partial sums).
+// ------------------------------------------------------------------ split top-k / top-p
+// Restricted draws over kSplitChunks workgroups per row, four launches, the same integer rule
+// as block_sample:
+//  (1) chunk maxima (split_max_kernel), unless the row's maxima parts are given;
+//  (2) per chunk, a 256-bin histogram over the fixed-point exponent a (fg_common.h), 8 bins
+//      per octave below the row maximum: q-mass for top-p, counts for top-k. a never grows
+//      with x, so the bins are runs of the candidate order; elements of weight 0 are in no bin;
+//  (3) each chunk merges the row's 16 histograms, finds the bin that holds the cut and appends
+//      the indices of its own elements of that bin (top-k: of that bin and the ones above) to
+//      the row's list;
+//  (4) one workgroup per row selects the cut exactly among the list (64-bit rank keys, so ties
+//      resolve in index order) and locates the draw: top-k among the list, top-p in the one
+//      chunk whose running kept mass crosses the target.
+// A row whose list overflows (flat rows), whose total is 0 or whose top-k slots are all taken by
+// NaN is drawn by block_sample in launch (4).
+//
+// Bound by VALU and LDS issue of the two weighing passes. An 8-bit radix select over the key
+// bits needed four histogram launches instead of one: the first level's 256 bins are the sign
+// and exponent bits, so nearly every LDS atomic hit the same few words (17 us per level at
+// 64 x 152,064), and a bf16 row's last two levels had nothing left to separate. Measured, a draw:
+// top-p 0.95 at 64 x 152,064 bf16 114 -> 57 us (seven launches before); top-k 50 at
+// 32 x 151,936 bf16 210 -> 47 us (one workgroup per row before).
+constexpr int kSelBins = 256;
+constexpr int kSelBinShift = 17;             // 2^17 steps of a: 8 bins per octave
+constexpr uint32_t kSelAMax = 40u << 20;     // larger a weigh 0
+constexpr int kSelList = 8192;               // list entries per row
+constexpr int kSelTopK = 4096;               // largest top_k the list path takes
+static_assert(kSelBins == kSplitThreads, "one histogram bin per thread");
 
-// Calls f(i, s, key) for the elements of chunk c of row r (8 per thread per step).
-template <int DT, class F>
-FG_DEVICE void for_chunk(const SplitArgs& a, int r, int c, F&& f) {
+// Where the cut of one row lies (written by chunk 0 of launch 3).
+struct SelState {
+  uint64_t rest;  // position of the cut within the list: q-mass (top-p) or count (top-k) before it
+  int32_t slow;   // the row is drawn by block_sample
+  int32_t all;    // every listed element is kept (top-k with no more candidates than slots)
+};
+
+FG_DEVICE uint32_t fixed_exponent(float m, float x, float kt) {
+#pragma clang fp contract(off)
+  return (uint32_t)fminf((m - x) * kt, fg::kWeightZmax);
+}
+FG_DEVICE int sel_bin(uint32_t a) { return min((int)(a >> kSelBinShift), kSelBins - 1); }
+
+template <int DT, bool COUNT>
+__global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) {
+  const int c = blockIdx.x, r = blockIdx.y, tid = threadIdx.x;
+  if (split_skip(a, r)) return;
+  using Bin = std::conditional_t<COUNT, uint32_t, uint64_t>;
+  using AtomicBin = std::conditional_t<COUNT, unsigned int, unsigned long long>;
+  __shared__ uint64_t tbl[COUNT ? 1 : 1024];
+  __shared__ Bin h[kSplitWaves][kSelBins];  // one copy per wave: fewer waves meet on a word
+  __shared__ float smax[kSplitWaves];
+  __shared__ int s_nan;
   const char* p = split_row<DT>(a, r);
   const int lo = c * a.chunk, hi = min(a.vocab, lo + a.chunk);
-  for (int i0 = lo + threadIdx.x * 8; i0 < hi; i0 += kSplitThreads * 8) {
-    float x[8];
-    if (i0 + 8 <= hi) {
-      fg::load8<DT>(p, i0, x);
-    } else {
+  float x[kSplitLoads][8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = i0 + j < hi ? fg::load_elem<DT>(p, i0 + j) : 0.0f;
+  for (int u = 0; u < kSplitLoads; ++u)
+    if (split_group_live(lo, u, hi)) split_load8<DT>(p, lo + (u * kSplitThreads + tid) * 8, hi, x[u]);
+  if constexpr (!COUNT) fg::exp2_table_to_lds(tbl);
+#pragma unroll
+  for (int w = 0; w < kSplitWaves; ++w) h[w][tid] = 0;
+  if (tid == 0) s_nan = 0;
+  float mx = -INFINITY;  // row maximum from the parts
+  for (int q = tid; q < a.src_parts; q += kSplitThreads) mx = fmaxf(mx, a.src_max[r * a.src_stride + q]);
+  mx = fg::wave_max(mx);
+  if ((tid & 63) == 0) smax[tid >> 6] = mx;
+  __syncthreads();
+  mx = smax[0];
+#pragma unroll
+  for (int w = 1; w < kSplitWaves; ++w) mx = fmaxf(mx, smax[w]);
+  const float m = mx, kt = split_kt(a);
+  Bin* mine = h[tid >> 6];
+  int nan = 0;
+  for (int base = lo; base < hi; base += kSplitPass) {
+    if (base != lo) {
+#pragma unroll
+      for (int u = 0; u < kSplitLoads; ++u)
+        if (split_group_live(base, u, hi)) split_load8<DT>(p, base + (u * kSplitThreads + tid) * 8, hi, x[u]);
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (i0 + j < hi) {
-        f(i0 + j, x[j], fg::sort_key32(x[j]));
+    for (int u = 0; u < kSplitLoads; ++u) {
+      if (!split_group_live(base, u, hi)) continue;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t e = fixed_exponent(m, x[u][j], kt);
+        if constexpr (COUNT) nan += x[u][j] != x[u][j];
+        if (e <= kSelAMax) {
+          const Bin w = COUNT ? (Bin)1 : (Bin)fg::weight_q40(m, x[u][j], kt, tbl);
+          atomicAdd((AtomicBin*)&mine[sel_bin(e)], (AtomicBin)w);
+        }
       }
+    }
+  }
+  if constexpr (COUNT) {
+    if (nan) atomicAdd(&s_nan, nan);
+  }
+  __syncthreads();
+  Bin t = 0;
+#pragma unroll
+  for (int w = 0; w < kSplitWaves; ++w) t += h[w][tid];
+  a.hist[((size_t)r * kSplitChunks + c) * kSelBins + tid] = t;
+  if (tid == 0) {
+    if constexpr (COUNT) a.part_nan[r * kSplitChunks + c] = s_nan;
+    if (c == 0) {
+      a.list_n[r] = 0;
+      a.row_m[r] = m;
+    }
   }
 }
 
-// Sum of v over the workgroup (kSplitThreads threads).
-FG_DEVICE uint64_t split_block_sum(uint64_t v, uint64_t* red) {
+// Inclusive sum of v over the workgroup's threads in order, and its total.
+FG_DEVICE uint64_t split_incl_scan(uint64_t v, uint64_t* wsum, uint64_t& total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t incl = fg::wave_incl_scan_u64(v);
+  __syncthreads();  // wsum of an earlier scan has been read
+  if (lane == 63) wsum[wave] = incl;
+  __syncthreads();
+  uint64_t off = 0;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < kSplitWaves; ++w) {
+    if (w < wave) off += wsum[w];
+    total += wsum[w];
+  }
+  return off + incl;
+}
+
+template <int DT, bool COUNT>
+__global__ void __launch_bounds__(kSplitThreads) split_gather_kernel(SplitArgs a) {
+  const int c = blockIdx.x, r = blockIdx.y, tid = threadIdx.x;
+  if (split_skip(a, r)) return;
+  __shared__ uint64_t wsum[kSplitWaves];
+  __shared__ int s_bin, s_base;
+  __shared__ uint64_t s_before;
+  const char* p = split_row<DT>(a, r);
+  const int lo = c * a.chunk, hi = min(a.vocab, lo + a.chunk);
+  float x[kSplitLoads][8];
+#pragma unroll
+  for (int u = 0; u < kSplitLoads; ++u)
+    if (split_group_live(lo, u, hi)) split_load8<DT>(p, lo + (u * kSplitThreads + tid) * 8, hi, x[u]);
+  const uint64_t* hp = a.hist + (size_t)r * kSplitChunks * kSelBins;
+  uint64_t v = 0, own = 0;
+#pragma unroll
+  for (int q = 0; q < kSplitChunks; ++q) {
+    const uint64_t w = hp[q * kSelBins + tid];
+    v += w;
+    own = q == c ? w : own;
+  }
+  uint64_t total;
+  const uint64_t incl = split_incl_scan(v, wsum, total);
+  // the cut is the candidate position whose running sum first exceeds target
+  uint64_t target = 0;
+  bool slow = total == 0, all = false;
+  if constexpr (COUNT) {
+    uint64_t nan = 0;  // NaN ranks first and takes slots
+    for (int q = 0; q < kSplitChunks; ++q) nan += (uint64_t)a.part_nan[r * kSplitChunks + q];
+    slow |= (uint64_t)a.top_k <= nan;
+    const uint64_t slots = slow ? 1 : (uint64_t)a.top_k - nan;
+    all = total <= slots;
+    target = all ? (total ? total - 1 : 0) : slots - 1;
+  } else {
+    target = fg::mulhi_u64_u32(total, a.tp32);
+  }
+  if (tid == 0) s_bin = kSelBins - 1;
+  __syncthreads();
+  if (incl - v <= target && target < incl) {  // one thread, unless the total is 0
+    s_bin = tid;
+    s_before = incl - v;
+  }
+  __syncthreads();
+  const int bin = s_bin;
+  if (c == 0 && tid == 0) a.sel[r] = SelState{slow ? 0 : COUNT ? target : target - s_before, slow, all};
+  if (slow) return;
+  if constexpr (!COUNT) {  // this chunk's q-mass above the cut's bin
+    uint64_t above;
+    split_incl_scan(tid < bin ? own : 0, wsum, above);
+    if (tid == 0) a.part_a[r * kSplitChunks + c] = above;
+  }
+  const float m = a.row_m[r], kt = split_kt(a);
+  uint32_t* list = a.list + (size_t)r * kSelList;
+  const auto listed = [&](float xv) {
+    const uint32_t e = fixed_exponent(m, xv, kt);
+    return e <= kSelAMax && (COUNT ? sel_bin(e) <= bin : sel_bin(e) == bin);
+  };
+  for (int base = lo; base < hi; base += kSplitPass) {
+    if (base != lo) {
+#pragma unroll
+      for (int u = 0; u < kSplitLoads; ++u)
+        if (split_group_live(base, u, hi)) split_load8<DT>(p, base + (u * kSplitThreads + tid) * 8, hi, x[u]);
+    }
+    uint64_t hit = 0;  // bit 8 u + j: element j of group u is listed
+#pragma unroll
+    for (int u = 0; u < kSplitLoads; ++u) {
+      if (!split_group_live(base, u, hi)) continue;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (listed(x[u][j])) hit |= 1ull << (8 * u + j);
+    }
+    uint64_t count;
+    const int at = (int)split_incl_scan((uint64_t)__popcll(hit), wsum, count) - __popcll(hit);
+    if (tid == 0 && count) s_base = atomicAdd(&a.list_n[r], (int)count);
+    __syncthreads();
+    int o = s_base + at;
+    while (hit) {
+      const int bit = __builtin_ctzll(hit);
+      hit &= hit - 1;
+      if (o < kSelList) list[o] = (uint32_t)(base + ((bit >> 3) * kSplitThreads + tid) * 8 + (bit & 7));
+      ++o;
+    }
+  }
+}
+
+// Largest-first selection over the keys ck[0, n) >= cut (whole block of kThreads; the keys are
+// distinct): the key at which the running count, or the running q-mass of the logit that a key
+// holds, first exceeds target. LOW orders by the low word alone (index ascending). The caller
+// guarantees that the total exceeds target. Radix select from the highest differing bit, 8
+// bits a level, ending early where one key is left.
+struct SelectShared {
+  uint64_t hist[256];
+  uint32_t cnt[256];
+  uint64_t wred[kWaves];
+  uint64_t above, found;
+  int digit;
+};
+
+template <bool MASS, bool LOW>
+FG_DEVICE uint64_t list_select(const uint64_t* ck, int n, uint64_t cut, uint64_t target, float m, float kt,
+                               const uint64_t* tbl, SelectShared& sh) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const auto value = [](uint64_t k) { return LOW ? (k & 0xffffffffull) : k; };
+  // bits in which the considered keys differ
+  uint64_t ones = 0, zeros = 0;
+  for (int i = tid; i < n; i += kThreads)
+    if (ck[i] >= cut) {
+      ones |= value(ck[i]);
+      zeros |= ~value(ck[i]);
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    ones |= fg::shfl_xor_u64(ones, o);
+    zeros |= fg::shfl_xor_u64(zeros, o);
+  }
+  __syncthreads();  // sh is free
+  if (lane == 0) {
+    sh.wred[tid >> 6] = ones;
+    sh.hist[tid >> 6] = zeros;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    ones |= sh.wred[w];
+    zeros |= sh.hist[w];
+  }
+  const uint64_t diff = ones & zeros;
+  if (diff == 0) return value(ones);  // one key
+  int shift = max(0, 56 - __builtin_clzll(diff));
+  // the chosen bits so far: the ones above the highest differing bit are common to all
+  uint64_t fixed = shift + 8 >= 64 ? 0ull : ~0ull << (shift + 8);
+  uint64_t prefix = ones & fixed, above = 0;
+  for (;;) {
+    __syncthreads();
+    if (tid < 256) {
+      sh.hist[tid] = 0;
+      sh.cnt[tid] = 0;
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += kThreads) {
+      const uint64_t k = ck[i], v = value(k);
+      if (k >= cut && (v & fixed) == prefix) {
+        const int d = (int)(v >> shift) & 255;
+        atomicAdd(&sh.cnt[d], 1u);
+        if constexpr (MASS)
+          atomicAdd((unsigned long long*)&sh.hist[d],
+                    (unsigned long long)fg::weight_q40(m, fg::rank_key_value(k), kt, tbl));
+      }
+    }
+    __syncthreads();
+    if (tid < 64) {  // lane l owns digits 255 - 4 l .. 252 - 4 l
+      uint64_t h[4], mine = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int d = 255 - 4 * lane - j;
+        h[j] = MASS ? sh.hist[d] : (uint64_t)sh.cnt[d];
+        mine += h[j];
+      }
+      const uint64_t incl = fg::wave_incl_scan_u64(mine), excl = incl - mine;
+      if (above + excl <= target && target < above + incl) {
+        uint64_t c = above + excl;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (c + h[j] > target) {
+            sh.digit = 255 - 4 * lane - j;
+            sh.above = c;
+            break;
+          }
+          c += h[j];
+        }
+      }
+    }
+    __syncthreads();
+    above = sh.above;
+    prefix |= (uint64_t)sh.digit << shift;
+    fixed |= 255ull << shift;
+    if (sh.cnt[sh.digit] == 1) {
+      for (int i = tid; i < n; i += kThreads)
+        if (ck[i] >= cut && (value(ck[i]) & fixed) == prefix) sh.found = value(ck[i]);
+      __syncthreads();
+      return sh.found;
+    }
+    if (shift == 0) return prefix;
+    shift = max(0, shift - 8);
+  }
+}
+
+// Sum over the block (kThreads) of v.
+FG_DEVICE uint64_t select_block_sum(uint64_t v, SelectShared& sh) {
   v = fg::wave_sum_u64(v);
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  if ((threadIdx.x & 63) == 0) sh.wred[threadIdx.x >> 6] = v;
   __syncthreads();
   uint64_t t = 0;
 #pragma unroll
-  for (int w = 0; w < kSplitThreads / 64; ++w) t += red[w];
+  for (int w = 0; w < kWaves; ++w) t += sh.wred[w];
   return t;
 }
 
-// Merges the 16 chunk histograms of the level at `shift` into st (radix_select's
-// digit rule); level 0's merge first sets the top-p target from the row total.
-FG_DEVICE void split_merge_level(const SplitArgs& a, int r, int shift, bool first, SelState& st, uint64_t* hs,
-                                 uint64_t* red, int* sdig, uint64_t* sabove) {
-  const uint64_t* hp = a.hist + (size_t)r * kSplitChunks * 256;
-  uint64_t v = 0;
-  for (int c = 0; c < kSplitChunks; ++c) v += hp[c * 256 + threadIdx.x];
-  hs[threadIdx.x] = v;
-  if (first) st.target = fg::mulhi_u64_u32(split_block_sum(v, red), a.tp32);
-  if (threadIdx.x == 0) {
-    *sdig = 0;  // no digit holds the target only when the row total is 0 (then the draw is the argmax)
-    *sabove = st.above;
+// Elements of a row at or above a cut rank key, for block_sum / block_locate over a chunk that
+// starts at vocabulary index lo.
+struct KeptFrom {
+  uint64_t cut;
+  uint32_t lo;
+  FG_DEVICE bool operator()(uint32_t key, uint32_t i) const {
+    return (((uint64_t)key << 32) | (uint64_t)(0xffffffffu - (lo + i))) >= cut;
   }
-  __syncthreads();
-  if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
-    uint64_t h[4], mine = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      h[j] = hs[255 - 4 * lane - j];
-      mine += h[j];
-    }
-    const uint64_t incl = fg::wave_incl_scan_u64(mine);
-    const uint64_t excl = incl - mine;
-    if (st.above + excl <= st.target && st.target < st.above + incl) {
-      uint64_t c = st.above + excl;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (c + h[j] > st.target) {
-          *sdig = 255 - 4 * lane - j;
-          *sabove = c;
-          break;
-        }
-        c += h[j];
-      }
-    }
-  }
-  __syncthreads();
-  st.prefix |= (uint32_t)*sdig << shift;
-  st.pmask |= 255u << shift;
-  st.above = *sabove;
-}
-
-// One radix level (level 0..3, digit bits 31-8l .. 24-8l): merge the previous
-// level, then this chunk's q-mass histogram under the prefix.
-template <int DT>
-__global__ void __launch_bounds__(kSplitThreads) split_topp_level_kernel(SplitArgs a, int level) {
-  const int c = blockIdx.x, r = blockIdx.y;
-  if (split_skip(a, r)) return;
-  __shared__ uint64_t tbl[1024];
-  __shared__ uint64_t hs[256];
-  __shared__ uint64_t red[kSplitThreads / 64];
-  __shared__ int sdig;
-  __shared__ uint64_t sabove;
-  fg::exp2_table_to_lds(tbl);  // visible after the barriers below
-  SelState st{0u, 0u, 0ull, 0ull};
-  if (level >= 2) st = a.sel[r * 2 + ((level - 2) & 1)];
-  if (level >= 1) {
-    split_merge_level(a, r, 24 - 8 * (level - 1), level == 1, st, hs, red, &sdig, &sabove);
-    if (c == 0 && threadIdx.x == 0) a.sel[r * 2 + ((level - 1) & 1)] = st;
-  }
-  const float m = split_row_max(a, r), kt = split_kt(a);
-  const int shift = 24 - 8 * level;
-  __syncthreads();
-  hs[threadIdx.x] = 0;
-  __syncthreads();
-  for_chunk<DT>(a, r, c, [&](int, float sv, uint32_t key) {
-    if ((key & st.pmask) == st.prefix)
-      atomicAdd((unsigned long long*)&hs[(key >> shift) & 255u],
-                (unsigned long long)fg::weight_q40(m, sv, kt, tbl));
-  });
-  __syncthreads();
-  a.hist[((size_t)r * kSplitChunks + c) * 256 + threadIdx.x] = hs[threadIdx.x];
-}
-
-// Last merge (the cut key), then this chunk's q-mass above the cut key and tied with it.
-template <int DT>
-__global__ void __launch_bounds__(kSplitThreads) split_topp_cut_kernel(SplitArgs a) {
-  const int c = blockIdx.x, r = blockIdx.y;
-  if (split_skip(a, r)) return;
-  __shared__ uint64_t tbl[1024];
-  __shared__ uint64_t hs[256];
-  __shared__ uint64_t red[kSplitThreads / 64];
-  __shared__ int sdig;
-  __shared__ uint64_t sabove;
-  fg::exp2_table_to_lds(tbl);  // visible after the barriers of the merge
-  SelState st = a.sel[r * 2 + 0];  // after level 2
-  split_merge_level(a, r, 0, false, st, hs, red, &sdig, &sabove);
-  if (c == 0 && threadIdx.x == 0) a.sel[r * 2 + 1] = st;
-  const float m = split_row_max(a, r), kt = split_kt(a);
-  const uint32_t kappa = st.prefix;
-  uint64_t above = 0, tie = 0;
-  for_chunk<DT>(a, r, c, [&](int, float sv, uint32_t key) {
-    if (key >= kappa) {
-      const uint64_t w = fg::weight_q40(m, sv, kt, tbl);
-      if (key > kappa) above += w;
-      else tie += w;
-    }
-  });
-  above = split_block_sum(above, red);
-  tie = split_block_sum(tie, red);
-  if (threadIdx.x == 0) {
-    a.part_a[r * kSplitChunks + c] = above;
-    a.part_t[r * kSplitChunks + c] = tie;
-  }
-}
-
-// Chunk-relative predicates for the pick (element index i is relative to chunk start lo).
-struct TieAt {
-  uint32_t kappa;
-  FG_DEVICE bool operator()(uint32_t key, uint32_t) const { return key == kappa; }
-};
-struct TieUpTo {
-  uint32_t kappa, last_rel;
-  FG_DEVICE bool operator()(uint32_t key, uint32_t i) const { return key == kappa && i <= last_rel; }
-};
-struct KeptIn {
-  uint32_t kappa, last, lo;
-  FG_DEVICE bool operator()(uint32_t key, uint32_t i) const { return key > kappa || (key == kappa && lo + i <= last); }
 };
 
 template <int DT>
@@ -1021,114 +1181,116 @@ FG_DEVICE Row<DT> chunk_row(const SplitArgs& a, int r, int c, const uint64_t* tb
   rr.seg = (((rr.V + kWaves - 1) / kWaves) + kStep - 1) / kStep * kStep;
   rr.kt = split_kt(a);
   rr.tbl = tbl;
-  rr.m = split_row_max(a, r);
+  rr.m = a.row_m[r];
   return rr;
 }
 
-// The token of row r (whole block; every thread returns it).
-template <int DT>
-FG_DEVICE int split_topp_pick(const SplitArgs& a, int r, uint32_t u, Shared& sh) {
-  fg::exp2_table_to_lds(sh.exp2);  // visible after the first barrier of block_sum
-  const SelState st = a.sel[r * 2 + 1];
-  const uint32_t kappa = st.prefix;
-  const uint64_t* pa = a.part_a + r * kSplitChunks;
-  const uint64_t* pt = a.part_t + r * kSplitChunks;
-  const uint64_t need = st.target - st.above;
-  // ties on the cut key are kept in index order up to the one whose running mass exceeds `need`
-  uint64_t tb = 0;
-  int cs = -1;
-  for (int c = 0; c < kSplitChunks; ++c) {
-    if (tb + pt[c] > need) {
-      cs = c;
-      break;
+template <int DT, bool COUNT, bool WALK>
+__global__ void __launch_bounds__(kThreads) split_select_kernel(SplitArgs a, DrawOut d, SampleParams sp) {
+  __shared__ Shared sh;
+  __shared__ SelectShared sel;
+  __shared__ uint64_t ck[kSelList];
+  __shared__ unsigned long long s_kept[kSplitChunks];
+  const int r = blockIdx.x, tid = threadIdx.x;
+  if constexpr (WALK) {
+    if (!d.state[d.batch + r]) return;
+  } else {
+    if (a.forced && a.forced[r] >= 0) {
+      if (tid == 0) d.out[r] = a.forced[r];
+      return;
     }
-    tb += pt[c];
   }
-  uint32_t last = 0xffffffffu;
-  uint64_t tie_cs = 0;  // tie mass kept in chunk cs
-  if (cs >= 0) {
-    const Row<DT> rr = chunk_row<DT>(a, r, cs, sh.exp2);
-    block_sum<true, DT>(rr, TieAt{kappa}, sh);
-    const int idx = block_locate<true, DT>(rr, TieAt{kappa}, need - tb, sh);
-    if (idx >= 0) {
-      last = (uint32_t)(cs * a.chunk + idx);
-      tie_cs = block_sum<true, DT>(rr, TieUpTo{kappa, (uint32_t)idx}, sh);
+  const uint32_t seq = d.seq_ids ? (uint32_t)d.seq_ids[r] : (uint32_t)r;
+  const int ws = WALK ? d.walk_step : 0;
+  const uint32_t u = noise_value(d.noise, (int64_t)r * d.noise_stride + d.noise_col + ws, d.seed, d.step, seq,
+                                 (uint32_t)(d.draw + ws));
+  const SelState st = a.sel[r];
+  const int n = a.list_n[r];
+  const char* rowp = split_row<DT>(a, r);
+  int tok;
+  if (st.slow || n > kSelList) {
+    tok = block_sample<DT>(rowp, a.vocab, sp, u, sh);
+  } else {
+    const float m = a.row_m[r], kt = split_kt(a);
+    for (int i = tid; i < n; i += kThreads) {
+      const uint32_t idx = a.list[(size_t)r * kSelList + i];
+      ck[i] = fg::rank_key(fg::load_elem<DT>(rowp, idx), idx);
+    }
+    fg::exp2_table_to_lds(sh.exp2);
+    if (tid < kSplitChunks) s_kept[tid] = 0;
+    __syncthreads();
+    const auto weight = [&](uint64_t k) { return fg::weight_q40(m, fg::rank_key_value(k), kt, sh.exp2); };
+    if constexpr (COUNT) {
+      uint64_t cut = 0, kept = 0;
+      if (!st.all) cut = list_select<false, false>(ck, n, 0, st.rest, m, kt, sh.exp2, sel);
+      for (int i = tid; i < n; i += kThreads)
+        if (ck[i] >= cut) kept += weight(ck[i]);
+      uint64_t total = select_block_sum(kept, sel);
+      if (sp.tp32) {
+        cut = list_select<true, false>(ck, n, cut, fg::mulhi_u64_u32(total, sp.tp32), m, kt, sh.exp2, sel);
+        kept = 0;
+        for (int i = tid; i < n; i += kThreads)
+          if (ck[i] >= cut) kept += weight(ck[i]);
+        total = select_block_sum(kept, sel);
+      }
+      const uint64_t low = list_select<true, true>(ck, n, cut, fg::mulhi_u64_u32(total, u), m, kt, sh.exp2, sel);
+      tok = (int)fg::rank_key_index(low);
     } else {
-      cs = -1;  // cannot happen: chunk cs holds the crossing tie
+      const uint64_t cut = list_select<true, false>(ck, n, 0, st.rest, m, kt, sh.exp2, sel);
+      for (int i = tid; i < n; i += kThreads)
+        if (ck[i] >= cut)
+          atomicAdd(&s_kept[fg::rank_key_index(ck[i]) / (uint32_t)a.chunk], (unsigned long long)weight(ck[i]));
+      __syncthreads();
+      uint64_t total = 0;
+      for (int c = 0; c < kSplitChunks; ++c) total += a.part_a[r * kSplitChunks + c] + s_kept[c];
+      const uint64_t target = fg::mulhi_u64_u32(total, u);
+      uint64_t before = 0;
+      int c2 = kSplitChunks - 1;
+      for (int c = 0; c < kSplitChunks; ++c) {
+        const uint64_t kc = a.part_a[r * kSplitChunks + c] + s_kept[c];
+        if (before + kc > target) {
+          c2 = c;
+          break;
+        }
+        before += kc;
+      }
+      const Row<DT> rr = chunk_row<DT>(a, r, c2, sh.exp2);
+      const KeptFrom kept{cut, (uint32_t)(c2 * a.chunk)};
+      block_sum<true, DT>(rr, kept, sh);
+      tok = c2 * a.chunk + block_locate<true, DT>(rr, kept, target - before, sh);
     }
   }
-  uint64_t total = 0;
-  for (int c = 0; c < kSplitChunks; ++c)
-    total += pa[c] + (cs < 0 || c < cs ? pt[c] : (c == cs ? tie_cs : 0ull));
-  uint64_t best = 0;
-  for (int c = 0; c < kSplitChunks; ++c) {
-    const uint64_t k = a.part_key[r * kSplitChunks + c];
-    best = k > best ? k : best;
+  if constexpr (WALK) {
+    if (tid < 64)
+      walk_apply(r, tok, d.state[r], d.tree_tokens, d.parents, d.n_nodes, d.nmax, d.batch, d.walk_step, d.acc_tokens,
+                 d.acc_nodes, d.acc_stride, d.acc_len, d.last_node, d.correction, d.state, d.err_flag, d.next_rows,
+                 d.next_active);
+  } else {
+    if (tid == 0) d.out[r] = tok;
   }
-  if (total == 0) return (int)fg::rank_key_index(best);
-  const uint64_t target = fg::mulhi_u64_u32(total, u);
-  uint64_t before = 0;
-  int c2 = kSplitChunks - 1;
-  for (int c = 0; c < kSplitChunks; ++c) {
-    const uint64_t kc = pa[c] + (cs < 0 || c < cs ? pt[c] : (c == cs ? tie_cs : 0ull));
-    if (before + kc > target) {
-      c2 = c;
-      break;
-    }
-    before += kc;
-  }
-  const Row<DT> r2 = chunk_row<DT>(a, r, c2, sh.exp2);
-  const KeptIn kept{kappa, last, (uint32_t)(c2 * a.chunk)};
-  block_sum<true, DT>(r2, kept, sh);
-  const int idx = block_locate<true, DT>(r2, kept, target - before, sh);
-  return idx >= 0 ? c2 * a.chunk + idx : (int)fg::rank_key_index(best);
 }
 
-template <int DT>
-__global__ void __launch_bounds__(kThreads) split_topp_sample_kernel(SplitArgs a, const uint32_t* __restrict__ noise,
-                                                                     int noise_stride, int noise_col, uint64_t seed,
-                                                                     uint64_t step, const int32_t* __restrict__ seq_ids,
-                                                                     int draw, int32_t* __restrict__ out) {
-  __shared__ Shared sh;
-  const int r = blockIdx.x;
-  if (a.forced && a.forced[r] >= 0) {
-    if (threadIdx.x == 0) out[r] = a.forced[r];
-    return;
+template <int DT, bool COUNT, bool WALK>
+void split_select_launch(const SplitArgs& a, const DrawOut& d, const SampleParams& sp, int rows, bool with_max,
+                         hipStream_t s) {
+  const dim3 grid(kSplitChunks, rows), block(kSplitThreads);
+  if (with_max) hipLaunchKernelGGL(split_max_kernel<DT>, grid, block, 0, s, a);
+  hipLaunchKernelGGL((split_hist_kernel<DT, COUNT>), grid, block, 0, s, a);
+  hipLaunchKernelGGL((split_gather_kernel<DT, COUNT>), grid, block, 0, s, a);
+  hipLaunchKernelGGL((split_select_kernel<DT, COUNT, WALK>), dim3(rows), dim3(kThreads), 0, s, a, d, sp);
+}
+
+// A draw with a top-k and / or top-p cut.
+template <bool WALK>
+void split_select(int dtype, const SplitArgs& a, const DrawOut& d, const SampleParams& sp, int rows, bool with_max,
+                  hipStream_t s) {
+  if (dtype == fg::kBF16) {
+    if (sp.top_k) split_select_launch<fg::kBF16, true, WALK>(a, d, sp, rows, with_max, s);
+    else split_select_launch<fg::kBF16, false, WALK>(a, d, sp, rows, with_max, s);
+  } else {
+    if (sp.top_k) split_select_launch<fg::kF32, true, WALK>(a, d, sp, rows, with_max, s);
+    else split_select_launch<fg::kF32, false, WALK>(a, d, sp, rows, with_max, s);
   }
-  const uint32_t seq = seq_ids ? (uint32_t)seq_ids[r] : (uint32_t)r;
-  const uint32_t u = noise_value(noise, (int64_t)r * noise_stride + noise_col, seed, step, seq, (uint32_t)draw);
-  const int tok = split_topp_pick<DT>(a, r, u, sh);
-  if (threadIdx.x == 0) out[r] = tok;
-}
-
-template <int DT>
-__global__ void __launch_bounds__(kThreads) split_topp_walk_kernel(
-    SplitArgs a, const int32_t* __restrict__ tree_tokens, const int32_t* __restrict__ parents,
-    const int32_t* __restrict__ n_nodes, int nmax, int batch, int walk_step, const uint32_t* __restrict__ noise,
-    int noise_stride, int noise_col0, uint64_t seed, uint64_t step, const int32_t* __restrict__ seq_ids, int draw0,
-    int32_t* acc_tokens, int32_t* acc_nodes, int acc_stride, int32_t* acc_len, int32_t* last_node,
-    int32_t* correction, int32_t* state, int32_t* err_flag, int32_t* next_rows, int32_t* next_active) {
-  __shared__ Shared sh;
-  const int b = blockIdx.x;
-  if (!state[batch + b]) return;
-  const int parent = state[b];
-  const uint32_t seq = seq_ids ? (uint32_t)seq_ids[b] : (uint32_t)b;
-  const uint32_t u = noise_value(noise, (int64_t)b * noise_stride + noise_col0 + walk_step, seed, step, seq,
-                                 (uint32_t)(draw0 + walk_step));
-  const int tok = split_topp_pick<DT>(a, b, u, sh);
-  if (threadIdx.x < 64)
-    walk_apply(b, tok, parent, tree_tokens, parents, n_nodes, nmax, batch, walk_step, acc_tokens, acc_nodes,
-               acc_stride, acc_len, last_node, correction, state, err_flag, next_rows, next_active);
-}
-
-// Chunk partials of the split top-p path: max, four radix levels, the cut (6 launches).
-template <int DT>
-void split_topp_partials(const SplitArgs& a, int rows, hipStream_t s) {
-  dim3 grid(kSplitChunks, rows);
-  hipLaunchKernelGGL(split_max_kernel<DT>, grid, dim3(kSplitThreads), 0, s, a);
-  for (int level = 0; level < 4; ++level)
-    hipLaunchKernelGGL(split_topp_level_kernel<DT>, grid, dim3(kSplitThreads), 0, s, a, level);
-  hipLaunchKernelGGL(split_topp_cut_kernel<DT>, grid, dim3(kSplitThreads), 0, s, a);
 }
 
 // A split draw: the chunk maxima unless a.src_* already hold row maxima parts, the
@@ -1140,14 +1302,17 @@ void split_draw(const SplitArgs& a, const DrawOut& d, int rows, bool with_max, h
   hipLaunchKernelGGL((split_pick_kernel<DT, WALK>), dim3(rows), dim3(kSplitThreads), 0, s, a, d);
 }
 
+// Scratch of unrestricted and greedy draws, and of restricted ones on top of it.
+constexpr size_t split_base_bytes(int rows) {
+  return (size_t)rows * (kSplitChunks * (4 + 8 + 8) + (8 + 4) + kSplitChunks * kSplitMaxGroups * 8) + 256;
+}
 constexpr size_t split_workspace_bytes(int rows) {
-  return (size_t)rows * kSplitChunks * (4 + 8 + 8) + (size_t)rows * kSplitChunks * 256 * 8 +
-         (size_t)rows * 2 * sizeof(SelState) + (size_t)rows * kSplitChunks * 16 + (size_t)rows * (8 + 4) +
-         (size_t)rows * kSplitChunks * kSplitMaxGroups * 8 + 256;
+  return split_base_bytes(rows) + (size_t)rows * (kSplitChunks * (kSelBins * 8 + 8 + 4) + sizeof(SelState) +
+                                                  kSelList * 4 + 4) + 64;
 }
 
 // Scratch of fg_sample_tokens_noalloc: the split partials of up to
-// kNoAllocMaxRows rows (9.1 MB per device, held until the process ends). Each
+// kNoAllocMaxRows rows (17.5 MB per device, held until the process ends). Each
 // kernel of the split paths writes every partial it owns before a later launch
 // reads it, so nothing in it has to start at zero. Host code never hands
 // `scratch` itself to a kernel (in host code the name is only a stand-in): it
@@ -1178,33 +1343,41 @@ int scratch_for_current_device(void** out) {
   return 0;
 }
 
-// Carves the split partials out of a caller workspace; false when it is too small.
+// Carves the split partials out of a caller workspace; false when it is too small (restricted
+// draws need more than the others).
 bool split_setup(SplitArgs& a, void* workspace, size_t bytes, int rows, const void* logits, int64_t row_stride,
-                 int vocab, float temperature, int greedy) {
-  if (!workspace || bytes < split_workspace_bytes(rows)) return false;
+                 int vocab, float temperature, const SampleParams& sp) {
+  const bool cut = !sp.greedy && (sp.top_k > 0 || sp.tp32 != 0);
+  if (sp.top_k > kSelTopK && cut) return false;
+  if (!workspace || bytes < (cut ? split_workspace_bytes(rows) : split_base_bytes(rows))) return false;
   char* w = (char*)(((uintptr_t)workspace + 15) & ~(uintptr_t)15);
+  const size_t chunks = (size_t)rows * kSplitChunks;
   a.part_key = (uint64_t*)w;
-  a.part_sum = a.part_key + (size_t)rows * kSplitChunks;
-  a.hist = a.part_sum + (size_t)rows * kSplitChunks;
-  a.part_a = a.hist + (size_t)rows * kSplitChunks * 256;
-  a.part_t = a.part_a + (size_t)rows * kSplitChunks;
-  a.sel = (SelState*)(a.part_t + (size_t)rows * kSplitChunks);
-  a.row_best = (uint64_t*)(a.sel + (size_t)rows * 2);
+  a.part_sum = a.part_key + chunks;
+  a.row_best = a.part_sum + chunks;
   a.part_gsum = a.row_best + rows;
-  a.part_max = (float*)(a.part_gsum + (size_t)rows * kSplitChunks * kSplitMaxGroups);
-  a.row_m = a.part_max + (size_t)rows * kSplitChunks;
+  a.part_max = (float*)(a.part_gsum + chunks * kSplitMaxGroups);
+  a.row_m = a.part_max + chunks;
+  w = (char*)(((uintptr_t)(a.row_m + rows) + 15) & ~(uintptr_t)15);
+  a.hist = cut ? (uint64_t*)w : nullptr;
+  a.part_a = cut ? a.hist + chunks * kSelBins : nullptr;
+  a.sel = cut ? (SelState*)(a.part_a + chunks) : nullptr;
+  a.part_nan = cut ? (int32_t*)(a.sel + rows) : nullptr;
+  a.list = cut ? (uint32_t*)(a.part_nan + chunks) : nullptr;
+  a.list_n = cut ? (int32_t*)(a.list + (size_t)rows * kSelList) : nullptr;
   a.src_max = a.part_max;
   a.src_key = a.part_key;
   a.src_parts = kSplitChunks;
   a.src_stride = kSplitChunks;
-  a.tp32 = 0;
+  a.top_k = sp.top_k;
+  a.tp32 = sp.tp32;
   a.logits = logits;
   a.row_stride = row_stride;
   a.vocab = vocab;
   a.chunk = ((vocab + kSplitChunks - 1) / kSplitChunks + 7) / 8 * 8;
   a.groups = (a.chunk + kSplitGroup - 1) / kSplitGroup;
   a.temperature = temperature;
-  a.greedy = greedy || temperature == 0.0f;
+  a.greedy = sp.greedy;
   a.scale = !a.greedy && temperature > 0.0f && temperature != 1.0f;
   a.row_index = nullptr;
   a.forced = nullptr;
@@ -1264,31 +1437,15 @@ int sample_tokens_impl(const char* who, const void* logits, int dtype, int64_t r
   SampleParams sp = make_params(temperature, greedy, top_k, vocab, top_p_fixed);
   hipStream_t s = (hipStream_t)stream;
   SplitArgs a;
-  if ((sp.greedy || (sp.top_k == 0 && sp.tp32 == 0)) &&
-      split_setup(a, workspace, workspace_bytes, rows, logits, row_stride, vocab, temperature, sp.greedy)) {
+  if (split_setup(a, workspace, workspace_bytes, rows, logits, row_stride, vocab, temperature, sp)) {
     a.row_index = row_index;
     a.forced = forced;
     DrawOut d{};
     d.noise = noise; d.noise_stride = noise_stride; d.noise_col = noise_col;
     d.seed = seed; d.step = step; d.seq_ids = seq_ids; d.draw = draw; d.out = out_tokens;
-    if (dtype == fg::kBF16) split_draw<fg::kBF16, false>(a, d, rows, true, s);
+    if (!sp.greedy && (sp.top_k || sp.tp32)) split_select<false>(dtype, a, d, sp, rows, true, s);
+    else if (dtype == fg::kBF16) split_draw<fg::kBF16, false>(a, d, rows, true, s);
     else split_draw<fg::kF32, false>(a, d, rows, true, s);
-    return fg::check_launch(who);
-  }
-  if (!sp.greedy && sp.top_k == 0 && sp.tp32 != 0 &&
-      split_setup(a, workspace, workspace_bytes, rows, logits, row_stride, vocab, temperature, 0)) {
-    a.row_index = row_index;
-    a.forced = forced;
-    a.tp32 = sp.tp32;
-    if (dtype == fg::kBF16) {
-      split_topp_partials<fg::kBF16>(a, rows, s);
-      hipLaunchKernelGGL(split_topp_sample_kernel<fg::kBF16>, dim3(rows), dim3(kThreads), 0, s, a, noise,
-                         noise_stride, noise_col, seed, step, seq_ids, draw, out_tokens);
-    } else {
-      split_topp_partials<fg::kF32>(a, rows, s);
-      hipLaunchKernelGGL(split_topp_sample_kernel<fg::kF32>, dim3(rows), dim3(kThreads), 0, s, a, noise,
-                         noise_stride, noise_col, seed, step, seq_ids, draw, out_tokens);
-    }
     return fg::check_launch(who);
   }
   if (dtype == fg::kBF16)
@@ -1407,9 +1564,9 @@ int fg_walk_step(const void* step_logits, int dtype, int64_t row_stride, int voc
   SampleParams sp = make_params(temperature, greedy, top_k, vocab, top_p_fixed);
   hipStream_t s = (hipStream_t)stream;
   SplitArgs a;
-  if ((sp.greedy || (sp.top_k == 0 && sp.tp32 == 0)) &&
-      split_setup(a, workspace, workspace_bytes, batch, step_logits, row_stride, vocab, temperature, sp.greedy)) {
+  if (split_setup(a, workspace, workspace_bytes, batch, step_logits, row_stride, vocab, temperature, sp)) {
     a.active = state + batch;
+    const bool cut = !sp.greedy && (sp.top_k || sp.tp32);
     const bool with_max = part_max == nullptr;
     if (!with_max) {
       a.src_max = part_max;
@@ -1425,27 +1582,9 @@ int fg_walk_step(const void* step_logits, int dtype, int64_t row_stride, int voc
     d.acc_tokens = acc_tokens; d.acc_nodes = acc_nodes; d.acc_stride = acc_stride; d.acc_len = acc_len;
     d.last_node = last_node; d.correction = correction; d.state = state; d.err_flag = err_flag;
     d.next_rows = next_row_index; d.next_active = next_row_active;
-    if (dtype == fg::kBF16) split_draw<fg::kBF16, true>(a, d, batch, with_max, s);
+    if (cut) split_select<true>(dtype, a, d, sp, batch, with_max, s);
+    else if (dtype == fg::kBF16) split_draw<fg::kBF16, true>(a, d, batch, with_max, s);
     else split_draw<fg::kF32, true>(a, d, batch, with_max, s);
-    return fg::check_launch("fg_walk_step");
-  }
-  if (!sp.greedy && sp.top_k == 0 && sp.tp32 != 0 &&
-      split_setup(a, workspace, workspace_bytes, batch, step_logits, row_stride, vocab, temperature, 0)) {
-    a.active = state + batch;
-    a.tp32 = sp.tp32;
-    if (dtype == fg::kBF16) {
-      split_topp_partials<fg::kBF16>(a, batch, s);
-      hipLaunchKernelGGL(split_topp_walk_kernel<fg::kBF16>, dim3(batch), dim3(kThreads), 0, s, a, tree_tokens, parents,
-                         n_nodes, nmax, batch, walk_step, noise, noise_stride, noise_col0, seed, step, seq_ids, draw0,
-                         acc_tokens, acc_nodes, acc_stride, acc_len, last_node, correction, state, err_flag,
-                         next_row_index, next_row_active);
-    } else {
-      split_topp_partials<fg::kF32>(a, batch, s);
-      hipLaunchKernelGGL(split_topp_walk_kernel<fg::kF32>, dim3(batch), dim3(kThreads), 0, s, a, tree_tokens, parents,
-                         n_nodes, nmax, batch, walk_step, noise, noise_stride, noise_col0, seed, step, seq_ids, draw0,
-                         acc_tokens, acc_nodes, acc_stride, acc_len, last_node, correction, state, err_flag,
-                         next_row_index, next_row_active);
-    }
     return fg::check_launch("fg_walk_step");
   }
   if (dtype == fg::kBF16)
