@@ -146,10 +146,18 @@ __global__ void __launch_bounds__(W * 64, 2) tree_attn_bf16_kernel(AttnArgs a, i
   // read of each K/V tile served from that XCD's L2.
   int unit = blockIdx.x, mt = 0;
   if (m_tiles > 1) {
-    const int grp = blockIdx.x / (8 * m_tiles), rem = blockIdx.x % (8 * m_tiles);
-    mt = rem / 8;
-    unit = grp * 8 + rem % 8;
-    if (unit >= a.batch * a.Hkv * a.splits) return;  // grid padded to whole groups of 8 units
+    const int units8 = gridDim.x / m_tiles;  // units padded to whole groups of 8
+    if (a.anc) {
+      const int grp = blockIdx.x / (8 * m_tiles), rem = blockIdx.x % (8 * m_tiles);
+      mt = rem / 8;
+      unit = grp * 8 + rem % 8;
+    } else {
+      // A chain's later row tiles see more keys: they start first, so the last workgroups to
+      // finish are the short ones. A unit's tiles still meet on one XCD (units8 % 8 == 0).
+      mt = m_tiles - 1 - (int)blockIdx.x / units8;
+      unit = blockIdx.x % units8;
+    }
+    if (unit >= a.batch * a.Hkv * a.splits) return;
   }
   const int sp = unit % a.splits;
   const int hkv = (unit / a.splits) % a.Hkv;
@@ -160,7 +168,11 @@ __global__ void __launch_bounds__(W * 64, 2) tree_attn_bf16_kernel(AttnArgs a, i
   const int s0 = a.seq_len[b];
   // Keys past the cache's capacity were never written (fg_rope_kv_write flags them):
   // they are not attended, as in the fp32 kernel.
-  const int total = min(s0 + a.N, a.capacity);
+  // A chain's row tile sees no new key past its last row's own: the tile stops there (over a
+  // prefill chunk without prefix that is half of all tiles; a 4 x 1024-token chunk after ragged
+  // 750-1000-token prefixes, Llama-3.1-8B heads: 137.5 -> 107.7 us).
+  const int last_new = a.anc ? a.N : (min((mt + 1) * kRowsTile, M) - 1) / G + 1;
+  const int total = min(s0 + last_new, a.capacity);
   const int cb = a.row_map ? a.row_map[b] : b;
   const uint16_t* kbase = (const uint16_t*)a.k + (int64_t)cb * a.cache_batch + (int64_t)hkv * a.cache_head;
   const uint16_t* vbase = (const uint16_t*)a.v + (int64_t)cb * a.cache_batch + (int64_t)hkv * a.cache_head;
