@@ -6,8 +6,8 @@
 // bf16 path: MFMA v_mfma_f32_32x32x16_bf16 tiles, LDS double buffering, fp32
 // accumulation, XCD-aware block order (consecutive tiles of one N column
 // stripe land on the same XCD so the weight stripe is read from HBM once and
-// reused from that XCD's L2 across the M tiles). fp32 path: LDS-tiled FMA
-// kernel used by the fp32 configuration.
+// reused from that XCD's L2 across the M tiles). fp32 path: a weight stream on
+// fp32 MFMAs up to 64 rows, else an LDS-tiled FMA kernel.
 //
 // Replaces the lm_head calls of flashgrpo/decoding/flash_medusa_decoder.py:289-294,
 // 414-433, 1079-1091 and MedusaPredictionHead.project_hidden
@@ -670,6 +670,95 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(GemmArgs g, int epi) {
     for (int j = 0; j < 4; ++j) epilogue_store<CDT, fg::kF32>(g, z, m0 + ty * 4 + i, n0 + tx * 4 + j, acc[i][j], epi);
 }
 
+// fp32 rows <= 64 (the LM head of a small rollout: a weight read per launch). Each wave owns 16
+// rows of B and streams them in 128-wide k-tiles, the next tile's eight 16-byte loads per lane
+// in flight during the current one's products; A is staged per k-tile in LDS (double-buffered,
+// rows padded by 4 floats so the 16 rows of a fragment read lie on distinct banks) and shared by
+// the four waves. v_mfma_f32_16x16x4_f32 with B's rows as its first operand: fp32 products and
+// sums, and lane l holds row m = l % 16 of C with 4 consecutive columns. MFMA step e of a 32-wide
+// chunk takes k = chunk + 8 (l / 16) + e on both operands.
+// Bound by the weight bytes: 8 x 32,000 x 512 fp32 (65.5 MB) 74.1 -> 14.0 us against the
+// 64 x 64 FMA tile below, which loads 4 bytes a thread with no load in flight during its products.
+constexpr int kF32Tile = 128;
+
+template <int MB, int CDT>
+__global__ void __launch_bounds__(256) gemm_f32_rows_kernel(GemmArgs g) {
+  constexpr int ROWS = 16 * MB, XR = kF32Tile + 4, XC = ROWS * (kF32Tile / 4) / 256;
+  __shared__ __attribute__((aligned(16))) float xs[2][ROWS * XR];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, q = lane >> 4;
+  if (g.row_active && !tile_has_active_row(g, 0, g.M)) return;
+  const int n_base = blockIdx.x * 64 + wave * 16;
+  const float* wsrc = (const float*)g.B + (int64_t)min(n_base + l16, g.N - 1) * g.ldb + q * 8;
+  const float* xsrc[XC];
+  int xdst[XC];
+#pragma unroll
+  for (int c = 0; c < XC; ++c) {
+    const int idx = tid + c * 256, r = idx / (kF32Tile / 4), col = idx % (kF32Tile / 4) * 4;
+    const int m = min(r, g.M - 1);
+    xsrc[c] = (const float*)g.A + (int64_t)(g.a_rows ? g.a_rows[m] : m) * g.lda + col;
+    xdst[c] = r * XR + col;
+  }
+  floatx4 acc[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) acc[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  floatx4 w[4][2], wn[4][2], xr[XC];
+  const auto load = [&](floatx4(&wd)[4][2], int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < XC; ++c) xr[c] = *(const floatx4*)(xsrc[c] + k0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wd[c][h] = *(const floatx4*)(wsrc + k0 + c * 32 + h * 4);
+  };
+  load(w, 0);
+#pragma unroll
+  for (int c = 0; c < XC; ++c) *(floatx4*)&xs[0][xdst[c]] = xr[c];
+  const int tiles = g.K / kF32Tile;
+  for (int t = 0; t < tiles; ++t) {
+    const bool more = t + 1 < tiles;
+    if (more) load(wn, (t + 1) * kF32Tile);
+    __syncthreads();  // tile t is in LDS and every wave is done with tile t - 1
+    const float* x = xs[t & 1] + l16 * XR + q * 8;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+          const floatx4 xv = *(const floatx4*)(x + i * 16 * XR + c * 32 + h * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[c][h][e], xv[e], acc[i], 0, 0, 0);
+        }
+    if (more) {
+#pragma unroll
+      for (int c = 0; c < XC; ++c) *(floatx4*)&xs[(t + 1) & 1][xdst[c]] = xr[c];
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) w[c][h] = wn[c][h];
+    }
+  }
+  const int n = n_base + 4 * q;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) epilogue_store<CDT, fg::kF32>(g, 0, i * 16 + l16, n + e, acc[i][e], kEpiNone);
+}
+
+template <int CDT>
+void launch_f32_rows(const GemmArgs& g, hipStream_t s) {
+  const dim3 grid((g.N + 63) / 64), block(256);
+  if (g.M <= 16) hipLaunchKernelGGL((gemm_f32_rows_kernel<1, CDT>), grid, block, 0, s, g);
+  else if (g.M <= 32) hipLaunchKernelGGL((gemm_f32_rows_kernel<2, CDT>), grid, block, 0, s, g);
+  else hipLaunchKernelGGL((gemm_f32_rows_kernel<4, CDT>), grid, block, 0, s, g);
+}
+
+// Up to 64 rows without an epilogue, K a multiple of 128, 16-byte aligned rows.
+bool f32_rows_ok(const GemmArgs& g, int epi, int batch) {
+  return batch == 1 && epi == kEpiNone && g.M <= 64 && g.K % kF32Tile == 0 && g.lda % 4 == 0 && g.ldb % 4 == 0 &&
+         ((uintptr_t)g.A & 15) == 0 && ((uintptr_t)g.B & 15) == 0;
+}
+
 // fp32 Medusa block, split over K: blockIdx.z = z * ksplit + p takes k in [p * kper, (p + 1) * kper)
 // of batch z's product and writes the raw sums to parts[p][z][m][n] (64 x 64 tile, 4 x 4 outputs
 // per thread, each thread loading one 16-byte run of 4 k values of A and of B per 16-deep k-step).
@@ -833,6 +922,9 @@ int launch_gemm(const GemmArgs& g, int dtype, int out_dtype, int epi, int batch,
       else
         hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, 64, 64, fg::kF32>), grid, dim3(256), 0, s, g, epi, tm, tn);
     }
+  } else if (f32_rows_ok(g, epi, batch)) {
+    if (out_dtype == fg::kBF16) launch_f32_rows<fg::kBF16>(g, s);
+    else launch_f32_rows<fg::kF32>(g, s);
   } else {
     dim3 grid((g.N + 63) / 64, (g.M + 63) / 64, batch);
     if (out_dtype == fg::kBF16)
