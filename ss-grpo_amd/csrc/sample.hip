@@ -13,7 +13,9 @@
 //   order) whose inclusive q prefix exceeds target.
 // Integer sums make every result independent of reduction order.
 //
-// Unrestricted and greedy draws with a workspace run split over 16 chunks per
+// Rows of up to 65,536 logits are drawn in one launch by one workgroup per row that holds the
+// row in registers (resident_sample). Longer rows with a workspace run over several workgroups:
+// unrestricted and greedy draws split over 16 chunks per
 // row (chunk maxima, then one draw launch; a walk step whose row maxima come from
 // the LM head's epilogue is the draw launch alone, see "split sampling"), top-p
 // draws without top-k over seven launches (see "split top-p"). Otherwise: one
@@ -251,6 +253,18 @@ FG_DEVICE int block_argmax(const Row<DT>& raw, Shared& sh) {
   return (int)fg::rank_key_index(b);
 }
 
+template <int DT>
+FG_DEVICE Row<DT> make_row(const void* rowp, int V) {
+  Row<DT> r;
+  r.p = (const char*)rowp;
+  r.V = V;
+  r.seg = (((V + kWaves - 1) / kWaves) + kStep - 1) / kStep * kStep;
+  r.kt = 0.0f;
+  r.tbl = nullptr;
+  r.m = 0.0f;
+  return r;
+}
+
 struct SampleParams {
   float temperature;
   int greedy;
@@ -262,13 +276,9 @@ struct SampleParams {
 template <int DT>
 FG_DEVICE int block_sample(const void* rowp, int V, const SampleParams& sp, uint32_t u, Shared& sh) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  Row<DT> r;
-  r.p = (const char*)rowp;
-  r.V = V;
-  r.seg = (((V + kWaves - 1) / kWaves) + kStep - 1) / kStep * kStep;
+  Row<DT> r = make_row<DT>(rowp, V);
   r.kt = fg::weight_kt(sp.temperature > 0.0f && sp.temperature != 1.0f, sp.temperature);
   r.tbl = sh.exp2;
-  r.m = 0.0f;
   if (sp.greedy) return block_argmax<DT>(r, sh);
   fg::exp2_table_to_lds(sh.exp2);  // visible after the barriers of the max below
   float mx = -INFINITY;
@@ -293,13 +303,524 @@ FG_DEVICE int block_sample(const void* rowp, int V, const SampleParams& sp, uint
   return block_locate<true, DT>(r, keep, fg::mulhi_u64_u32(total, u), sh);
 }
 
+// ------------------------------------------------------------------ selection by the fixed-point exponent
+// Bins of the exponent a (fg_common.h), 8 per octave below the row maximum: a never grows with
+// x, so the bins are runs of the candidate order. Elements of weight 0 are in no bin: they
+// cannot be drawn, and in the candidate order only NaN comes before one with weight.
+constexpr int kSelBins = 256;
+constexpr int kSelBinShift = 17;             // 2^17 steps of a: 8 bins per octave
+constexpr uint32_t kSelAMax = 40u << 20;     // larger a weigh 0
+constexpr int kSelList = 8192;               // list entries per row
+constexpr int kSelTopK = 4096;               // largest top_k the list path takes
+
+FG_DEVICE uint32_t fixed_exponent(float m, float x, float kt) {
+#pragma clang fp contract(off)
+  return (uint32_t)fminf((m - x) * kt, fg::kWeightZmax);
+}
+// The weight of weight_q40 from its exponent.
+FG_DEVICE uint64_t exponent_weight(uint32_t a, const uint64_t* tbl) {
+  const uint64_t e = tbl[(a >> 10) & 1023u];
+  const uint32_t w = (uint32_t)e - (__umul24((uint32_t)(e >> 32), a & 1023u) >> 10);
+  return ((uint64_t)w << 32) >> ((a >> 20) + 23u);
+}
+FG_DEVICE int sel_bin(uint32_t a) { return min((int)(a >> kSelBinShift), kSelBins - 1); }
+
+// Largest-first selection over the keys ck[0, n) >= cut (whole block of kThreads; the keys are
+// distinct): the key at which the running count, or the running q-mass of the logit that a key
+// holds, first exceeds target. LOW orders by the low word alone (index ascending). The caller
+// guarantees that the total exceeds target. Radix select from the highest differing bit, 8
+// bits a level, ending early where one key is left.
+struct SelectShared {
+  uint64_t hist[256];
+  uint32_t cnt[256];
+  uint64_t wred[kWaves];
+  uint64_t above, found;
+  int digit;
+};
+
+template <bool MASS, bool LOW>
+FG_DEVICE uint64_t list_select(const uint64_t* ck, int n, uint64_t cut, uint64_t target, float m, float kt,
+                               const uint64_t* tbl, SelectShared& sh) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const auto value = [](uint64_t k) { return LOW ? (k & 0xffffffffull) : k; };
+  // bits in which the considered keys differ
+  uint64_t ones = 0, zeros = 0;
+#pragma unroll 1
+  for (int i = tid; i < n; i += kThreads)
+    if (ck[i] >= cut) {
+      ones |= value(ck[i]);
+      zeros |= ~value(ck[i]);
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    ones |= fg::shfl_xor_u64(ones, o);
+    zeros |= fg::shfl_xor_u64(zeros, o);
+  }
+  __syncthreads();  // sh is free
+  if (lane == 0) {
+    sh.wred[tid >> 6] = ones;
+    sh.hist[tid >> 6] = zeros;
+  }
+  __syncthreads();
+#pragma unroll 2
+  for (int w = 0; w < kWaves; ++w) {
+    ones |= sh.wred[w];
+    zeros |= sh.hist[w];
+  }
+  const uint64_t diff = ones & zeros;
+  if (diff == 0) return value(ones);  // one key
+  int shift = max(0, 56 - __builtin_clzll(diff));
+  // the chosen bits so far: the ones above the highest differing bit are common to all
+  uint64_t fixed = shift + 8 >= 64 ? 0ull : ~0ull << (shift + 8);
+  uint64_t prefix = ones & fixed, above = 0;
+  for (;;) {
+    __syncthreads();
+    if (tid < 256) {
+      sh.hist[tid] = 0;
+      sh.cnt[tid] = 0;
+    }
+    __syncthreads();
+#pragma unroll 1
+  for (int i = tid; i < n; i += kThreads) {
+      const uint64_t k = ck[i], v = value(k);
+      if (k >= cut && (v & fixed) == prefix) {
+        const int d = (int)(v >> shift) & 255;
+        atomicAdd(&sh.cnt[d], 1u);
+        if constexpr (MASS)
+          atomicAdd((unsigned long long*)&sh.hist[d],
+                    (unsigned long long)fg::weight_q40(m, fg::rank_key_value(k), kt, tbl));
+      }
+    }
+    __syncthreads();
+    if (tid < 64) {  // lane l owns digits 255 - 4 l .. 252 - 4 l
+      uint64_t h[4], mine = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int d = 255 - 4 * lane - j;
+        h[j] = MASS ? sh.hist[d] : (uint64_t)sh.cnt[d];
+        mine += h[j];
+      }
+      const uint64_t incl = fg::wave_incl_scan_u64(mine), excl = incl - mine;
+      if (above + excl <= target && target < above + incl) {
+        uint64_t c = above + excl;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (c + h[j] > target) {
+            sh.digit = 255 - 4 * lane - j;
+            sh.above = c;
+            break;
+          }
+          c += h[j];
+        }
+      }
+    }
+    __syncthreads();
+    above = sh.above;
+    prefix |= (uint64_t)sh.digit << shift;
+    fixed |= 255ull << shift;
+    if (sh.cnt[sh.digit] == 1) {
+#pragma unroll 1
+  for (int i = tid; i < n; i += kThreads)
+        if (ck[i] >= cut && (value(ck[i]) & fixed) == prefix) sh.found = value(ck[i]);
+      __syncthreads();
+      return sh.found;
+    }
+    if (shift == 0) return prefix;
+    shift = max(0, shift - 8);
+  }
+}
+
+// The draw among at most kSmallList listed candidates: the first `slots` of them in candidate
+// order, of those the ones whose preceding q-mass is at most the top-p target (tp32 != 0), then
+// the one in index order that the noise u selects. Every candidate's preceding count and mass
+// comes from a comparison with every other one, eight threads a candidate: two passes and five
+// barriers, where each radix select above takes four barriers a level. -1 when nothing has weight.
+constexpr int kSmallList = 128;
+
+struct SmallShared {
+  uint64_t w[kSmallList], mass[kSmallList], at[kSmallList];
+  int rank[kSmallList];
+  int tok;
+};
+
+FG_DEVICE int small_draw(const uint64_t* ck, int n, int64_t slots, uint32_t tp32, uint32_t u, float m, float kt,
+                         const uint64_t* tbl, SmallShared& sh) {
+  static_assert(kThreads == 8 * kSmallList, "eight threads a candidate");
+  const int tid = threadIdx.x, lane = tid & 63, i = tid & (kSmallList - 1), s0 = (tid / kSmallList) * (kSmallList / 8);
+  if (tid < kSmallList) {
+    sh.w[i] = i < n ? fg::weight_q40(m, fg::rank_key_value(ck[i]), kt, tbl) : 0ull;
+    sh.mass[i] = 0;
+    sh.at[i] = 0;
+    sh.rank[i] = 0;
+    if (tid == 0) sh.tok = -1;
+  }
+  __syncthreads();
+  const uint64_t key = ck[i < n ? i : 0];
+  const int s1 = min(n, s0 + kSmallList / 8);
+  if (i < n) {
+    int rank = 0;
+    uint64_t mass = 0;
+#pragma unroll 4
+    for (int j = s0; j < s1; ++j)
+      if (ck[j] > key) {
+        ++rank;
+        mass += sh.w[j];
+      }
+    if (rank) {
+      atomicAdd(&sh.rank[i], rank);
+      atomicAdd((unsigned long long*)&sh.mass[i], (unsigned long long)mass);
+    }
+  }
+  __syncthreads();
+  // every wave: the candidates lane and lane + 64
+  uint64_t kw[2];
+  uint64_t total = 0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    kw[h] = sh.rank[lane + 64 * h] < slots ? sh.w[lane + 64 * h] : 0ull;
+    total += kw[h];
+  }
+  total = fg::wave_sum_u64(total);
+  if (tp32) {
+    const uint64_t thr = fg::mulhi_u64_u32(total, tp32);
+    total = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (sh.mass[lane + 64 * h] > thr) kw[h] = 0;
+      total += kw[h];
+    }
+    total = fg::wave_sum_u64(total);
+  }
+  __syncthreads();
+  if (tid < 64) {
+    sh.w[lane] = kw[0];
+    sh.w[lane + 64] = kw[1];
+  }
+  __syncthreads();
+  if (total == 0) return -1;
+  const uint64_t target = fg::mulhi_u64_u32(total, u);
+  if (i < n) {
+    uint64_t before = 0;  // the low word of a key falls with the index
+#pragma unroll 4
+    for (int j = s0; j < s1; ++j)
+      if ((uint32_t)ck[j] > (uint32_t)key) before += sh.w[j];
+    if (before) atomicAdd((unsigned long long*)&sh.at[i], (unsigned long long)before);
+  }
+  __syncthreads();
+  if (tid < n && sh.at[tid] <= target && target < sh.at[tid] + sh.w[tid]) sh.tok = (int)fg::rank_key_index(key);
+  __syncthreads();
+  return sh.tok;
+}
+
+// Sum over the block (kThreads) of v.
+FG_DEVICE uint64_t select_block_sum(uint64_t v, SelectShared& sh) {
+  v = fg::wave_sum_u64(v);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) sh.wred[threadIdx.x >> 6] = v;
+  __syncthreads();
+  uint64_t t = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) t += sh.wred[w];
+  return t;
+}
+
+// ------------------------------------------------------------------ one workgroup, the row in registers
+// A row of up to 8,192 G logits held by one workgroup, 8 G per thread (element 8 (1024 u + t) + j
+// of thread t): one memory pass and one launch for every kind of draw, by the rule of block_sample.
+//  * the maximum;
+//  * top-k / top-p: a histogram over the bins above (counts / q-mass), the bin of the cut, a
+//    list of its elements (top-k: and of those above), the exact cut among them;
+//  * the draw: q-mass sums per (group, wave) in vocabulary order, then the one wave that holds the
+//    target scans its lanes. Top-k draws among its list.
+// Bound by latency: one memory round trip and about 32 G weights per thread between some ten
+// barriers. Against the launches it replaces (three for an unrestricted draw, seven for top-p),
+// a draw of 8 x 32,000 bf16 rows took, us: unrestricted 16.6 -> 10.9, top-p 48.8 -> 31.1, top-k 50
+// 49.0 -> 17.0; of 512 rows 43.2 -> 19.9, 220.7 -> 63.4, 102.0 -> 33.9.
+template <bool CUTS>
+struct ResidentShared {
+  uint64_t hist[4][CUTS ? kSelBins : 1];  // copies shared by four waves each
+  uint64_t ck[CUTS ? kSelList : 1];
+  uint64_t wsum[kWaves * 8];   // [group][wave]
+  SelectShared sel;
+  SmallShared small;
+  uint64_t before;
+  int bin, n, nan, tok;
+};
+
+template <int DT, int G, bool CUTS>
+FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, uint32_t u, Shared& sh,
+                              ResidentShared<CUTS>& rs) {
+  static_assert(G * kWaves <= kWaves * 8, "group sums");
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const auto load_group = [&](int g, float(&v)[8]) {
+    const int i0 = (g * kThreads + tid) * 8;
+    if (i0 + 8 <= V) {
+      fg::load8<DT>(rowp, i0, v);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = i0 + j < V ? fg::load_elem<DT>(rowp, i0 + j) : -INFINITY;
+    }
+  };
+  float x[G][8];
+#pragma unroll
+  for (int g = 0; g < G; ++g) load_group(g, x[g]);
+  // Each pass computes from the logits alone, one group at a time: values kept from one pass to
+  // the next, or several groups in flight, would not fit the 128 registers of 1,024 threads.
+  [[maybe_unused]] const auto fresh = [&](int g) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(x[g][j]));
+  };
+  if (!CUTS && sp.greedy) {  // first maximum: value desc (NaN first), index asc
+    uint64_t best = 0;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      fresh(g);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int i = (g * kThreads + tid) * 8 + j;
+        const uint64_t k = i < V ? fg::rank_key(x[g][j], (uint32_t)i) : 0ull;
+        best = k > best ? k : best;
+      }
+    }
+    best = fg::wave_max_u64(best);
+    if (lane == 0) sh.wkey[wave] = best;
+    __syncthreads();
+    best = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) best = sh.wkey[w] > best ? sh.wkey[w] : best;
+    return (int)fg::rank_key_index(best);
+  }
+  fg::exp2_table_to_lds(sh.exp2);
+  const float kt = fg::weight_kt(sp.temperature > 0.0f && sp.temperature != 1.0f, sp.temperature);
+  const bool count = CUTS && sp.top_k > 0;
+  if constexpr (CUTS) {
+    for (int i = tid; i < 4 * kSelBins; i += kThreads) (&rs.hist[0][0])[i] = 0;
+    if (tid == 0) {
+      rs.bin = kSelBins;
+      rs.n = 0;
+      rs.nan = 0;
+    }
+  }
+  float m = -INFINITY;
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m = fmaxf(m, x[g][j]);
+  m = fg::wave_max(m);
+  if (lane == 0) sh.wmax[wave] = m;
+  __syncthreads();
+  m = sh.wmax[0];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) m = fmaxf(m, sh.wmax[w]);
+  const auto weight = [&](float v) { return fg::weight_q40(m, v, kt, sh.exp2); };
+  int bin = 0;  // elements in lower bins are kept, those in it from `cut` on
+  uint64_t cut = 0;
+  uint64_t hit = 0;  // bit 8 g + j: this thread's element j of group g is listed, later: is kept
+  uint32_t e[CUTS ? G : 1][8];  // the exponents stand for the logits from here on
+  if constexpr (CUTS) {
+    uint64_t* h = rs.hist[wave & 3];
+    int nan = 0;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      fresh(g);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        e[g][j] = fixed_exponent(m, x[g][j], kt);
+        nan += x[g][j] != x[g][j];
+        if (e[g][j] <= kSelAMax)
+          atomicAdd((unsigned long long*)&h[sel_bin(e[g][j])],
+                    (unsigned long long)(count ? 1ull : exponent_weight(e[g][j], sh.exp2)));
+      }
+    }
+    if (nan) atomicAdd(&rs.nan, nan);
+    __syncthreads();
+    if (wave == 0) {  // the bin of the cut: lane l owns bins 4 l .. 4 l + 3
+      uint64_t b[4], mine = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        b[j] = rs.hist[0][4 * lane + j] + rs.hist[1][4 * lane + j] + rs.hist[2][4 * lane + j] +
+               rs.hist[3][4 * lane + j];
+        mine += b[j];
+      }
+      const uint64_t incl = fg::wave_incl_scan_u64(mine), total = fg::shfl_u64(incl, 63);
+      const uint64_t slots = (uint64_t)max(sp.top_k - rs.nan, 0);  // NaN ranks first and takes slots
+      // slow path (bin stays kSelBins): no weight, or every slot taken by NaN
+      const bool ok = total > 0 && (!count || slots > 0);
+      const uint64_t target = count ? (total <= slots ? total - 1 : slots - 1) : fg::mulhi_u64_u32(total, sp.tp32);
+      if (ok && incl - mine <= target && target < incl) {
+        uint64_t c = incl - mine;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (c + b[j] > target) {
+            rs.bin = 4 * lane + j;
+            rs.before = target - (count ? 0ull : c);  // position of the cut within the list
+            break;
+          }
+          c += b[j];
+        }
+      }
+    }
+    __syncthreads();
+    bin = rs.bin;
+    if (bin == kSelBins) {
+      __syncthreads();
+      return block_sample<DT>(rowp, V, sp, u, sh);
+    }
+    hit = 0;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      fresh(g);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (e[g][j] <= kSelAMax && (count ? sel_bin(e[g][j]) <= bin : sel_bin(e[g][j]) == bin))
+          hit |= 1ull << (8 * g + j);
+    }
+    const auto index_of = [&](int bit) { return ((bit >> 3) * kThreads + tid) * 8 + (bit & 7); };
+    if (hit) {
+      int at = atomicAdd(&rs.n, (int)__popcll(hit));
+      for (uint64_t rest = hit; rest; rest &= rest - 1) {
+        const int i = index_of(__builtin_ctzll(rest));
+        if (at < kSelList) rs.ck[at] = fg::rank_key(fg::load_elem<DT>(rowp, i), (uint32_t)i);
+        ++at;
+      }
+    }
+    __syncthreads();
+    const int n = rs.n;
+    if (n > kSelList || sp.top_k > kSelTopK) {
+      __syncthreads();
+      return block_sample<DT>(rowp, V, sp, u, sh);
+    }
+    if (count && n <= kSmallList) {
+      const int64_t slots = (int64_t)sp.top_k - rs.nan;
+      const int tok = small_draw(rs.ck, n, slots, sp.tp32, u, m, kt, sh.exp2, rs.small);
+      __syncthreads();
+      return tok;
+    }
+    if (count) {
+      const auto kept_sum = [&]() {
+        uint64_t k = 0;
+        for (int i = tid; i < n; i += kThreads)
+          if (rs.ck[i] >= cut) k += weight(fg::rank_key_value(rs.ck[i]));
+        return select_block_sum(k, rs.sel);
+      };
+      cut = list_select<false, false>(rs.ck, n, 0, rs.before, m, kt, sh.exp2, rs.sel);
+      uint64_t total = kept_sum();
+      if (sp.tp32) {
+        cut = list_select<true, false>(rs.ck, n, cut, fg::mulhi_u64_u32(total, sp.tp32), m, kt, sh.exp2, rs.sel);
+        total = kept_sum();
+      }
+      return (int)fg::rank_key_index(
+          list_select<true, true>(rs.ck, n, cut, fg::mulhi_u64_u32(total, u), m, kt, sh.exp2, rs.sel));
+    }
+    cut = list_select<true, false>(rs.ck, n, 0, rs.before, m, kt, sh.exp2, rs.sel);
+    for (uint64_t rest = hit; rest; rest &= rest - 1) {
+      const int i = index_of(__builtin_ctzll(rest));
+      if (fg::rank_key(fg::load_elem<DT>(rowp, i), (uint32_t)i) < cut) hit &= ~(rest & -rest);
+    }
+  }
+  // the draw among the kept elements, in vocabulary order: q-mass of each (group, wave)
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    if constexpr (CUTS) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(e[g][j]));
+    } else {
+      fresh(g);
+    }
+    uint64_t w = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if constexpr (CUTS) {
+        if (sel_bin(e[g][j]) < bin || ((hit >> (8 * g + j)) & 1)) w += exponent_weight(e[g][j], sh.exp2);
+      } else {
+        w += weight(x[g][j]);
+      }
+    }
+    w = fg::wave_sum_u64(w);
+    if (lane == 0) rs.wsum[g * kWaves + wave] = w;
+  }
+  if (tid == 0) rs.tok = -1;
+  __syncthreads();
+  // every wave finds the (group, wave) run that holds the target: lane l owns runs PL l ..
+  constexpr int PL = (G * kWaves + 63) / 64;
+  uint64_t run[PL], mine = 0;
+#pragma unroll
+  for (int j = 0; j < PL; ++j) {
+    run[j] = lane * PL + j < G * kWaves ? rs.wsum[lane * PL + j] : 0ull;
+    mine += run[j];
+  }
+  const uint64_t incl = fg::wave_incl_scan_u64(mine), total = fg::shfl_u64(incl, 63);
+  if (total == 0) {
+    __syncthreads();
+    return block_argmax<DT>(make_row<DT>(rowp, V), sh);
+  }
+  const uint64_t target = fg::mulhi_u64_u32(total, u);
+  uint64_t c = incl - mine, at = 0;
+  int sel = -1;
+#pragma unroll
+  for (int j = 0; j < PL; ++j) {
+    if (sel < 0 && c <= target && target < c + run[j]) {
+      sel = lane * PL + j;
+      at = c;
+    }
+    c += run[j];
+  }
+  const int src = (int)__builtin_ctzll(__ballot(sel >= 0));  // exactly one lane holds it
+  sel = __shfl(sel, src, 64);
+  at = fg::shfl_u64(at, src);
+  if (sel % kWaves == wave) {  // this wave weighs its elements of the group again
+    const int g = sel / kWaves;
+    float v[8];
+    load_group(g, v);
+    uint64_t w[8], sum = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int i = (g * kThreads + tid) * 8 + j;
+      w[j] = weight(v[j]);
+      if constexpr (CUTS) {
+        const int b = sel_bin(fixed_exponent(m, v[j], kt));
+        if (b > bin || (b == bin && fg::rank_key(v[j], (uint32_t)i) < cut)) w[j] = 0;
+      }
+      sum += w[j];
+    }
+    uint64_t cum = at + fg::wave_incl_scan_u64(sum) - sum;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (cum <= target && target < cum + w[j]) rs.tok = (g * kThreads + tid) * 8 + j;
+      cum += w[j];
+    }
+  }
+  __syncthreads();
+  return rs.tok;
+}
+
+// Groups of 8,192 logits a workgroup holds for a row of V: 0 when the row is too long.
+// One workgroup weighs 32,768 logits in about the time of a launch; twice as many still beat the
+// split launches without a cut (64 x 65,536 bf16: 14.3 against 17.1 us), but not with one, where
+// the weighing passes are two (64 x 65,536, top-p: 59.7 against 44.5 us split).
+constexpr int resident_groups(int vocab, bool cuts) {
+  return vocab <= 8192 * 4 ? 4 : vocab <= 8192 * 8 && !cuts ? 8 : 0;
+}
+
+template <int DT, int G, bool CUTS>
+FG_DEVICE int row_sample(const void* rowp, int V, const SampleParams& sp, uint32_t u, Shared& sh) {
+  if constexpr (G > 0) {
+    __shared__ ResidentShared<CUTS> rs;
+    return resident_sample<DT, G, CUTS>(rowp, V, sp, u, sh, rs);
+  } else {
+    return block_sample<DT>(rowp, V, sp, u, sh);
+  }
+}
+
 FG_DEVICE uint32_t noise_value(const uint32_t* noise, int64_t noise_index, uint64_t seed, uint64_t step,
                                uint32_t seq, uint32_t draw) {
   if (noise) return noise[noise_index];
   return fg::counter_noise(seed, step, seq, draw);
 }
 
-template <int DT>
+template <int DT, int G, bool CUTS>
 __global__ void __launch_bounds__(kThreads) sample_rows_kernel(
     const void* __restrict__ logits, int64_t row_stride, int vocab, const int32_t* __restrict__ row_index,
     const int32_t* __restrict__ forced, const uint32_t* __restrict__ noise, int noise_stride, int noise_col,
@@ -315,7 +836,7 @@ __global__ void __launch_bounds__(kThreads) sample_rows_kernel(
   const char* rowp = (const char*)logits + (int64_t)src * row_stride * (DT == fg::kBF16 ? 2 : 4);
   uint32_t seq = seq_ids ? (uint32_t)seq_ids[rrow] : (uint32_t)rrow;
   uint32_t u = noise_value(noise, (int64_t)rrow * noise_stride + noise_col, seed, step, seq, (uint32_t)draw);
-  int tok = block_sample<DT>(rowp, vocab, sp, u, sh);
+  int tok = row_sample<DT, G, CUTS>(rowp, vocab, sp, u, sh);
   if (threadIdx.x == 0) out[rrow] = tok;
 }
 
@@ -398,7 +919,7 @@ FG_DEVICE void walk_apply(int b, int tok, int parent, const int32_t* tree_tokens
   }
 }
 
-template <int DT>
+template <int DT, int G, bool CUTS>
 __global__ void __launch_bounds__(kThreads) walk_step_kernel(
     const void* __restrict__ logits, int64_t row_stride, int vocab, const int32_t* __restrict__ slot_map,
     const int32_t* __restrict__ tree_tokens, const int32_t* __restrict__ parents, const int32_t* __restrict__ n_nodes,
@@ -425,7 +946,7 @@ __global__ void __launch_bounds__(kThreads) walk_step_kernel(
   uint32_t seq = seq_ids ? (uint32_t)seq_ids[b] : (uint32_t)b;
   uint32_t u = noise_value(noise, (int64_t)b * noise_stride + noise_col0 + walk_step, seed, step, seq,
                            (uint32_t)(draw0 + walk_step));
-  int tok = block_sample<DT>(rowp, vocab, sp, u, sh);
+  int tok = row_sample<DT, G, CUTS>(rowp, vocab, sp, u, sh);
   if (threadIdx.x < 64)
     walk_apply(b, tok, parent, tree_tokens, parents, n_nodes, nmax, batch, walk_step, acc_tokens, acc_nodes, acc_stride,
                acc_len, last_node, correction, state, err_flag, next_rows, next_active);
@@ -840,9 +1361,8 @@ __global__ void __launch_bounds__(kSplitThreads) split_pick_kernel(SplitArgs a, 
 // Restricted draws over kSplitChunks workgroups per row, four launches, the same integer rule
 // as block_sample:
 //  (1) chunk maxima (split_max_kernel), unless the row's maxima parts are given;
-//  (2) per chunk, a 256-bin histogram over the fixed-point exponent a (fg_common.h), 8 bins
-//      per octave below the row maximum: q-mass for top-p, counts for top-k. a never grows
-//      with x, so the bins are runs of the candidate order; elements of weight 0 are in no bin;
+//  (2) per chunk, a histogram over the bins of the fixed-point exponent: q-mass for top-p,
+//      counts for top-k;
 //  (3) each chunk merges the row's 16 histograms, finds the bin that holds the cut and appends
 //      the indices of its own elements of that bin (top-k: of that bin and the ones above) to
 //      the row's list;
@@ -858,11 +1378,6 @@ __global__ void __launch_bounds__(kSplitThreads) split_pick_kernel(SplitArgs a, 
 // 64 x 152,064), and a bf16 row's last two levels had nothing left to separate. Measured, a draw:
 // top-p 0.95 at 64 x 152,064 bf16 114 -> 57 us (seven launches before); top-k 50 at
 // 32 x 151,936 bf16 210 -> 47 us (one workgroup per row before).
-constexpr int kSelBins = 256;
-constexpr int kSelBinShift = 17;             // 2^17 steps of a: 8 bins per octave
-constexpr uint32_t kSelAMax = 40u << 20;     // larger a weigh 0
-constexpr int kSelList = 8192;               // list entries per row
-constexpr int kSelTopK = 4096;               // largest top_k the list path takes
 static_assert(kSelBins == kSplitThreads, "one histogram bin per thread");
 
 // Where the cut of one row lies (written by chunk 0 of launch 3).
@@ -871,12 +1386,6 @@ struct SelState {
   int32_t slow;   // the row is drawn by block_sample
   int32_t all;    // every listed element is kept (top-k with no more candidates than slots)
 };
-
-FG_DEVICE uint32_t fixed_exponent(float m, float x, float kt) {
-#pragma clang fp contract(off)
-  return (uint32_t)fminf((m - x) * kt, fg::kWeightZmax);
-}
-FG_DEVICE int sel_bin(uint32_t a) { return min((int)(a >> kSelBinShift), kSelBins - 1); }
 
 template <int DT, bool COUNT>
 __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) {
@@ -1046,120 +1555,6 @@ __global__ void __launch_bounds__(kSplitThreads) split_gather_kernel(SplitArgs a
       ++o;
     }
   }
-}
-
-// Largest-first selection over the keys ck[0, n) >= cut (whole block of kThreads; the keys are
-// distinct): the key at which the running count, or the running q-mass of the logit that a key
-// holds, first exceeds target. LOW orders by the low word alone (index ascending). The caller
-// guarantees that the total exceeds target. Radix select from the highest differing bit, 8
-// bits a level, ending early where one key is left.
-struct SelectShared {
-  uint64_t hist[256];
-  uint32_t cnt[256];
-  uint64_t wred[kWaves];
-  uint64_t above, found;
-  int digit;
-};
-
-template <bool MASS, bool LOW>
-FG_DEVICE uint64_t list_select(const uint64_t* ck, int n, uint64_t cut, uint64_t target, float m, float kt,
-                               const uint64_t* tbl, SelectShared& sh) {
-  const int tid = threadIdx.x, lane = tid & 63;
-  const auto value = [](uint64_t k) { return LOW ? (k & 0xffffffffull) : k; };
-  // bits in which the considered keys differ
-  uint64_t ones = 0, zeros = 0;
-  for (int i = tid; i < n; i += kThreads)
-    if (ck[i] >= cut) {
-      ones |= value(ck[i]);
-      zeros |= ~value(ck[i]);
-    }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    ones |= fg::shfl_xor_u64(ones, o);
-    zeros |= fg::shfl_xor_u64(zeros, o);
-  }
-  __syncthreads();  // sh is free
-  if (lane == 0) {
-    sh.wred[tid >> 6] = ones;
-    sh.hist[tid >> 6] = zeros;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    ones |= sh.wred[w];
-    zeros |= sh.hist[w];
-  }
-  const uint64_t diff = ones & zeros;
-  if (diff == 0) return value(ones);  // one key
-  int shift = max(0, 56 - __builtin_clzll(diff));
-  // the chosen bits so far: the ones above the highest differing bit are common to all
-  uint64_t fixed = shift + 8 >= 64 ? 0ull : ~0ull << (shift + 8);
-  uint64_t prefix = ones & fixed, above = 0;
-  for (;;) {
-    __syncthreads();
-    if (tid < 256) {
-      sh.hist[tid] = 0;
-      sh.cnt[tid] = 0;
-    }
-    __syncthreads();
-    for (int i = tid; i < n; i += kThreads) {
-      const uint64_t k = ck[i], v = value(k);
-      if (k >= cut && (v & fixed) == prefix) {
-        const int d = (int)(v >> shift) & 255;
-        atomicAdd(&sh.cnt[d], 1u);
-        if constexpr (MASS)
-          atomicAdd((unsigned long long*)&sh.hist[d],
-                    (unsigned long long)fg::weight_q40(m, fg::rank_key_value(k), kt, tbl));
-      }
-    }
-    __syncthreads();
-    if (tid < 64) {  // lane l owns digits 255 - 4 l .. 252 - 4 l
-      uint64_t h[4], mine = 0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int d = 255 - 4 * lane - j;
-        h[j] = MASS ? sh.hist[d] : (uint64_t)sh.cnt[d];
-        mine += h[j];
-      }
-      const uint64_t incl = fg::wave_incl_scan_u64(mine), excl = incl - mine;
-      if (above + excl <= target && target < above + incl) {
-        uint64_t c = above + excl;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (c + h[j] > target) {
-            sh.digit = 255 - 4 * lane - j;
-            sh.above = c;
-            break;
-          }
-          c += h[j];
-        }
-      }
-    }
-    __syncthreads();
-    above = sh.above;
-    prefix |= (uint64_t)sh.digit << shift;
-    fixed |= 255ull << shift;
-    if (sh.cnt[sh.digit] == 1) {
-      for (int i = tid; i < n; i += kThreads)
-        if (ck[i] >= cut && (value(ck[i]) & fixed) == prefix) sh.found = value(ck[i]);
-      __syncthreads();
-      return sh.found;
-    }
-    if (shift == 0) return prefix;
-    shift = max(0, shift - 8);
-  }
-}
-
-// Sum over the block (kThreads) of v.
-FG_DEVICE uint64_t select_block_sum(uint64_t v, SelectShared& sh) {
-  v = fg::wave_sum_u64(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh.wred[threadIdx.x >> 6] = v;
-  __syncthreads();
-  uint64_t t = 0;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) t += sh.wred[w];
-  return t;
 }
 
 // Elements of a row at or above a cut rank key, for block_sum / block_locate over a chunk that
@@ -1423,6 +1818,28 @@ SampleParams make_params(float temperature, int greedy, int top_k, int vocab, ui
   return sp;
 }
 
+// f(dtype, resident groups, whether the draw has a cut), each an integral constant, for the
+// one-workgroup-per-row kernels on rows of `vocab` logits.
+template <class F>
+void for_row_kernel(int dtype, int vocab, const SampleParams& sp, F&& f) {
+  const bool cuts = !sp.greedy && (sp.top_k || sp.tp32);
+  const auto groups = [&](auto dt, auto g) {
+    if constexpr (decltype(g)::value == 4) {
+      if (cuts) return f(dt, g, std::true_type{});
+    }
+    f(dt, g, std::false_type{});
+  };
+  const auto types = [&](auto dt) {
+    switch (resident_groups(vocab, cuts)) {
+      case 4: groups(dt, std::integral_constant<int, 4>{}); break;
+      case 8: groups(dt, std::integral_constant<int, 8>{}); break;
+      default: f(dt, std::integral_constant<int, 0>{}, std::false_type{}); break;
+    }
+  };
+  if (dtype == fg::kBF16) types(std::integral_constant<int, fg::kBF16>{});
+  else types(std::integral_constant<int, fg::kF32>{});
+}
+
 int sample_tokens_impl(const char* who, const void* logits, int dtype, int64_t row_stride, int rows, int vocab,
                        const int32_t* row_index, const int32_t* forced, const uint32_t* noise,
                        int noise_stride, int noise_col, uint64_t seed, uint64_t step,
@@ -1437,7 +1854,8 @@ int sample_tokens_impl(const char* who, const void* logits, int dtype, int64_t r
   SampleParams sp = make_params(temperature, greedy, top_k, vocab, top_p_fixed);
   hipStream_t s = (hipStream_t)stream;
   SplitArgs a;
-  if (split_setup(a, workspace, workspace_bytes, rows, logits, row_stride, vocab, temperature, sp)) {
+  if (!resident_groups(vocab, !sp.greedy && (sp.top_k || sp.tp32)) &&
+      split_setup(a, workspace, workspace_bytes, rows, logits, row_stride, vocab, temperature, sp)) {
     a.row_index = row_index;
     a.forced = forced;
     DrawOut d{};
@@ -1448,12 +1866,11 @@ int sample_tokens_impl(const char* who, const void* logits, int dtype, int64_t r
     else split_draw<fg::kF32, false>(a, d, rows, true, s);
     return fg::check_launch(who);
   }
-  if (dtype == fg::kBF16)
-    hipLaunchKernelGGL(sample_rows_kernel<fg::kBF16>, dim3(rows), dim3(kThreads), 0, s, logits, row_stride, vocab,
-                       row_index, forced, noise, noise_stride, noise_col, seed, step, seq_ids, draw, sp, out_tokens);
-  else
-    hipLaunchKernelGGL(sample_rows_kernel<fg::kF32>, dim3(rows), dim3(kThreads), 0, s, logits, row_stride, vocab,
-                       row_index, forced, noise, noise_stride, noise_col, seed, step, seq_ids, draw, sp, out_tokens);
+  for_row_kernel(dtype, vocab, sp, [&](auto dt, auto g, auto cuts) {
+    hipLaunchKernelGGL((sample_rows_kernel<decltype(dt)::value, decltype(g)::value, decltype(cuts)::value>), dim3(rows), dim3(kThreads), 0, s,
+                       logits, row_stride, vocab, row_index, forced, noise, noise_stride, noise_col, seed, step,
+                       seq_ids, draw, sp, out_tokens);
+  });
   return fg::check_launch(who);
 }
 
@@ -1509,16 +1926,12 @@ int fg_accept_walk(const void* tree_logits, int dtype, int64_t row_stride, int v
   hipLaunchKernelGGL(walk_init_kernel, dim3((batch + 63) / 64), dim3(64), 0, s, tree_tokens, parents, n_nodes, nmax,
                      batch, acc_tokens, acc_nodes, acc_stride, acc_len, last_node, correction, workspace);
   for (int t = 0; t < max_walk_steps; ++t) {
-    if (dtype == fg::kBF16)
-      hipLaunchKernelGGL(walk_step_kernel<fg::kBF16>, dim3(batch), dim3(kThreads), 0, s, tree_logits, row_stride,
-                         vocab, slot_map, tree_tokens, parents, n_nodes, nmax, batch, t, 0, noise, noise_stride,
-                         noise_col0, seed, step, seq_ids, draw0, sp, acc_tokens, acc_nodes, acc_stride, acc_len,
-                         last_node, correction, workspace, err_flag, nullptr, nullptr);
-    else
-      hipLaunchKernelGGL(walk_step_kernel<fg::kF32>, dim3(batch), dim3(kThreads), 0, s, tree_logits, row_stride,
-                         vocab, slot_map, tree_tokens, parents, n_nodes, nmax, batch, t, 0, noise, noise_stride,
-                         noise_col0, seed, step, seq_ids, draw0, sp, acc_tokens, acc_nodes, acc_stride, acc_len,
-                         last_node, correction, workspace, err_flag, nullptr, nullptr);
+    for_row_kernel(dtype, vocab, sp, [&](auto dt, auto g, auto cuts) {
+      hipLaunchKernelGGL((walk_step_kernel<decltype(dt)::value, decltype(g)::value, decltype(cuts)::value>), dim3(batch), dim3(kThreads), 0, s,
+                         tree_logits, row_stride, vocab, slot_map, tree_tokens, parents, n_nodes, nmax, batch, t, 0,
+                         noise, noise_stride, noise_col0, seed, step, seq_ids, draw0, sp, acc_tokens, acc_nodes,
+                         acc_stride, acc_len, last_node, correction, workspace, err_flag, nullptr, nullptr);
+    });
   }
   return fg::check_launch("fg_accept_walk");
 }
@@ -1564,7 +1977,8 @@ int fg_walk_step(const void* step_logits, int dtype, int64_t row_stride, int voc
   SampleParams sp = make_params(temperature, greedy, top_k, vocab, top_p_fixed);
   hipStream_t s = (hipStream_t)stream;
   SplitArgs a;
-  if (split_setup(a, workspace, workspace_bytes, batch, step_logits, row_stride, vocab, temperature, sp)) {
+  if (!resident_groups(vocab, !sp.greedy && (sp.top_k || sp.tp32)) &&
+      split_setup(a, workspace, workspace_bytes, batch, step_logits, row_stride, vocab, temperature, sp)) {
     a.active = state + batch;
     const bool cut = !sp.greedy && (sp.top_k || sp.tp32);
     const bool with_max = part_max == nullptr;
@@ -1587,16 +2001,12 @@ int fg_walk_step(const void* step_logits, int dtype, int64_t row_stride, int voc
     else split_draw<fg::kF32, true>(a, d, batch, with_max, s);
     return fg::check_launch("fg_walk_step");
   }
-  if (dtype == fg::kBF16)
-    hipLaunchKernelGGL(walk_step_kernel<fg::kBF16>, dim3(batch), dim3(kThreads), 0, s, step_logits, row_stride, vocab,
-                       nullptr, tree_tokens, parents, n_nodes, nmax, batch, walk_step, 1, noise, noise_stride,
-                       noise_col0, seed, step, seq_ids, draw0, sp, acc_tokens, acc_nodes, acc_stride, acc_len,
-                       last_node, correction, state, err_flag, next_row_index, next_row_active);
-  else
-    hipLaunchKernelGGL(walk_step_kernel<fg::kF32>, dim3(batch), dim3(kThreads), 0, s, step_logits, row_stride, vocab,
-                       nullptr, tree_tokens, parents, n_nodes, nmax, batch, walk_step, 1, noise, noise_stride,
-                       noise_col0, seed, step, seq_ids, draw0, sp, acc_tokens, acc_nodes, acc_stride, acc_len,
-                       last_node, correction, state, err_flag, next_row_index, next_row_active);
+  for_row_kernel(dtype, vocab, sp, [&](auto dt, auto g, auto cuts) {
+    hipLaunchKernelGGL((walk_step_kernel<decltype(dt)::value, decltype(g)::value, decltype(cuts)::value>), dim3(batch), dim3(kThreads), 0, s,
+                       step_logits, row_stride, vocab, nullptr, tree_tokens, parents, n_nodes, nmax, batch, walk_step, 1,
+                       noise, noise_stride, noise_col0, seed, step, seq_ids, draw0, sp, acc_tokens, acc_nodes,
+                       acc_stride, acc_len, last_node, correction, state, err_flag, next_row_index, next_row_active);
+  });
   return fg::check_launch("fg_walk_step");
 }
 
