@@ -317,6 +317,11 @@ FG_DEVICE uint32_t fixed_exponent(float m, float x, float kt) {
 #pragma clang fp contract(off)
   return (uint32_t)fminf((m - x) * kt, fg::kWeightZmax);
 }
+// Histogram copies: lane l adds to copy l % kCopies of a bin, the copies of a bin side by side on
+// banks of their own, so that logits close to each other wait less for one word (the q-mass
+// pass of 64 x 152,064: 13.4 -> 12.2 us with 8 copies instead of one per wave).
+constexpr int kCopies = 8;
+
 // The weight of weight_q40 from its exponent.
 FG_DEVICE uint64_t exponent_weight(uint32_t a, const uint64_t* tbl) {
   const uint64_t e = tbl[(a >> 10) & 1023u];
@@ -430,23 +435,22 @@ FG_DEVICE uint64_t list_select(const uint64_t* ck, int n, uint64_t cut, uint64_t
   }
 }
 
-// The draw among at most kSmallList listed candidates: the first `slots` of them in candidate
-// order, of those the ones whose preceding q-mass is at most the top-p target (tp32 != 0), then
-// the one in index order that the noise u selects. Every candidate's preceding count and mass
-// comes from a comparison with every other one, eight threads a candidate: two passes and five
-// barriers, where each radix select above takes four barriers a level. -1 when nothing has weight.
-constexpr int kSmallList = 128;
+// At most kSmallList keys are ranked by comparing each with every other, kSmallPer threads a
+// key: one pass instead of the four barriers a level of the radix select.
+constexpr int kSmallList = 256;
+constexpr int kSmallPer = kThreads / kSmallList;
 
 struct SmallShared {
-  uint64_t w[kSmallList], mass[kSmallList], at[kSmallList];
-  int rank[kSmallList];
+  uint64_t w[kSmallList];     // q-mass
+  uint64_t mass[kSmallList];  // q-mass of the keys before it in candidate order
+  uint64_t at[kSmallList];    // kept q-mass of the keys before it in index order
+  int rank[kSmallList];       // keys before it in candidate order
+  uint64_t key;
   int tok;
 };
 
-FG_DEVICE int small_draw(const uint64_t* ck, int n, int64_t slots, uint32_t tp32, uint32_t u, float m, float kt,
-                         const uint64_t* tbl, SmallShared& sh) {
-  static_assert(kThreads == 8 * kSmallList, "eight threads a candidate");
-  const int tid = threadIdx.x, lane = tid & 63, i = tid & (kSmallList - 1), s0 = (tid / kSmallList) * (kSmallList / 8);
+FG_DEVICE void small_rank(const uint64_t* ck, int n, float m, float kt, const uint64_t* tbl, SmallShared& sh) {
+  const int tid = threadIdx.x, i = tid & (kSmallList - 1);
   if (tid < kSmallList) {
     sh.w[i] = i < n ? fg::weight_q40(m, fg::rank_key_value(ck[i]), kt, tbl) : 0ull;
     sh.mass[i] = 0;
@@ -455,13 +459,12 @@ FG_DEVICE int small_draw(const uint64_t* ck, int n, int64_t slots, uint32_t tp32
     if (tid == 0) sh.tok = -1;
   }
   __syncthreads();
-  const uint64_t key = ck[i < n ? i : 0];
-  const int s1 = min(n, s0 + kSmallList / 8);
   if (i < n) {
+    const uint64_t key = ck[i];
     int rank = 0;
     uint64_t mass = 0;
-#pragma unroll 4
-    for (int j = s0; j < s1; ++j)
+#pragma unroll 2
+    for (int j = tid / kSmallList; j < n; j += kSmallPer)
       if (ck[j] > key) {
         ++rank;
         mass += sh.w[j];
@@ -472,11 +475,28 @@ FG_DEVICE int small_draw(const uint64_t* ck, int n, int64_t slots, uint32_t tp32
     }
   }
   __syncthreads();
-  // every wave: the candidates lane and lane + 64
-  uint64_t kw[2];
-  uint64_t total = 0;
+}
+
+// The key at which the running q-mass of the n <= kSmallList keys first exceeds target.
+FG_DEVICE uint64_t small_cut(const uint64_t* ck, int n, uint64_t target, float m, float kt, const uint64_t* tbl,
+                             SmallShared& sh) {
+  small_rank(ck, n, m, kt, tbl, sh);
+  const int i = threadIdx.x;
+  if (i < n && sh.mass[i] <= target && target < sh.mass[i] + sh.w[i]) sh.key = ck[i];
+  __syncthreads();
+  return sh.key;
+}
+
+// list_draw of n <= kSmallList keys.
+FG_DEVICE int small_draw(const uint64_t* ck, int n, int64_t slots, uint32_t tp32, uint32_t u, float m, float kt,
+                         const uint64_t* tbl, SmallShared& sh) {
+  const int tid = threadIdx.x, lane = tid & 63, i = tid & (kSmallList - 1);
+  small_rank(ck, n, m, kt, tbl, sh);
+  // every wave sums the kept mass: keys lane, lane + 64, ...
+  constexpr int P = kSmallList / 64;
+  uint64_t kw[P], total = 0;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int h = 0; h < P; ++h) {
     kw[h] = sh.rank[lane + 64 * h] < slots ? sh.w[lane + 64 * h] : 0ull;
     total += kw[h];
   }
@@ -485,7 +505,7 @@ FG_DEVICE int small_draw(const uint64_t* ck, int n, int64_t slots, uint32_t tp32
     const uint64_t thr = fg::mulhi_u64_u32(total, tp32);
     total = 0;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < P; ++h) {
       if (sh.mass[lane + 64 * h] > thr) kw[h] = 0;
       total += kw[h];
     }
@@ -493,21 +513,23 @@ FG_DEVICE int small_draw(const uint64_t* ck, int n, int64_t slots, uint32_t tp32
   }
   __syncthreads();
   if (tid < 64) {
-    sh.w[lane] = kw[0];
-    sh.w[lane + 64] = kw[1];
+#pragma unroll
+    for (int h = 0; h < P; ++h) sh.w[lane + 64 * h] = kw[h];
   }
   __syncthreads();
   if (total == 0) return -1;
   const uint64_t target = fg::mulhi_u64_u32(total, u);
   if (i < n) {
-    uint64_t before = 0;  // the low word of a key falls with the index
-#pragma unroll 4
-    for (int j = s0; j < s1; ++j)
-      if ((uint32_t)ck[j] > (uint32_t)key) before += sh.w[j];
+    const uint32_t low = (uint32_t)ck[i];  // falls with the index
+    uint64_t before = 0;
+#pragma unroll 2
+    for (int j = tid / kSmallList; j < n; j += kSmallPer)
+      if ((uint32_t)ck[j] > low) before += sh.w[j];
     if (before) atomicAdd((unsigned long long*)&sh.at[i], (unsigned long long)before);
   }
   __syncthreads();
-  if (tid < n && sh.at[tid] <= target && target < sh.at[tid] + sh.w[tid]) sh.tok = (int)fg::rank_key_index(key);
+  if (tid < n && sh.at[tid] <= target && target < sh.at[tid] + sh.w[tid])
+    sh.tok = (int)fg::rank_key_index(ck[tid]);
   __syncthreads();
   return sh.tok;
 }
@@ -524,6 +546,29 @@ FG_DEVICE uint64_t select_block_sum(uint64_t v, SelectShared& sh) {
   return t;
 }
 
+// The draw among n listed candidates (whole block): the first `slots` of them in candidate order,
+// then the top-p cut (tp32 != 0), then the noise u. -1 when nothing has weight.
+FG_DEVICE int list_draw(const uint64_t* ck, int n, int64_t slots, uint32_t tp32, uint32_t u, float m, float kt,
+                        const uint64_t* tbl, SelectShared& sel, SmallShared& small) {
+  if (n <= kSmallList) return small_draw(ck, n, slots, tp32, u, m, kt, tbl, small);
+  uint64_t cut = 0;
+  const auto kept_sum = [&]() {
+    uint64_t k = 0;
+#pragma unroll 1
+    for (int i = threadIdx.x; i < n; i += kThreads)
+      if (ck[i] >= cut) k += fg::weight_q40(m, fg::rank_key_value(ck[i]), kt, tbl);
+    return select_block_sum(k, sel);
+  };
+  if (slots < n) cut = list_select<false, false>(ck, n, 0, (uint64_t)(slots - 1), m, kt, tbl, sel);
+  uint64_t total = kept_sum();
+  if (total == 0) return -1;
+  if (tp32) {
+    cut = list_select<true, false>(ck, n, cut, fg::mulhi_u64_u32(total, tp32), m, kt, tbl, sel);
+    total = kept_sum();
+  }
+  return (int)fg::rank_key_index(list_select<true, true>(ck, n, cut, fg::mulhi_u64_u32(total, u), m, kt, tbl, sel));
+}
+
 // ------------------------------------------------------------------ one workgroup, the row in registers
 // A row of up to 8,192 G logits held by one workgroup, 8 G per thread (element 8 (1024 u + t) + j
 // of thread t): one memory pass and one launch for every kind of draw, by the rule of block_sample.
@@ -535,10 +580,10 @@ FG_DEVICE uint64_t select_block_sum(uint64_t v, SelectShared& sh) {
 // Bound by latency: one memory round trip and about 32 G weights per thread between some ten
 // barriers. Against the launches it replaces (three for an unrestricted draw, seven for top-p),
 // a draw of 8 x 32,000 bf16 rows took, us: unrestricted 16.6 -> 10.9, top-p 48.8 -> 31.1, top-k 50
-// 49.0 -> 17.0; of 512 rows 43.2 -> 19.9, 220.7 -> 63.4, 102.0 -> 33.9.
+// 49.0 -> 15.7; of 512 rows 43.2 -> 19.9, 220.7 -> 63.4, 102.0 -> 32.0.
 template <bool CUTS>
 struct ResidentShared {
-  uint64_t hist[4][CUTS ? kSelBins : 1];  // copies shared by four waves each
+  uint64_t hist[CUTS ? kSelBins : 1][kCopies];
   uint64_t ck[CUTS ? kSelList : 1];
   uint64_t wsum[kWaves * 8];   // [group][wave]
   SelectShared sel;
@@ -595,7 +640,7 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
   const float kt = fg::weight_kt(sp.temperature > 0.0f && sp.temperature != 1.0f, sp.temperature);
   const bool count = CUTS && sp.top_k > 0;
   if constexpr (CUTS) {
-    for (int i = tid; i < 4 * kSelBins; i += kThreads) (&rs.hist[0][0])[i] = 0;
+    for (int i = tid; i < kCopies * kSelBins; i += kThreads) (&rs.hist[0][0])[i] = 0;
     if (tid == 0) {
       rs.bin = kSelBins;
       rs.n = 0;
@@ -619,7 +664,7 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
   uint64_t hit = 0;  // bit 8 g + j: this thread's element j of group g is listed, later: is kept
   uint32_t e[CUTS ? G : 1][8];  // the exponents stand for the logits from here on
   if constexpr (CUTS) {
-    uint64_t* h = rs.hist[wave & 3];
+    uint64_t* h = &rs.hist[0][lane % kCopies];
     int nan = 0;
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -629,7 +674,7 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
         e[g][j] = fixed_exponent(m, x[g][j], kt);
         nan += x[g][j] != x[g][j];
         if (e[g][j] <= kSelAMax)
-          atomicAdd((unsigned long long*)&h[sel_bin(e[g][j])],
+          atomicAdd((unsigned long long*)&h[sel_bin(e[g][j]) * kCopies],
                     (unsigned long long)(count ? 1ull : exponent_weight(e[g][j], sh.exp2)));
       }
     }
@@ -639,8 +684,9 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
       uint64_t b[4], mine = 0;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        b[j] = rs.hist[0][4 * lane + j] + rs.hist[1][4 * lane + j] + rs.hist[2][4 * lane + j] +
-               rs.hist[3][4 * lane + j];
+        b[j] = 0;
+#pragma unroll
+        for (int q = 0; q < kCopies; ++q) b[j] += rs.hist[4 * lane + j][q];
         mine += b[j];
       }
       const uint64_t incl = fg::wave_incl_scan_u64(mine), total = fg::shfl_u64(incl, 63);
@@ -691,29 +737,13 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
       __syncthreads();
       return block_sample<DT>(rowp, V, sp, u, sh);
     }
-    if (count && n <= kSmallList) {
-      const int64_t slots = (int64_t)sp.top_k - rs.nan;
-      const int tok = small_draw(rs.ck, n, slots, sp.tp32, u, m, kt, sh.exp2, rs.small);
+    if (count) {
+      const int tok = list_draw(rs.ck, n, (int64_t)sp.top_k - rs.nan, sp.tp32, u, m, kt, sh.exp2, rs.sel, rs.small);
       __syncthreads();
       return tok;
     }
-    if (count) {
-      const auto kept_sum = [&]() {
-        uint64_t k = 0;
-        for (int i = tid; i < n; i += kThreads)
-          if (rs.ck[i] >= cut) k += weight(fg::rank_key_value(rs.ck[i]));
-        return select_block_sum(k, rs.sel);
-      };
-      cut = list_select<false, false>(rs.ck, n, 0, rs.before, m, kt, sh.exp2, rs.sel);
-      uint64_t total = kept_sum();
-      if (sp.tp32) {
-        cut = list_select<true, false>(rs.ck, n, cut, fg::mulhi_u64_u32(total, sp.tp32), m, kt, sh.exp2, rs.sel);
-        total = kept_sum();
-      }
-      return (int)fg::rank_key_index(
-          list_select<true, true>(rs.ck, n, cut, fg::mulhi_u64_u32(total, u), m, kt, sh.exp2, rs.sel));
-    }
-    cut = list_select<true, false>(rs.ck, n, 0, rs.before, m, kt, sh.exp2, rs.sel);
+    cut = n <= kSmallList ? small_cut(rs.ck, n, rs.before, m, kt, sh.exp2, rs.small)
+                          : list_select<true, false>(rs.ck, n, 0, rs.before, m, kt, sh.exp2, rs.sel);
     for (uint64_t rest = hit; rest; rest &= rest - 1) {
       const int i = index_of(__builtin_ctzll(rest));
       if (fg::rank_key(fg::load_elem<DT>(rowp, i), (uint32_t)i) < cut) hit &= ~(rest & -rest);
@@ -997,6 +1027,7 @@ struct SplitArgs {
   struct SelState* sel;      // [rows]
   uint64_t* part_a;          // [rows, kSplitChunks] q-mass above the cut's bin
   int32_t* part_nan;         // [rows, kSplitChunks] NaN count
+  int32_t* part_n;           // the same words: listed candidates (short top-k)
   uint32_t* list;            // [rows, kSelList] indices of the elements around the cut
   int32_t* list_n;           // [rows] listed elements (may exceed kSelList: then not all are there)
 };
@@ -1039,11 +1070,11 @@ FG_DEVICE void split_load8(const char* p, int i0, int hi, float (&x)[8]) {
   for (int j = 0; j < 8; ++j) x[j] = i0 + j < hi ? fg::load_elem<DT>(p, i0 + j) : -INFINITY;
 }
 
-// Chunk maxima (raw maximum, NaN ignored, and the first-maximum rank key). Per pass a thread
+// Chunk maxima (raw maximum, NaN ignored, and with KEY the first-maximum rank key). Per pass a thread
 // takes the maximum of its elements (NaN ignored) and then the first index holding it (the
 // first NaN when there is one, which ranks highest), and forms one rank key per pass instead
 // of one per element.
-template <int DT>
+template <int DT, bool KEY>
 __global__ void __launch_bounds__(kSplitThreads) split_max_kernel(SplitArgs a) {
   const int c = blockIdx.x, r = blockIdx.y;
   if (split_skip(a, r)) return;
@@ -1071,6 +1102,10 @@ __global__ void __launch_bounds__(kSplitThreads) split_max_kernel(SplitArgs a) {
         nan |= x[u][j] != x[u][j];
       }
     }
+    if constexpr (!KEY) {
+      mx = fmaxf(mx, pm);
+      continue;
+    }
     int first = -1;
     float kv = pm;
 #pragma unroll
@@ -1088,7 +1123,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_max_kernel(SplitArgs a) {
     }
   }
   mx = fg::wave_max(mx);
-  best = fg::wave_max_u64(best);
+  if constexpr (KEY) best = fg::wave_max_u64(best);
   const int wave = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
     smax[wave] = mx;
@@ -1102,7 +1137,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_max_kernel(SplitArgs a) {
       best = skey[w] > best ? skey[w] : best;
     }
     a.part_max[r * kSplitChunks + c] = fmaxf(smax[0], mx);
-    a.part_key[r * kSplitChunks + c] = skey[0] > best ? skey[0] : best;
+    if constexpr (KEY) a.part_key[r * kSplitChunks + c] = skey[0] > best ? skey[0] : best;
   }
 }
 
@@ -1198,43 +1233,45 @@ __global__ void __launch_bounds__(kSplitThreads) split_sum_kernel(SplitArgs a) {
   }
 }
 
-// First index in [lo, hi) whose inclusive running q-mass exceeds target (the whole
-// block; -1 if none), scanned in index order one group of kSplitThreads x 8 elements at a
+// First index in [lo, hi) whose inclusive running mass w(x, index) exceeds target (the whole
+// block of THREADS; -1 if none), scanned in index order one group of THREADS x 8 elements at a
 // time (thread t holds 8 consecutive elements of a group), stopping at the group that holds
-// the target: on average half the chunk is weighed. A pass's groups are loaded together.
-template <int DT>
-FG_DEVICE int split_locate(const char* p, int lo, int hi, float m, float kt, const uint64_t* tbl, uint64_t target,
-                           uint64_t* wsum, int* found) {
+// the target. The LOADS groups of a pass are loaded together. wsum: THREADS / 64 words.
+template <int DT, int THREADS, int LOADS, class W>
+FG_DEVICE int split_locate(const char* p, int lo, int hi, W&& weight, uint64_t target, uint64_t* wsum, int* found) {
+  constexpr int WAVES = THREADS / 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (tid == 0) *found = -1;
   uint64_t run = 0;  // block-uniform
   bool done = false;
-  for (int base = lo; base < hi && !done; base += kSplitPass) {
-    float x[kSplitLoads][8];
+  for (int base = lo; base < hi && !done; base += THREADS * 8 * LOADS) {
+    float x[LOADS][8];
 #pragma unroll
-    for (int u = 0; u < kSplitLoads; ++u)
-      if (split_group_live(base, u, hi)) split_load8<DT>(p, base + (u * kSplitThreads + tid) * 8, hi, x[u]);
+    for (int u = 0; u < LOADS; ++u)
+      if (base + u * THREADS * 8 < hi) split_load8<DT>(p, base + (u * THREADS + tid) * 8, hi, x[u]);
 #pragma unroll
-    for (int u = 0; u < kSplitLoads; ++u) {
-      if (!split_group_live(base, u, hi)) break;  // uniform
-      const uint64_t mine = split_weight8(x[u], kt, m, tbl);
+    for (int u = 0; u < LOADS; ++u) {
+      if (base + u * THREADS * 8 >= hi) break;  // uniform
+      const int i0 = base + (u * THREADS + tid) * 8;
+      uint64_t mine = 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) mine += weight(x[u][j], i0 + j);
       const uint64_t incl = fg::wave_incl_scan_u64(mine);
       __syncthreads();  // wsum of the previous group has been read
       if (lane == 63) wsum[wave] = incl;
       __syncthreads();
       uint64_t woff = 0, stot = 0;
-#pragma unroll
-      for (int w = 0; w < kSplitWaves; ++w) {
+#pragma unroll 4
+      for (int w = 0; w < WAVES; ++w) {
         if (w < wave) woff += wsum[w];
         stot += wsum[w];
       }
       if (run + stot > target) {  // uniform: this group holds the target
         uint64_t cum = run + woff + incl - mine;
         if (cum <= target && target < cum + mine) {
-          const int i0 = base + (u * kSplitThreads + tid) * 8;
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            cum += fg::weight_q40(m, x[u][j], kt, tbl);
+            cum += weight(x[u][j], i0 + j);
             if (cum > target) {
               *found = i0 + j;
               break;
@@ -1342,8 +1379,10 @@ __global__ void __launch_bounds__(kSplitThreads) split_pick_kernel(SplitArgs a, 
         clo += q * kSplitGroup;
         chi = min(chi, clo + kSplitGroup);
       }
-      const int idx = split_locate<DT>(split_row<DT>(a, r), clo, chi, a.row_m[r], split_kt(a), tbl, target - before,
-                                       wsum, &s_found);
+      const float m = a.row_m[r], kt = split_kt(a);
+      const int idx = split_locate<DT, kSplitThreads, kSplitLoads>(
+          split_row<DT>(a, r), clo, chi, [&](float x, int) { return fg::weight_q40(m, x, kt, tbl); }, target - before,
+          wsum, &s_found);
       if (idx >= 0) tok = idx;  // always: the chunk holds the target
     }
   }
@@ -1358,8 +1397,8 @@ __global__ void __launch_bounds__(kSplitThreads) split_pick_kernel(SplitArgs a, 
 }
 
 // ------------------------------------------------------------------ split top-k / top-p
-// Restricted draws over kSplitChunks workgroups per row, four launches, the same integer rule
-// as block_sample:
+// Restricted draws over kSplitChunks workgroups per row, four launches (two for a short top-k, see
+// split_topk_kernel), the same integer rule as block_sample:
 //  (1) chunk maxima (split_max_kernel), unless the row's maxima parts are given;
 //  (2) per chunk, a histogram over the bins of the fixed-point exponent: q-mass for top-p,
 //      counts for top-k;
@@ -1376,8 +1415,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_pick_kernel(SplitArgs a, 
 // bits needed four histogram launches instead of one: the first level's 256 bins are the sign
 // and exponent bits, so nearly every LDS atomic hit the same few words (17 us per level at
 // 64 x 152,064), and a bf16 row's last two levels had nothing left to separate. Measured, a draw:
-// top-p 0.95 at 64 x 152,064 bf16 114 -> 57 us (seven launches before); top-k 50 at
-// 32 x 151,936 bf16 210 -> 47 us (one workgroup per row before).
+// top-p 0.95 at 64 x 152,064 bf16 114 -> 50 us (seven launches before).
 static_assert(kSelBins == kSplitThreads, "one histogram bin per thread");
 
 // Where the cut of one row lies (written by chunk 0 of launch 3).
@@ -1385,6 +1423,8 @@ struct SelState {
   uint64_t rest;  // position of the cut within the list: q-mass (top-p) or count (top-k) before it
   int32_t slow;   // the row is drawn by block_sample
   int32_t all;    // every listed element is kept (top-k with no more candidates than slots)
+  int32_t bin;    // the cut's bin
+  int32_t pad;
 };
 
 template <int DT, bool COUNT>
@@ -1394,7 +1434,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) 
   using Bin = std::conditional_t<COUNT, uint32_t, uint64_t>;
   using AtomicBin = std::conditional_t<COUNT, unsigned int, unsigned long long>;
   __shared__ uint64_t tbl[COUNT ? 1 : 1024];
-  __shared__ Bin h[kSplitWaves][kSelBins];  // one copy per wave: fewer waves meet on a word
+  __shared__ Bin h[kSelBins][kCopies];
   __shared__ float smax[kSplitWaves];
   __shared__ int s_nan;
   const char* p = split_row<DT>(a, r);
@@ -1405,7 +1445,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) 
     if (split_group_live(lo, u, hi)) split_load8<DT>(p, lo + (u * kSplitThreads + tid) * 8, hi, x[u]);
   if constexpr (!COUNT) fg::exp2_table_to_lds(tbl);
 #pragma unroll
-  for (int w = 0; w < kSplitWaves; ++w) h[w][tid] = 0;
+  for (int q = 0; q < kCopies; ++q) (&h[0][0])[q * kSplitThreads + tid] = 0;
   if (tid == 0) s_nan = 0;
   float mx = -INFINITY;  // row maximum from the parts
   for (int q = tid; q < a.src_parts; q += kSplitThreads) mx = fmaxf(mx, a.src_max[r * a.src_stride + q]);
@@ -1416,7 +1456,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) 
 #pragma unroll
   for (int w = 1; w < kSplitWaves; ++w) mx = fmaxf(mx, smax[w]);
   const float m = mx, kt = split_kt(a);
-  Bin* mine = h[tid >> 6];
+  Bin* mine = &h[0][tid % kCopies];
   int nan = 0;
   for (int base = lo; base < hi; base += kSplitPass) {
     if (base != lo) {
@@ -1433,7 +1473,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) 
         if constexpr (COUNT) nan += x[u][j] != x[u][j];
         if (e <= kSelAMax) {
           const Bin w = COUNT ? (Bin)1 : (Bin)fg::weight_q40(m, x[u][j], kt, tbl);
-          atomicAdd((AtomicBin*)&mine[sel_bin(e)], (AtomicBin)w);
+          atomicAdd((AtomicBin*)&mine[sel_bin(e) * kCopies], (AtomicBin)w);
         }
       }
     }
@@ -1444,7 +1484,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) 
   __syncthreads();
   Bin t = 0;
 #pragma unroll
-  for (int w = 0; w < kSplitWaves; ++w) t += h[w][tid];
+  for (int q = 0; q < kCopies; ++q) t += h[tid][q];
   a.hist[((size_t)r * kSplitChunks + c) * kSelBins + tid] = t;
   if (tid == 0) {
     if constexpr (COUNT) a.part_nan[r * kSplitChunks + c] = s_nan;
@@ -1516,7 +1556,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_gather_kernel(SplitArgs a
   }
   __syncthreads();
   const int bin = s_bin;
-  if (c == 0 && tid == 0) a.sel[r] = SelState{slow ? 0 : COUNT ? target : target - s_before, slow, all};
+  if (c == 0 && tid == 0) a.sel[r] = SelState{slow ? 0 : COUNT ? target : target - s_before, slow, all, bin, 0};
   if (slow) return;
   if constexpr (!COUNT) {  // this chunk's q-mass above the cut's bin
     uint64_t above;
@@ -1557,35 +1597,13 @@ __global__ void __launch_bounds__(kSplitThreads) split_gather_kernel(SplitArgs a
   }
 }
 
-// Elements of a row at or above a cut rank key, for block_sum / block_locate over a chunk that
-// starts at vocabulary index lo.
-struct KeptFrom {
-  uint64_t cut;
-  uint32_t lo;
-  FG_DEVICE bool operator()(uint32_t key, uint32_t i) const {
-    return (((uint64_t)key << 32) | (uint64_t)(0xffffffffu - (lo + i))) >= cut;
-  }
-};
-
-template <int DT>
-FG_DEVICE Row<DT> chunk_row(const SplitArgs& a, int r, int c, const uint64_t* tbl) {
-  const int lo = c * a.chunk;
-  Row<DT> rr;
-  rr.p = split_row<DT>(a, r) + (int64_t)lo * (DT == fg::kBF16 ? 2 : 4);
-  rr.V = max(0, min(a.vocab, lo + a.chunk) - lo);
-  rr.seg = (((rr.V + kWaves - 1) / kWaves) + kStep - 1) / kStep * kStep;
-  rr.kt = split_kt(a);
-  rr.tbl = tbl;
-  rr.m = a.row_m[r];
-  return rr;
-}
-
 template <int DT, bool COUNT, bool WALK>
 __global__ void __launch_bounds__(kThreads) split_select_kernel(SplitArgs a, DrawOut d, SampleParams sp) {
   __shared__ Shared sh;
   __shared__ SelectShared sel;
+  __shared__ SmallShared small;
   __shared__ uint64_t ck[kSelList];
-  __shared__ unsigned long long s_kept[kSplitChunks];
+  __shared__ uint64_t s_kept[kSplitChunks][kCopies];  // kept q-mass per chunk
   const int r = blockIdx.x, tid = threadIdx.x;
   if constexpr (WALK) {
     if (!d.state[d.batch + r]) return;
@@ -1612,49 +1630,208 @@ __global__ void __launch_bounds__(kThreads) split_select_kernel(SplitArgs a, Dra
       ck[i] = fg::rank_key(fg::load_elem<DT>(rowp, idx), idx);
     }
     fg::exp2_table_to_lds(sh.exp2);
-    if (tid < kSplitChunks) s_kept[tid] = 0;
+    if (!COUNT && tid < kSplitChunks * kCopies)
+      s_kept[tid / kCopies][tid % kCopies] = tid % kCopies ? 0ull : a.part_a[r * kSplitChunks + tid / kCopies];
     __syncthreads();
-    const auto weight = [&](uint64_t k) { return fg::weight_q40(m, fg::rank_key_value(k), kt, sh.exp2); };
     if constexpr (COUNT) {
-      uint64_t cut = 0, kept = 0;
-      if (!st.all) cut = list_select<false, false>(ck, n, 0, st.rest, m, kt, sh.exp2, sel);
-      for (int i = tid; i < n; i += kThreads)
-        if (ck[i] >= cut) kept += weight(ck[i]);
-      uint64_t total = select_block_sum(kept, sel);
-      if (sp.tp32) {
-        cut = list_select<true, false>(ck, n, cut, fg::mulhi_u64_u32(total, sp.tp32), m, kt, sh.exp2, sel);
-        kept = 0;
-        for (int i = tid; i < n; i += kThreads)
-          if (ck[i] >= cut) kept += weight(ck[i]);
-        total = select_block_sum(kept, sel);
-      }
-      const uint64_t low = list_select<true, true>(ck, n, cut, fg::mulhi_u64_u32(total, u), m, kt, sh.exp2, sel);
-      tok = (int)fg::rank_key_index(low);
+      tok = list_draw(ck, n, st.all ? (int64_t)n : (int64_t)st.rest + 1, sp.tp32, u, m, kt, sh.exp2, sel, small);
     } else {
-      const uint64_t cut = list_select<true, false>(ck, n, 0, st.rest, m, kt, sh.exp2, sel);
+      const uint64_t cut = n <= kSmallList ? small_cut(ck, n, st.rest, m, kt, sh.exp2, small)
+                                           : list_select<true, false>(ck, n, 0, st.rest, m, kt, sh.exp2, sel);
+      const int bin = st.bin;
       for (int i = tid; i < n; i += kThreads)
         if (ck[i] >= cut)
-          atomicAdd(&s_kept[fg::rank_key_index(ck[i]) / (uint32_t)a.chunk], (unsigned long long)weight(ck[i]));
+          atomicAdd((unsigned long long*)&s_kept[fg::rank_key_index(ck[i]) / (uint32_t)a.chunk][tid % kCopies],
+                    (unsigned long long)fg::weight_q40(m, fg::rank_key_value(ck[i]), kt, sh.exp2));
       __syncthreads();
-      uint64_t total = 0;
-      for (int c = 0; c < kSplitChunks; ++c) total += a.part_a[r * kSplitChunks + c] + s_kept[c];
-      const uint64_t target = fg::mulhi_u64_u32(total, u);
-      uint64_t before = 0;
-      int c2 = kSplitChunks - 1;
-      for (int c = 0; c < kSplitChunks; ++c) {
-        const uint64_t kc = a.part_a[r * kSplitChunks + c] + s_kept[c];
-        if (before + kc > target) {
-          c2 = c;
-          break;
-        }
-        before += kc;
-      }
-      const Row<DT> rr = chunk_row<DT>(a, r, c2, sh.exp2);
-      const KeptFrom kept{cut, (uint32_t)(c2 * a.chunk)};
-      block_sum<true, DT>(rr, kept, sh);
-      tok = c2 * a.chunk + block_locate<true, DT>(rr, kept, target - before, sh);
+      // every wave: lane l holds chunk l's kept mass
+      uint64_t kept = 0;
+      if ((tid & 63) < kSplitChunks)
+#pragma unroll
+        for (int q = 0; q < kCopies; ++q) kept += s_kept[tid & 63][q];
+      const uint64_t incl = fg::wave_incl_scan_u64(kept), target = fg::mulhi_u64_u32(fg::shfl_u64(incl, 63), u);
+      const int c2 = (int)__builtin_ctzll(__ballot(target < incl));  // the total exceeds the target
+      const uint64_t before = fg::shfl_u64(incl - kept, c2);
+      const auto kept_weight = [&](float x, int i) -> uint64_t {
+        const uint32_t e = fixed_exponent(m, x, kt);
+        const int b = sel_bin(e);
+        return b < bin || (b == bin && fg::rank_key(x, (uint32_t)i) >= cut) ? exponent_weight(e, sh.exp2) : 0ull;
+      };
+      tok = split_locate<DT, kThreads, 2>(rowp, c2 * a.chunk, min(a.vocab, (c2 + 1) * a.chunk), kept_weight,
+                                          target - before, sh.wsum, &sh.i32b[0]);
     }
   }
+  if constexpr (WALK) {
+    if (tid < 64)
+      walk_apply(r, tok, d.state[r], d.tree_tokens, d.parents, d.n_nodes, d.nmax, d.batch, d.walk_step, d.acc_tokens,
+                 d.acc_nodes, d.acc_stride, d.acc_len, d.last_node, d.correction, d.state, d.err_flag, d.next_rows,
+                 d.next_active);
+  } else {
+    if (tid == 0) d.out[r] = tok;
+  }
+}
+
+// Short top-k (top_k <= kTopkMax, rows of one pass per chunk) in two launches and without the row
+// maximum. Each chunk takes the maxima of 512 disjoint sets of its elements (two per thread): the
+// top_k-th largest of them bounds the chunk's own top_k-th element from below, and listing the
+// elements from there on lists little more than top_k. One workgroup per row draws among the
+// lists, dropping first what lies below (a) some chunk's bound or (b) the least of the
+// chunks' bounds on their ceil(top_k / 16)-th elements: at least top_k elements of the row lie at
+// or above either. Elements 40 octaves below the chunk's maximum and -inf weigh 0 against any
+// row maximum and are not listed; NaN, which ranks first, always is. A chunk with more than
+// kTopkList candidates (long ties) sends the row to block_sample.
+// Bound by launch and memory latency: top-k 50 at 32 x 151,936 bf16 took 207 us in one workgroup per
+// row, 47 with the four launches above, 25 with these two.
+constexpr int kTopkMax = 256;
+constexpr int kTopkList = kSelList / kSplitChunks;  // list entries per chunk
+
+template <int DT>
+__global__ void __launch_bounds__(kSplitThreads) split_topk_kernel(SplitArgs a) {
+  const int c = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, wave = tid >> 6;
+  if (split_skip(a, r)) return;
+  __shared__ uint32_t h[kSelBins];
+  __shared__ float smax[kSplitWaves], slow[2][kSplitWaves];
+  __shared__ uint64_t wsum[kSplitWaves];
+  __shared__ int s_bin[2];
+  const char* p = split_row<DT>(a, r);
+  const int lo = c * a.chunk, hi = min(a.vocab, lo + a.chunk);
+  float x[kSplitLoads][8];
+#pragma unroll
+  for (int u = 0; u < kSplitLoads; ++u)
+    if (split_group_live(lo, u, hi)) split_load8<DT>(p, lo + (u * kSplitThreads + tid) * 8, hi, x[u]);
+  h[tid] = 0;
+  if (tid < 2) s_bin[tid] = kSelBins;
+  float sm[2] = {-INFINITY, -INFINITY};  // maxima of this thread's two sets
+#pragma unroll
+  for (int u = 0; u < kSplitLoads; ++u) {
+    if (!split_group_live(lo, u, hi)) continue;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sm[j >> 2] = fmaxf(sm[j >> 2], x[u][j]);
+  }
+  float m = fg::wave_max(fmaxf(sm[0], sm[1]));
+  if ((tid & 63) == 0) smax[wave] = m;
+  __syncthreads();
+  m = smax[0];
+#pragma unroll
+  for (int w = 1; w < kSplitWaves; ++w) m = fmaxf(m, smax[w]);
+  const float kt = split_kt(a);
+  // bin of a set's maximum, kSelBins for one that weighs 0 against any maximum from m on
+  int sb[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const uint32_t e = fixed_exponent(m, sm[q], kt);
+    sb[q] = e <= kSelAMax ? sel_bin(e) : kSelBins;
+    if (sb[q] < kSelBins) atomicAdd(&h[sb[q]], 1u);
+  }
+  __syncthreads();
+  const uint64_t v = h[tid];
+  uint64_t total;
+  const uint64_t incl = split_incl_scan(v, wsum, total);
+  const uint64_t want[2] = {(uint64_t)a.top_k, (uint64_t)((a.top_k + kSplitChunks - 1) / kSplitChunks)};
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+    if (incl - v < want[q] && want[q] <= incl) s_bin[q] = tid;  // none when there are fewer sets with weight
+  __syncthreads();
+  // the least set maximum in the bins up to that one: at least want[q] elements reach it
+  float t[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    float l = INFINITY;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) l = sb[k] <= s_bin[q] && sb[k] < kSelBins ? fminf(l, sm[k]) : l;
+    l = -fg::wave_max(-l);
+    if ((tid & 63) == 0) slow[q][wave] = l;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    t[q] = slow[q][0];
+#pragma unroll
+    for (int w = 1; w < kSplitWaves; ++w) t[q] = fminf(t[q], slow[q][w]);
+    if (s_bin[q] == kSelBins) t[q] = -INFINITY;
+  }
+  uint64_t hit = 0;  // listed elements
+#pragma unroll
+  for (int u = 0; u < kSplitLoads; ++u) {
+    if (!split_group_live(lo, u, hi)) continue;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float xv = x[u][j];
+      if (xv != xv || (xv >= t[0] && fixed_exponent(m, xv, kt) <= kSelAMax)) hit |= 1ull << (8 * u + j);
+    }
+  }
+  uint64_t count;
+  int o = (int)split_incl_scan((uint64_t)__popcll(hit), wsum, count) - __popcll(hit);
+  const size_t at = ((size_t)r * kSplitChunks + c) * kTopkList;
+  for (; hit; hit &= hit - 1, ++o) {
+    const int bit = __builtin_ctzll(hit);
+    const int i = lo + ((bit >> 3) * kSplitThreads + tid) * 8 + (bit & 7);
+    if (o < kTopkList) a.list[at + o] = (uint32_t)i;
+  }
+  if (tid == 0) {
+    a.part_n[r * kSplitChunks + c] = (int32_t)count;
+    a.part_key[r * kSplitChunks + c] = ((uint64_t)fg::sort_key32(t[0]) << 32) | fg::sort_key32(t[1]);
+    a.part_max[r * kSplitChunks + c] = m;
+  }
+}
+
+template <int DT, bool WALK>
+__global__ void __launch_bounds__(kThreads) split_topk_draw_kernel(SplitArgs a, DrawOut d, SampleParams sp) {
+  static_assert(kWaves == kSplitChunks, "one wave per chunk list");
+  __shared__ Shared sh;
+  __shared__ SelectShared sel;
+  __shared__ SmallShared small;
+  __shared__ uint64_t ck[kSelList];
+  __shared__ int s_n;
+  const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, c = tid >> 6;
+  if constexpr (WALK) {
+    if (!d.state[d.batch + r]) return;
+  } else {
+    if (a.forced && a.forced[r] >= 0) {
+      if (tid == 0) d.out[r] = a.forced[r];
+      return;
+    }
+  }
+  const char* rowp = split_row<DT>(a, r);
+  const size_t at = ((size_t)r * kSplitChunks + c) * kTopkList;
+  uint32_t idx = a.list[at + lane];  // the first entries, before their count is known
+  const int mine = a.part_n[r * kSplitChunks + c];
+  const uint32_t seq = d.seq_ids ? (uint32_t)d.seq_ids[r] : (uint32_t)r;
+  const int ws = WALK ? d.walk_step : 0;
+  const uint32_t u = noise_value(d.noise, (int64_t)r * d.noise_stride + d.noise_col + ws, d.seed, d.step, seq,
+                                 (uint32_t)(d.draw + ws));
+  float m = lane < kSplitChunks ? a.part_max[r * kSplitChunks + lane] : -INFINITY;
+  const uint64_t bounds = a.part_key[r * kSplitChunks + (lane & (kSplitChunks - 1))];
+  m = fg::wave_max(m);
+  uint32_t hi_key = (uint32_t)(bounds >> 32), lo_key = (uint32_t)bounds;
+#pragma unroll
+  for (int q = kSplitChunks / 2; q > 0; q >>= 1) {
+    hi_key = max(hi_key, (uint32_t)__shfl_xor((int)hi_key, q, 64));
+    lo_key = min(lo_key, (uint32_t)__shfl_xor((int)lo_key, q, 64));
+  }
+  const uint64_t floor = (uint64_t)max(hi_key, lo_key) << 32;
+  fg::exp2_table_to_lds(sh.exp2);
+  if (tid == 0) s_n = 0;
+  const bool full = __syncthreads_or(mine > kTopkList) != 0;
+  if (!full)
+    for (int o = lane;;) {
+      const uint64_t key = o < mine ? fg::rank_key(fg::load_elem<DT>(rowp, idx), idx) : 0ull;
+      const bool in = o < mine && key >= floor;
+      const uint64_t mask = __ballot(in);
+      int base = 0;
+      if (lane == 0 && mask) base = atomicAdd(&s_n, (int)__popcll(mask));
+      base = __shfl(base, 0, 64);
+      if (in) ck[base + (int)__popcll(mask & ((1ull << lane) - 1))] = key;
+      o += 64;
+      if (o - lane >= mine) break;  // wave-uniform
+      idx = a.list[at + min(o, kTopkList - 1)];
+    }
+  __syncthreads();
+  int tok = -1;
+  if (!full && s_n > 0)
+    tok = list_draw(ck, s_n, sp.top_k, sp.tp32, u, m, split_kt(a), sh.exp2, sel, small);
+  __syncthreads();
+  if (tok < 0) tok = block_sample<DT>(rowp, a.vocab, sp, u, sh);
   if constexpr (WALK) {
     if (tid < 64)
       walk_apply(r, tok, d.state[r], d.tree_tokens, d.parents, d.n_nodes, d.nmax, d.batch, d.walk_step, d.acc_tokens,
@@ -1669,7 +1846,12 @@ template <int DT, bool COUNT, bool WALK>
 void split_select_launch(const SplitArgs& a, const DrawOut& d, const SampleParams& sp, int rows, bool with_max,
                          hipStream_t s) {
   const dim3 grid(kSplitChunks, rows), block(kSplitThreads);
-  if (with_max) hipLaunchKernelGGL(split_max_kernel<DT>, grid, block, 0, s, a);
+  if (COUNT && sp.top_k <= kTopkMax && a.chunk <= kSplitPass) {
+    hipLaunchKernelGGL(split_topk_kernel<DT>, grid, block, 0, s, a);
+    hipLaunchKernelGGL((split_topk_draw_kernel<DT, WALK>), dim3(rows), dim3(kThreads), 0, s, a, d, sp);
+    return;
+  }
+  if (with_max) hipLaunchKernelGGL((split_max_kernel<DT, false>), grid, block, 0, s, a);
   hipLaunchKernelGGL((split_hist_kernel<DT, COUNT>), grid, block, 0, s, a);
   hipLaunchKernelGGL((split_gather_kernel<DT, COUNT>), grid, block, 0, s, a);
   hipLaunchKernelGGL((split_select_kernel<DT, COUNT, WALK>), dim3(rows), dim3(kThreads), 0, s, a, d, sp);
@@ -1692,7 +1874,8 @@ void split_select(int dtype, const SplitArgs& a, const DrawOut& d, const SampleP
 // chunk sums (not for greedy draws), the pick (1 to 3 launches).
 template <int DT, bool WALK>
 void split_draw(const SplitArgs& a, const DrawOut& d, int rows, bool with_max, hipStream_t s) {
-  if (with_max) hipLaunchKernelGGL(split_max_kernel<DT>, dim3(kSplitChunks, rows), dim3(kSplitThreads), 0, s, a);
+  if (with_max)
+    hipLaunchKernelGGL((split_max_kernel<DT, true>), dim3(kSplitChunks, rows), dim3(kSplitThreads), 0, s, a);
   if (!a.greedy) hipLaunchKernelGGL(split_sum_kernel<DT>, dim3(kSplitChunks, rows), dim3(kSplitThreads), 0, s, a);
   hipLaunchKernelGGL((split_pick_kernel<DT, WALK>), dim3(rows), dim3(kSplitThreads), 0, s, a, d);
 }
@@ -1758,6 +1941,7 @@ bool split_setup(SplitArgs& a, void* workspace, size_t bytes, int rows, const vo
   a.part_a = cut ? a.hist + chunks * kSelBins : nullptr;
   a.sel = cut ? (SelState*)(a.part_a + chunks) : nullptr;
   a.part_nan = cut ? (int32_t*)(a.sel + rows) : nullptr;
+  a.part_n = a.part_nan;
   a.list = cut ? (uint32_t*)(a.part_nan + chunks) : nullptr;
   a.list_n = cut ? (int32_t*)(a.list + (size_t)rows * kSelList) : nullptr;
   a.src_max = a.part_max;
