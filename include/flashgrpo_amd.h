@@ -225,6 +225,11 @@ int fg_linear_rope_kv_write(const void* x, int64_t ldx, const void* w_pairs, int
                             int64_t cache_head_stride, int capacity, const int32_t* row_map, int32_t* err_flag,
                             void* stream);
 
+/* dst[i] = src[i] (bytes[i] bytes, a positive multiple of 4, 4-byte aligned device addresses, no
+ * overlaps) for i < count <= 8, in one launch; src, dst and bytes are host arrays. No counterpart in the
+ * reference: it brings a captured verify forward's inputs into the graph's static buffers. */
+int fg_copy_arrays(const void* const* src, void* const* dst, const int64_t* bytes, int count, void* stream);
+
 /* out[r] = [LayerNorm(state[r]) * state_w + state_b, LayerNorm(token[r]) * token_w + token_b]
  * ([rows, 2*hidden], row stride 2*hidden): the ChainDraftCell's normalised inputs side by side.
  * Weights and biases in the row dtype; hidden % 8 == 0, hidden <= 8192, 16-byte aligned rows. */

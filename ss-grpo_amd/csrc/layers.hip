@@ -293,6 +293,24 @@ __global__ void __launch_bounds__(256) chain_cell_norm_kernel(const void* __rest
   }
 }
 
+// Up to kCopyMax small arrays in one launch, one workgroup row per array (blockIdx.y), 4-byte words.
+// Replaces one copy engine launch per array: the inputs of a captured forward (tokens, offsets,
+// masks, lengths, rows: at most a few KB each) took 13.0 us as four copies, 4.0 this way.
+constexpr int kCopyMax = 8;
+
+struct CopyArgs {
+  const uint32_t* src[kCopyMax];
+  uint32_t* dst[kCopyMax];
+  int64_t words[kCopyMax];
+};
+
+__global__ void __launch_bounds__(256) copy_arrays_kernel(CopyArgs a) {
+  const uint32_t* src = a.src[blockIdx.y];
+  uint32_t* dst = a.dst[blockIdx.y];
+  const int64_t n = a.words[blockIdx.y];
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) dst[i] = src[i];
+}
+
 }  // namespace
 
 extern "C" {
@@ -415,6 +433,25 @@ int fg_swiglu(const void* gate_up, void* out, int dtype, int rows, int inter, vo
   else
     hipLaunchKernelGGL(swiglu_kernel<fg::kF32>, grid, dim3(256), 0, s, gate_up, out, inter, total);
   return fg::check_launch("fg_swiglu");
+}
+
+int fg_copy_arrays(const void* const* src, void* const* dst, const int64_t* bytes, int count, void* stream) {
+  FG_REQUIRE(src && dst && bytes && count > 0 && count <= kCopyMax, "fg_copy_arrays: count must be in [1, 8]");
+  CopyArgs a{};
+  int64_t most = 0;
+  for (int i = 0; i < count; ++i) {
+    FG_REQUIRE(src[i] && dst[i], "fg_copy_arrays: null pointer");
+    FG_REQUIRE(bytes[i] > 0 && bytes[i] % 4 == 0 && ((uintptr_t)src[i] & 3) == 0 && ((uintptr_t)dst[i] & 3) == 0,
+               "fg_copy_arrays: arrays must be whole 4-byte words");
+    a.src[i] = (const uint32_t*)src[i];
+    a.dst[i] = (uint32_t*)dst[i];
+    a.words[i] = bytes[i] / 4;
+    most = a.words[i] > most ? a.words[i] : most;
+  }
+  const int64_t blocks = (most + 255) / 256;
+  hipLaunchKernelGGL(copy_arrays_kernel, dim3((unsigned)(blocks < 64 ? blocks : 64), count), dim3(256), 0,
+                     (hipStream_t)stream, a);
+  return fg::check_launch("fg_copy_arrays");
 }
 
 }  // extern "C"

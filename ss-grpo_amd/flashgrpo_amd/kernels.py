@@ -388,6 +388,35 @@ def swiglu(gate_up, *, out=None):
     return out
 
 
+class ArrayCopies:
+    """Copies into a fixed set of at most 8 small device tensors (``fg_copy_arrays``): calling it with
+    one source per destination copies all of them in one launch on the current stream. A source
+    that is not a contiguous tensor of its destination's dtype and device is copied by torch."""
+
+    def __init__(self, dsts):
+        self.dsts = list(dsts)
+        n = len(self.dsts)
+        if not 0 < n <= 8 or any(not d.is_contiguous() or d.numel() == 0 for d in self.dsts):
+            raise ValueError("ArrayCopies: 1 to 8 contiguous non-empty tensors")
+        self.n = n
+        self._all = [(d.dtype, d.shape, d.device, d.numel() * d.element_size()) for d in self.dsts]
+
+    def __call__(self, srcs):
+        fast = []
+        for d, s, (dt, shape, dev, nbytes) in zip(self.dsts, srcs, self._all):
+            if (s.dtype == dt and s.shape == shape and s.device == dev and s.is_contiguous() and dev.type == "cuda"
+                    and nbytes % 4 == 0 and s.data_ptr() % 4 == 0):
+                if s.data_ptr() != d.data_ptr():
+                    fast.append((s.data_ptr(), d.data_ptr(), nbytes))
+            else:
+                d.copy_(s)
+        if not fast:
+            return
+        n = len(fast)
+        a, b, c = zip(*fast)
+        _call("fg_copy_arrays", (C.c_void_p * n)(*a), (C.c_void_p * n)(*b), (C.c_int64 * n)(*c), n, _stream())
+
+
 def chain_cell_norm(state, token, state_w, state_b, token_w, token_b, eps, *, out=None):
     """[rows, 2H] = [LayerNorm(state) * state_w + state_b, LayerNorm(token) * token_w + token_b]
     (``fg_chain_cell_norm``): the ChainDraftCell's two normalised inputs side by side. state and

@@ -359,6 +359,8 @@ class _ForwardGraph:
 
     def __init__(self, graphs, inputs, out):
         self.graphs, self.inputs, self.out = graphs, inputs, out
+        self.fill = K.ArrayCopies([inputs[k] for k in ("tokens", "pos", "anc", "seq", "row_map")
+                                   if inputs[k] is not None])
 
     @classmethod
     def capture(cls, model, tokens, cache, pos_offset, anc, seq_len, row_map, err_flag):
@@ -396,13 +398,8 @@ class _ForwardGraph:
         return cls((*graphs, st), inputs, out)
 
     def run(self, tokens, pos_offset, anc, seq_len, row_map):
-        st = self.inputs
-        st["tokens"].copy_(tokens)
-        st["pos"].copy_(pos_offset)
-        st["anc"].copy_(anc)
-        st["seq"].copy_(seq_len)
-        if row_map is not None:
-            st["row_map"].copy_(row_map)
+        srcs = (tokens, pos_offset, anc, seq_len)
+        self.fill(srcs if row_map is None else (*srcs, row_map))
         for g in self.graphs[:-1]:  # the last entry is the capture's forward state
             g.replay()
         return self.out
@@ -684,7 +681,10 @@ class TargetModel:
         if N > MAX_CHAIN_TOKENS:
             raise ValueError(f"at most {MAX_CHAIN_TOKENS} new tokens per forward")
         d = cfg.head_dim
-        x = self.w["embed"].index_select(0, tokens.reshape(-1).long())  # [T, H] residual stream
+        ids = tokens.reshape(-1)
+        if ids.dtype not in (torch.int32, torch.int64):
+            ids = ids.long()
+        x = self.w["embed"].index_select(0, ids)  # [T, H] residual stream
         return dict(x=x, B=B, N=N, cache=cache, pos_offset=pos_offset, anc=anc, seq_len=seq_len, row_map=row_map,
                     err_flag=err_flag, q=self._buf("q", (B, N, cfg.q_heads, d)),
                     attn=self._buf("attn", (B, N, cfg.q_heads, d)))
