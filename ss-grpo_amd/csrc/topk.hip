@@ -6,10 +6,14 @@
 // tree topology (parent, depth, candidate rank of each node) depends only on
 // the plan and is supplied by the host, the kernel fills in the tokens.
 //
-// Phase 1: grid (rows, chunks). Each thread keeps a sorted top-K of 64-bit
-// rank keys over its strided elements (and, optionally, a running max and
-// sum of exp for the row's log-sum-exp); lists merge across the wave with the
-// bitonic "max(A[i], B[K-1-i]) then sort" step, then across waves in LDS.
+// Phase 1: grid (rows, chunks), 10,240 elements per workgroup pass, held in registers. The maxima of
+// at least K disjoint groups of threads bound the pass's K-th element from below, so only the few
+// elements from the least of them on are listed in LDS as 64-bit rank keys and ranked by
+// comparing each with every other; the other elements cost a comparison each, and (optionally)
+// their part of the maximum and sum of exp. A chunk whose list overflows (long ties) keeps a
+// sorted top-K per thread instead, merged with the bitonic "max(A[i], B[K-1-i]) then sort" step.
+// Bound by VALU and HBM about equally: the top-2 with sums of exp of 384 x 128,256 bf16 logits
+// (98 MB) 43.7 us inserting every element into such lists, 31.9 this way; the top-16 275 and 35.
 // Phase 2: one wave per row merges the chunk lists.
 //
 // With `sanitize` the values are first mapped as torch.nan_to_num(x.float(),
@@ -33,6 +37,10 @@ using fg::sanitize;
 using fg::wave_merge;
 
 constexpr int kThreads = 256;
+constexpr int kLoads = 5;                // groups of 8 elements per thread and pass
+constexpr int kGroup = kThreads * 8;
+constexpr int kPass = kGroup * kLoads;   // elements per workgroup pass
+constexpr int kList = 256;               // listed candidates per chunk
 
 template <int DT, int K, bool STATS, bool SAN>
 __global__ void __launch_bounds__(kThreads) topk_phase1(const void* __restrict__ logits, int64_t row_stride,
@@ -44,65 +52,142 @@ __global__ void __launch_bounds__(kThreads) topk_phase1(const void* __restrict__
   const char* rowp = (const char*)logits + (int64_t)row * row_stride * (DT == fg::kBF16 ? 2 : 4);
   const int lo = c * chunk;
   const int hi = min(vocab, lo + chunk);
-  uint64_t top[K];
-#pragma unroll
-  for (int i = 0; i < K; ++i) top[i] = 0;
+  const int tid = threadIdx.x;
+  __shared__ float s_bound[kThreads / 64];
+  __shared__ uint64_t s_list[kList];
+  __shared__ int s_n;
+  if (tid == 0) s_n = 0;
   LseAcc acc{-INFINITY, 0.0f};
-  // Vector body: 8 elements per thread per step; chunk starts are multiples of 8.
-  const int vec_hi = lo + ((hi - lo) & ~7);
-  for (int i = lo + threadIdx.x * 8; i < vec_hi; i += kThreads * 8) {
-    float v[8];
-    fg::load8<DT>(rowp, i, v);
+  for (int base = lo; base < hi; base += kPass) {
+    float x[kLoads][8];
+    // groups wholly past hi are skipped (uniform); the last one is padded with -inf
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = sanitize<SAN>(v[j]);
+    for (int u = 0; u < kLoads; ++u) {
+      if (base + u * kGroup >= hi) continue;
+      const int i0 = base + u * kGroup + tid * 8;
+      if (i0 + 8 <= hi) {
+        fg::load8<DT>(rowp, i0, x[u]);
+      } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) insert_key<K>(top, fg::rank_key(v[j], (uint32_t)(i + j)));
+        for (int j = 0; j < 8; ++j) x[u][j] = i0 + j < hi ? fg::load_elem<DT>(rowp, i0 + j) : -INFINITY;
+      }
+    }
+    float mx = -INFINITY;  // this thread's maximum, NaN ignored
+    bool nan = false;
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      if (base + u * kGroup >= hi) continue;
+      // 0 * x is 0 for a finite x and NaN otherwise
+      float z = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) z = fmaf(x[u][j], 0.0f, z);
+      if (z != z) {  // some non-finite value (or padding)
+        const int i0 = base + u * kGroup + tid * 8;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          if (i0 + j < hi) x[u][j] = sanitize<SAN>(x[u][j]);
+          nan |= x[u][j] != x[u][j];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) mx = fmaxf(mx, x[u][j]);
+    }
+    // bound: at least K of the 4 S groups of 64 / S threads have a maximum from it on, so the pass
+    // has K elements there
+    constexpr int S = K > 4 ? K / 4 : 1;
+    float gm = mx;
+#pragma unroll
+    for (int o = 32 / S; o > 0; o >>= 1) gm = fmaxf(gm, __shfl_xor(gm, o, 64));
+#pragma unroll
+    for (int o = 32; o >= 64 / S; o >>= 1) gm = fminf(gm, __shfl_xor(gm, o, 64));
+    __syncthreads();  // s_bound of the previous pass has been read
+    if ((tid & 63) == 0) s_bound[tid >> 6] = gm;
+    __syncthreads();
+    const float b0 = s_bound[0], b1 = s_bound[1], b2 = s_bound[2], b3 = s_bound[3];
+    const float h01 = fmaxf(b0, b1), l01 = fminf(b0, b1), h23 = fmaxf(b2, b3), l23 = fminf(b2, b3);
+    const float bound = K == 1 ? fmaxf(h01, h23)
+                        : K == 2 ? fmaxf(fminf(h01, h23), fmaxf(l01, l23))  // the second largest
+                                 : fminf(l01, l23);
+    uint64_t hit = 0;
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      if (base + u * kGroup >= hi) continue;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (!(x[u][j] < bound)) hit |= 1ull << (8 * u + j);  // NaN too
+    }
+    for (; hit; hit &= hit - 1) {
+      const int bit = __builtin_ctzll(hit);
+      const int i = base + (bit >> 3) * kGroup + tid * 8 + (bit & 7);
+      if (i >= hi) continue;
+      const int at = atomicAdd(&s_n, 1);
+      if (at < kList) s_list[at] = fg::rank_key(sanitize<SAN>(fg::load_elem<DT>(rowp, i)), (uint32_t)i);
+    }
     if constexpr (STATS) {
-      float m8 = v[0];
+      float s = nan ? __uint_as_float(0x7fc00000u) : 0.0f;
+      if (mx != -INFINITY) {
 #pragma unroll
-      for (int j = 1; j < 8; ++j) m8 = fmaxf(m8, v[j]);
-      float m = fmaxf(acc.m, m8);
-      float s = (acc.m == -INFINITY) ? 0.0f : acc.s * __expf(acc.m - m);
+        for (int u = 0; u < kLoads; ++u) {
+          if (base + u * kGroup >= hi) continue;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s += __expf(v[j] - m);
-      acc = {m, s};
+          for (int j = 0; j < 8; ++j) s += __expf(x[u][j] - mx);
+        }
+      }
+      acc = lse_combine(acc, LseAcc{mx, s});
     }
   }
-  for (int i = vec_hi + threadIdx.x; i < hi; i += kThreads) {
-    float v = sanitize<SAN>(fg::load_elem<DT>(rowp, i));
-    insert_key<K>(top, fg::rank_key(v, (uint32_t)i));
-    if constexpr (STATS) acc = lse_combine(acc, LseAcc{v, 1.0f});
-  }
-  wave_merge<K>(top);
-  __shared__ uint64_t s_top[kThreads / 64][K];
   __shared__ float2 s_lse[kThreads / 64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = tid >> 6, lane = tid & 63;
   if constexpr (STATS) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       LseAcc other{__shfl_xor(acc.m, o, 64), __shfl_xor(acc.s, o, 64)};
       acc = lse_combine(acc, other);
     }
-  }
-  if (lane == 0) {
-#pragma unroll
-    for (int i = 0; i < K; ++i) s_top[wave][i] = top[i];
-    s_lse[wave] = make_float2(acc.m, acc.s);
+    if (lane == 0) s_lse[wave] = make_float2(acc.m, acc.s);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int w = 1; w < kThreads / 64; ++w) {
-      uint64_t other[K];
-#pragma unroll
-      for (int i = 0; i < K; ++i) other[i] = s_top[w][i];
-      merge_desc<K>(top, other);
-      if constexpr (STATS) acc = lse_combine(acc, LseAcc{s_lse[w].x, s_lse[w].y});
+  const int n = s_n;
+  uint64_t* out = part_keys + ((int64_t)row * nchunks + c) * K;
+  if (n <= kList) {
+    // rank of key i = how many are larger (the keys are distinct)
+    if (tid < n) {
+      const uint64_t key = s_list[tid];
+      int rank = 0;
+      for (int j = 0; j < n; ++j) rank += s_list[j] > key;
+      if (rank < K) out[rank] = key;
     }
-    uint64_t* out = part_keys + ((int64_t)row * nchunks + c) * K;
+    if (tid >= n && tid < K) out[tid] = 0;
+  } else {
+    __shared__ uint64_t s_top[kThreads / 64][K];
+    uint64_t top[K];
 #pragma unroll
-    for (int i = 0; i < K; ++i) out[i] = top[i];
-    if constexpr (STATS) part_lse[(int64_t)row * nchunks + c] = make_float2(acc.m, acc.s);
+    for (int i = 0; i < K; ++i) top[i] = 0;
+    for (int i = lo + tid; i < hi; i += kThreads)
+      insert_key<K>(top, fg::rank_key(sanitize<SAN>(fg::load_elem<DT>(rowp, i)), (uint32_t)i));
+    wave_merge<K>(top);
+    if (lane == 0)
+#pragma unroll
+      for (int i = 0; i < K; ++i) s_top[wave][i] = top[i];
+    __syncthreads();
+    if (tid == 0) {
+#pragma unroll
+      for (int w = 1; w < kThreads / 64; ++w) {
+        uint64_t other[K];
+#pragma unroll
+        for (int i = 0; i < K; ++i) other[i] = s_top[w][i];
+        merge_desc<K>(top, other);
+      }
+#pragma unroll
+      for (int i = 0; i < K; ++i) out[i] = top[i];
+    }
+  }
+  if constexpr (STATS) {
+    if (tid == 0) {
+#pragma unroll
+      for (int w = 1; w < kThreads / 64; ++w) acc = lse_combine(acc, LseAcc{s_lse[w].x, s_lse[w].y});
+      part_lse[(int64_t)row * nchunks + c] = make_float2(acc.m, acc.s);
+    }
   }
 }
 
@@ -394,8 +479,9 @@ int fg_medusa_topk(const void* logits, int dtype, int64_t row_stride, int rows, 
   FG_REQUIRE(row_stride >= vocab && row_stride % 8 == 0, "fg_medusa_topk: row_stride must be >= vocab and a multiple of 8");
   FG_REQUIRE(((uintptr_t)logits & 31) == 0, "fg_medusa_topk: logits must be 32-byte aligned");
   int K = kmax <= 1 ? 1 : kmax <= 2 ? 2 : kmax <= 4 ? 4 : kmax <= 8 ? 8 : 16;
-  // Enough workgroups to cover the chip: ~2048 in total, chunks of >= 2048 elements.
-  int chunks = (2048 + rows - 1) / rows;
+  // Enough workgroups to cover the chip: ~2048 in total, chunks of >= 2048 elements and, up to
+  // 64 chunks, of one pass.
+  int chunks = std::max((2048 + rows - 1) / rows, (vocab + kPass - 1) / kPass);
   chunks = std::max(1, std::min(chunks, std::min(64, (vocab + 2047) / 2048)));
   int chunk = ((vocab + chunks - 1) / chunks + 7) & ~7;
   chunks = (vocab + chunk - 1) / chunk;
