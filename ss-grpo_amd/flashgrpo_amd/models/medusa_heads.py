@@ -63,10 +63,11 @@ class ChainDraftCell(nn.Module):
     def step(self, state, token_embedding):
         """The cell in its parameters' dtype, as ``medusa_heads.py:36-42`` runs it (the
         rollout calls it outside autocast, ``flash_medusa_decoder.py:435-539``): the state
-        and the embedding are cast to that dtype and the new state keeps it. On the GPU the
-        two LayerNorms are one HIP launch (``fg_chain_cell_norm``); the two projections,
-        their sum, SiLU, the output projection and the gated residual are the module's
-        own torch calls, so every intermediate is rounded where the module rounds it."""
+        and the embedding are cast to that dtype and the new state keeps it. On the GPU an
+        fp32 cell is one native call (``fg_chain_cell_step``). Otherwise the two LayerNorms are one
+        HIP launch (``fg_chain_cell_norm``) and the two projections, their sum, SiLU, the
+        output projection and the gated residual are the module's own torch calls, so every
+        bf16 intermediate is rounded where the module rounds it."""
         dt = self.state_norm.weight.dtype
         w = self._weights(dt, state.device)
         H = state.shape[-1]
@@ -77,7 +78,13 @@ class ChainDraftCell(nn.Module):
             from .. import kernels as K
 
             rows = lambda t: t.reshape(-1, H) if t.is_contiguous() else t.reshape(-1, H).contiguous()
-            x = K.chain_cell_norm(rows(s), rows(tok), w["sn_w"], w["sn_b"], w["tn_w"], w["tn_b"], w["eps"])
+            r, t = rows(s), rows(tok)
+            native = [w[k] for k in ("sn_w", "sn_b", "tn_w", "tn_b", "sp_w", "tp_w", "out_w", "out_b")]
+            # the torch form stays where autograd follows the state and where autocast rounds the products
+            if (w["gate"].dtype == torch.float32 and not (torch.is_grad_enabled() and s.requires_grad)
+                    and not torch.is_autocast_enabled("cuda") and K.chain_cell_step_ok(r, t, native)):
+                return K.chain_cell_step(r, t, *native, w["gate"], w["eps"]).view(*s.shape)
+            x = K.chain_cell_norm(r, t, w["sn_w"], w["sn_b"], w["tn_w"], w["tn_b"], w["eps"])
             xs, xt = x[:, :H].view(*s.shape), x[:, H:].view(*s.shape)
         else:
             xs = F.layer_norm(s, (H,), w["sn_w"], w["sn_b"], w["eps"])
