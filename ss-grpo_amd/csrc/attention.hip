@@ -31,7 +31,7 @@
 //  * the ancestor mask is evaluated only on tiles that reach the tree keys, and
 //    the running max (and the O rescale) only moves when a lane's max grows by
 //    more than 2^8, so after the first keys the rescale is almost never taken.
-// fp32 path: one wave per query row, 64 keys per step, exact online softmax in fp32.
+// fp32 path: four waves per query row, a group of lanes per key, exact online softmax in fp32.
 #include "fg_common.h"
 
 #include <algorithm>
@@ -442,67 +442,102 @@ __global__ void __launch_bounds__(256) tree_attn_combine_kernel(AttnArgs a, int 
       make_uint2(fg::pack_bf16x2(o[0] * inv, o[1] * inv), fg::pack_bf16x2(o[2] * inv, o[3] * inv));
 }
 
-// fp32: one wave per (sequence, node, q head), 64 keys per step. Lane j scores key
-// key0 + j (dot product over the head dim from float4 loads against q in LDS); the
-// step's max and sum are wave reductions; PV broadcasts each key's p with v_readlane
-// while lane j accumulates dims j and j + 64 of O (exact online softmax, fp32). All
-// loads of a step are independent and unconditional (addresses clamped to the last
-// key), so each step waits for memory about once per phase.
+// fp32: four waves per (sequence, node, q head). A group of D / 4 lanes takes one key, a lane 4 of its
+// dims, so a wave's 16-byte loads cover 4 (D = 64) or 2 (D = 128) whole K or V rows, and U of each are
+// in flight together. The dot product is a sum over the group's lanes (rotations within 16 lanes),
+// which leaves the score in every lane that then needs its p: no broadcast and no cross-group
+// reduction in the loop. Every group keeps its own running maximum, sum and O (exact online softmax,
+// fp32); the groups of all four waves are merged once, through LDS. A chain row's keys end at its own.
+// Bound by the latency of a step's loads and reductions where rows are few and by the vector ALU (about
+// 32 instructions per 4 keys and row) where they are many. Against one wave per row with a key per
+// lane and 64 keys per step, 8 q and 4 kv heads of 64: 8 sequences x 20 nodes on 256 keys 23.7 -> 13.5
+// us, one node 17.6 -> 6.3, 64 x 32 on 600 keys 383 -> 212, a chunk of 8 x 1024 2352 -> 692 (half of it
+// the chain bound); 16 and 8 heads of 128, 8 x 20 on 256 keys 91.9 -> 35.2.
+constexpr int kF32Waves = 4;
+constexpr int kF32Keys = 8;  // keys of a group per step
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));  // q and V may be dword-aligned only
+
 template <int D>
-__global__ void __launch_bounds__(64) tree_attn_f32_kernel(AttnArgs a) {
-  __shared__ __attribute__((aligned(16))) float qs[D];
+__device__ __forceinline__ float group_sum(float v) {
+#define FG_ROT(ctrl) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xF, 0xF, false))
+  v += FG_ROT(0x128);  // row_ror:8, 4, 2, 1
+  v += FG_ROT(0x124);
+  v += FG_ROT(0x122);
+  v += FG_ROT(0x121);
+#undef FG_ROT
+  if (D == 128) v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));  // lane ^ 16
+  return v;
+}
+
+template <int D>
+__global__ void __launch_bounds__(kF32Waves * 64) tree_attn_f32_kernel(AttnArgs a) {
+  constexpr int L = D / 4, G = 64 / L, U = kF32Keys;  // lanes of a key, keys of a load, loads of a step
+  constexpr int P = kF32Waves * G;                    // partial results
+  __shared__ __attribute__((aligned(16))) float os[P * D];
+  __shared__ float ms[P], ls[P];
   const int qh = blockIdx.x % a.Hq;
   const int n = (blockIdx.x / a.Hq) % a.N;
   const int b = blockIdx.x / (a.Hq * a.N);
-  const int lane = threadIdx.x;
-  const int G = a.Hq / a.Hkv, hkv = qh / G;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane / L, dim = lane % L * 4;
+  const int hkv = qh / (a.Hq / a.Hkv);
   const int s0 = a.seq_len[b];
   const int cb = a.row_map ? a.row_map[b] : b;
-  const float* kbase = (const float*)a.k + (int64_t)cb * a.cache_batch + (int64_t)hkv * a.cache_head;
-  const float* vbase = (const float*)a.v + (int64_t)cb * a.cache_batch + (int64_t)hkv * a.cache_head;
-  const float* qrow = (const float*)a.q + (((int64_t)b * a.N + n) * a.Hq + qh) * D;
+  const float* kbase = (const float*)a.k + (int64_t)cb * a.cache_batch + (int64_t)hkv * a.cache_head + dim;
+  const float* vbase = (const float*)a.v + (int64_t)cb * a.cache_batch + (int64_t)hkv * a.cache_head + dim;
+  const int64_t row = (((int64_t)b * a.N + n) * a.Hq + qh) * D;
   const uint64_t anc = a.anc ? a.anc[(int64_t)b * a.anc_stride + n] : 0ull;
-  for (int j = lane; j < D; j += 64) qs[j] = qrow[j];
-  __syncthreads();
-  float m = -INFINITY, l = 0.0f, o0 = 0.0f, o1 = 0.0f;
-  const int total = min(s0 + a.N, a.capacity);
-  for (int key0 = 0; key0 < total; key0 += 64) {
-    const int key = key0 + lane;
-    const bool ok = key < total && (key < s0 || (a.anc ? ((anc >> (key - s0)) & 1ull) != 0 : key <= s0 + n));
-    const float* kr = kbase + (int64_t)min(key, total - 1) * D;
-    float acc = 0.0f;
+  const float4u q = *(const float4u*)((const float*)a.q + row + dim);
+  const int total = min(s0 + (a.anc ? a.N : n + 1), a.capacity);
+  float m = -INFINITY, l = 0.0f;
+  float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int key0 = wave * G * U; key0 < total; key0 += P * U) {
+    float4 kv[U];
+    float4u vv[U];
 #pragma unroll
-    for (int j = 0; j < D; j += 4) {
-      const float4 kv = *(const float4*)(kr + j);
-      const float4 qv = *(const float4*)(qs + j);
-      acc = fmaf(qv.x, kv.x, acc);
-      acc = fmaf(qv.y, kv.y, acc);
-      acc = fmaf(qv.z, kv.z, acc);
-      acc = fmaf(qv.w, kv.w, acc);
+    for (int u = 0; u < U; ++u)  // unconditional: past the end, the last key's row with p = 0
+      kv[u] = *(const float4*)(kbase + (int64_t)min(key0 + u * G + grp, total - 1) * D);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      vv[u] = *(const float4u*)(vbase + (int64_t)min(key0 + u * G + grp, total - 1) * D);
+    float s[U], m_new = m;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int key = key0 + u * G + grp;
+      const bool ok = key < total && (key < s0 || !a.anc || ((anc >> (key - s0)) & 1ull) != 0);
+      const float dot = group_sum<D>(fmaf(q.w, kv[u].w, fmaf(q.z, kv[u].z, fmaf(q.y, kv[u].y, q.x * kv[u].x))));
+      s[u] = ok ? dot * a.scale : -INFINITY;
+      m_new = fmaxf(m_new, s[u]);
     }
-    const float s = ok ? acc * a.scale : -INFINITY;
-    const float m_new = fmaxf(m, fg::wave_max(s));
-    if (m_new == -INFINITY) continue;  // wave-uniform: no allowed key yet
-    const float alpha = expf(m - m_new);
-    const float p = ok ? expf(s - m_new) : 0.0f;
-    l = l * alpha + fg::wave_sum(p);
-    o0 *= alpha;
-    o1 *= alpha;
-    // Keys past the end carry p = 0 and read the last key's row, so they add 0.
-    const int last = total - 1 - key0;
-    const float* vr = vbase + (int64_t)key0 * D + lane;
+    const float ref = m_new == -INFINITY ? 0.0f : m_new;  // no allowed key yet: every p is 0
+    const float alpha = expf(m - ref);
+    l *= alpha;
+    o.x *= alpha; o.y *= alpha; o.z *= alpha; o.w *= alpha;
 #pragma unroll
-    for (int j = 0; j < 64; ++j) {
-      const float pj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), j));
-      const float* v_ = vr + (int64_t)min(j, last) * D;
-      if (D > 0) o0 = fmaf(pj, lane < D ? v_[0] : 0.0f, o0);
-      if (D > 64) o1 = fmaf(pj, v_[64], o1);
+    for (int u = 0; u < U; ++u) {
+      const float p = expf(s[u] - ref);
+      l += p;
+      o.x = fmaf(p, vv[u].x, o.x);
+      o.y = fmaf(p, vv[u].y, o.y);
+      o.z = fmaf(p, vv[u].z, o.z);
+      o.w = fmaf(p, vv[u].w, o.w);
     }
     m = m_new;
   }
-  float* orow = (float*)a.out + (((int64_t)b * a.N + n) * a.Hq + qh) * D;
-  if (lane < D) orow[lane] = o0 / l;
-  if (lane + 64 < D) orow[lane + 64] = o1 / l;
+  const int part = wave * G + grp;
+  *(float4*)&os[part * D + dim] = o;
+  if (dim == 0) ms[part] = m, ls[part] = l;
+  __syncthreads();
+  if (threadIdx.x >= D) return;
+  float mx = ms[0], den = 0.0f, sum = 0.0f;
+#pragma unroll
+  for (int i = 1; i < P; ++i) mx = fmaxf(mx, ms[i]);
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    const float w = expf(ms[i] - mx);  // a group without keys: 0 (its sums are 0 too)
+    den = fmaf(w, ls[i], den);
+    sum = fmaf(w, os[i * D + threadIdx.x], sum);
+  }
+  ((float*)a.out)[row + threadIdx.x] = sum / den;
 }
 
 
@@ -601,9 +636,9 @@ extern "C" int fg_tree_attention(const void* q, void* out, const void* k_cache, 
     FG_REQUIRE(((uintptr_t)k_cache & 15) == 0 && cache_head_stride % 4 == 0 && cache_batch_stride % 4 == 0,
                "fg_tree_attention: fp32 path needs 16-byte aligned K rows");
     if (head_dim == 64)
-      hipLaunchKernelGGL(tree_attn_f32_kernel<64>, dim3(batch * num_nodes * q_heads), dim3(64), 0, s, a);
+      hipLaunchKernelGGL(tree_attn_f32_kernel<64>, dim3(batch * num_nodes * q_heads), dim3(kF32Waves * 64), 0, s, a);
     else
-      hipLaunchKernelGGL(tree_attn_f32_kernel<128>, dim3(batch * num_nodes * q_heads), dim3(64), 0, s, a);
+      hipLaunchKernelGGL(tree_attn_f32_kernel<128>, dim3(batch * num_nodes * q_heads), dim3(kF32Waves * 64), 0, s, a);
   } else {
     return fg::fail("fg_tree_attention: dtype");
   }

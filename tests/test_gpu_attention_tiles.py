@@ -48,3 +48,30 @@ def test_chain_rows_stop_at_their_own_key(B, Hq, Hkv, N):
         v[b, :, int(seq[b]) + N:] = 1e4
     got = K.tree_attention(q, k, v, seq_len=seq, anc=None, num_nodes=N, q_heads=Hq, kv_heads=Hkv, head_dim=d)
     _close(got, _want(q, k, v, seq, torch.tril(torch.ones(N, N, dtype=torch.bool, device=DEV))))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("prefix", [0, 1, 30, 63, 127, 260])
+@pytest.mark.parametrize("chain", [True, False])
+def test_fp32_key_groups(d, prefix, chain):
+    """Key counts around the steps of the four waves, from one key to several rounds; q and V only
+    dword-aligned; slots behind a row's keys hold what no sum survives."""
+    from flashgrpo_amd import kernels as K
+
+    g = torch.Generator(device=DEV).manual_seed(prefix + d)
+    B, N, Hq, Hkv, cap = 2, 5, 4, 2, 300
+    seq = torch.tensor([prefix, prefix // 2], dtype=torch.int32, device=DEV)
+    n = lambda *s: torch.randn(math.prod(s) + 1, device=DEV, generator=g)[1:].view(*s)
+    q, k, v = n(B, N, Hq, d), n(B, Hkv, cap, d).clone(), n(B, Hkv, cap, d)
+    for b in range(B):
+        k[b, :, int(seq[b]) + N:], v[b, :, int(seq[b]) + N:] = 3e38, float("nan")
+    see = torch.tril(torch.ones(N, N, dtype=torch.bool, device=DEV))
+    anc = None
+    if not chain:  # two branches below node 0
+        see[2, 1] = see[4, 3] = False
+        anc = (see.long() << torch.arange(N, device=DEV)).sum(1).expand(B, N).contiguous()
+    got = K.tree_attention(q, k, v, seq_len=seq, anc=anc, num_nodes=N, q_heads=Hq, kv_heads=Hkv, head_dim=d)
+    want = _want(q, k, v, seq, see)
+    # fp32 scores of d terms and sums of at most 265 keys, each rounded to 2^-24
+    err = (got.double() - want).abs().amax(-1) / want.abs().amax(-1)
+    assert float(err.max()) < (d + 265) * 2.0 ** -24, float(err.max())
