@@ -241,6 +241,14 @@ __global__ void __launch_bounds__(W * 64, 1) lm_stream_kernel(LmArgs a) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[i][nb][v] = 0.0f;
 
+    if constexpr (KT == 0) {
+      // every wave is done with the last round's stages (with top-k its epilogue ends in a barrier)
+      if (rd > 0) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      }
+    }
 #pragma unroll
     for (int h = 0; h < kDist; ++h) {
       issue_x(xb + (h < kst ? h : 0) * xstep, h % kStages);
