@@ -240,14 +240,15 @@ int fg_chain_cell_norm(const void* state, int64_t ld_state, const void* token, i
 /* One ChainDraftCell step in fp32 (the heads' master weights):
  *   mixed = LayerNorm(state) . Ws^T + LayerNorm(token) . Wt^T      (the two norms as fg_chain_cell_norm)
  *   out[r] = state[r] + gate * (SiLU(mixed[r]) . out_w^T + out_b)
- * state / token [rows, hidden] (row strides ld_state, ld_token), state_proj_w (Ws) and token_proj_w
+ * state / token [rows, hidden] (row strides ld_state, ld_token; the token rows, embeddings, fp32 or bf16
+ * by token_dtype), state_proj_w (Ws) and token_proj_w
  * (Wt) [bottleneck, hidden], out_w [hidden, bottleneck], out_b [hidden], gate one device float (sigmoid applied), out
  * [rows, hidden] contiguous. hidden a multiple of 8 (at most 8192), bottleneck of 4, 16-byte aligned rows.
  * workspace >= fg_chain_cell_step_workspace(rows, hidden, bottleneck) bytes. Replaces
  * models/medusa_heads.py:36-42 (ChainDraftCell.forward). */
 size_t fg_chain_cell_step_workspace(int rows, int hidden, int bottleneck);
-int fg_chain_cell_step(const float* state, int64_t ld_state, const float* token, int64_t ld_token, int rows,
-                       int hidden, int bottleneck, const float* state_w, const float* state_b, const float* token_w,
+int fg_chain_cell_step(const float* state, int64_t ld_state, const void* token, int64_t ld_token, int token_dtype,
+                       int rows, int hidden, int bottleneck, const float* state_w, const float* state_b, const float* token_w,
                        const float* token_b, float eps, const float* state_proj_w, const float* token_proj_w,
                        const float* out_w, const float* out_b, const float* gate, float* out, void* workspace,
                        size_t workspace_bytes, void* stream);

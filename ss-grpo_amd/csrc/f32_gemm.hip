@@ -212,18 +212,14 @@ int f32_gemm_parts(const F32Gemm& g, int splits, float* parts, hipStream_t s) {
 
 extern "C" {
 
-int fg_chain_cell_norm(const void* state, int64_t ld_state, const void* token, int64_t ld_token, int dtype, int rows,
-                       int hidden, const void* state_w, const void* state_b, const void* token_w, const void* token_b,
-                       float eps, void* out, void* stream);  // layers.hip
-
 size_t fg_chain_cell_step_workspace(int rows, int hidden, int bottleneck) {
   if (rows <= 0 || hidden <= 0 || bottleneck <= 0) return 0;
   const ChainPlan p = chain_plan(rows, hidden, bottleneck);
   return (p.x + p.parts + p.mid) * sizeof(float) + 64;
 }
 
-int fg_chain_cell_step(const float* state, int64_t ld_state, const float* token, int64_t ld_token, int rows,
-                       int hidden, int bottleneck, const float* state_w, const float* state_b, const float* token_w,
+int fg_chain_cell_step(const float* state, int64_t ld_state, const void* token, int64_t ld_token, int token_dtype,
+                       int rows, int hidden, int bottleneck, const float* state_w, const float* state_b, const float* token_w,
                        const float* token_b, float eps, const float* state_proj_w, const float* token_proj_w, const float* out_w, 
                        const float* out_b, const float* gate, float* out, void* workspace, size_t workspace_bytes, void* stream) {
   FG_REQUIRE(state && token && state_w && state_b && token_w && token_b && state_proj_w && token_proj_w && out_w && out_b &&
@@ -241,8 +237,8 @@ int fg_chain_cell_step(const float* state, int64_t ld_state, const float* token,
   float* parts = x + p.x;
   float* mid = parts + p.parts;
   hipStream_t s = (hipStream_t)stream;
-  int rc = fg_chain_cell_norm(state, ld_state, token, ld_token, fg::kF32, rows, hidden, state_w, state_b, token_w,
-                              token_b, eps, x, stream);
+  int rc = fg::chain_cell_norm(state, ld_state, fg::kF32, token, ld_token, token_dtype, rows, hidden, state_w, state_b,
+                               token_w, token_b, eps, x, s);
   if (rc) return rc;
   // both projections as one product over the two halves of K
   const fg::F32Gemm first{x,          2 * hidden, 0, state_proj_w, hidden, 0, rows, bottleneck, 2 * hidden, 1,

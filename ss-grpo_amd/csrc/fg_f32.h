@@ -25,4 +25,10 @@ int f32_splits(int M, int N, int K, int batch);
 // parts[p][z][m][n]: the sums of part p, `splits` as f32_splits gives it.
 int f32_gemm_parts(const F32Gemm& g, int splits, float* parts, hipStream_t s);
 
+// fg_chain_cell_norm with token rows of their own dtype (layers.hip): that of the state and the
+// weights, or bf16.
+int chain_cell_norm(const void* state, int64_t ld_state, int dtype, const void* token, int64_t ld_token,
+                    int token_dtype, int rows, int hidden, const void* state_w, const void* state_b,
+                    const void* token_w, const void* token_b, float eps, void* out, hipStream_t s);
+
 }  // namespace fg

@@ -5,6 +5,7 @@
 // (flashgrpo/models/qwen_flashgrpo_wrapper.py:172-180). Also the chain proposals'
 // ChainDraftCell input normalisation (flashgrpo/models/medusa_heads.py:12-42).
 #include "fg_common.h"
+#include "fg_f32.h"
 
 namespace {
 
@@ -235,15 +236,18 @@ __global__ void __launch_bounds__(256) swiglu_kernel(const void* __restrict__ gu
 // The ChainDraftCell's two normalised inputs side by side: workgroup (r, 0) writes
 // out[r, 0:H] = LayerNorm(state[r]) * sw + sb and (r, 1) out[r, H:2H] = LayerNorm(token[r]) * tw + tb
 // (mean, then the mean squared deviation, over the row held in registers; fp32 math, affine
-// weights in the row dtype). H % 8 == 0, H <= 8192.
-template <int DT>
+// weights in the row dtype). H % 8 == 0, H <= 8192. The token rows have a dtype of their own (TT): an
+// fp32 cell reads the bf16 embedding rows as they are, which is exact, instead of a widened copy
+// (6.6 us of its own launch for 768 rows of 4096; this launch reads and writes its rows once, 12.8 us
+// there with fp32 token rows). With the ids gathered as int32, one depth of chain proposals at that size
+// went from 614 to 599 us.
+template <int DT, int TT>
 __global__ void __launch_bounds__(256) chain_cell_norm_kernel(const void* __restrict__ state, int64_t lds_,
                                                               const void* __restrict__ token, int64_t ldt,
                                                               const void* __restrict__ sw, const void* __restrict__ sb,
                                                               const void* __restrict__ tw, const void* __restrict__ tb,
                                                               int H, float eps, void* __restrict__ out) {
   const int r = blockIdx.x, which = blockIdx.y, tid = threadIdx.x;
-  const void* src = which ? token : state;
   const int64_t base = (int64_t)r * (which ? ldt : lds_);
   const void* w = which ? tw : sw;
   const void* bb = which ? tb : sb;
@@ -255,7 +259,8 @@ __global__ void __launch_bounds__(256) chain_cell_norm_kernel(const void* __rest
   for (int c = 0; c < kNormChunks; ++c) {
     const int ch = tid + c * 256;
     if (ch < nch) {
-      fg::load8<DT>(src, base + ch * 8, v[c]);
+      if (which) fg::load8<TT>(token, base + ch * 8, v[c]);  // one side per workgroup
+      else fg::load8<DT>(state, base + ch * 8, v[c]);
 #pragma unroll
       for (int j = 0; j < 8; ++j) s += v[c][j];
     }
@@ -312,6 +317,32 @@ __global__ void __launch_bounds__(256) copy_arrays_kernel(CopyArgs a) {
 }
 
 }  // namespace
+
+namespace fg {
+
+int chain_cell_norm(const void* state, int64_t ld_state, int dtype, const void* token, int64_t ld_token,
+                    int token_dtype, int rows, int hidden, const void* state_w, const void* state_b,
+                    const void* token_w, const void* token_b, float eps, void* out, hipStream_t s) {
+  FG_REQUIRE(state && token && state_w && state_b && token_w && token_b && out, "fg_chain_cell_norm: null pointer");
+  FG_REQUIRE((dtype == kBF16 || dtype == kF32) && (token_dtype == dtype || token_dtype == kBF16),
+             "fg_chain_cell_norm: dtype");
+  FG_REQUIRE(rows > 0 && rows <= 65535 && hidden > 0, "fg_chain_cell_norm: bad shape");
+  FG_REQUIRE(hidden % 8 == 0 && hidden <= 8 * 256 * kNormChunks, "fg_chain_cell_norm: hidden must be a multiple of 8, at most 8192");
+  FG_REQUIRE(ld_state >= hidden && ld_token >= hidden && ld_state % 8 == 0 && ld_token % 8 == 0,
+             "fg_chain_cell_norm: row strides must be multiples of 8, at least hidden");
+  const uintptr_t al = (uintptr_t)state | (uintptr_t)token | (uintptr_t)state_w | (uintptr_t)state_b |
+                       (uintptr_t)token_w | (uintptr_t)token_b | (uintptr_t)out;
+  FG_REQUIRE((al & 15) == 0, "fg_chain_cell_norm: 16-byte alignment");
+  const dim3 grid((unsigned)rows, 2);
+  const auto kernel = dtype == kBF16         ? chain_cell_norm_kernel<kBF16, kBF16>
+                      : token_dtype == kBF16 ? chain_cell_norm_kernel<kF32, kBF16>
+                                             : chain_cell_norm_kernel<kF32, kF32>;
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, state, ld_state, token, ld_token, state_w, state_b, token_w,
+                     token_b, hidden, eps, out);
+  return check_launch("fg_chain_cell_norm");
+}
+
+}  // namespace fg
 
 extern "C" {
 
@@ -400,24 +431,8 @@ int fg_rmsnorm(void* x, const void* delta, const void* weight, void* y, int dtyp
 int fg_chain_cell_norm(const void* state, int64_t ld_state, const void* token, int64_t ld_token, int dtype,
                        int rows, int hidden, const void* state_w, const void* state_b, const void* token_w,
                        const void* token_b, float eps, void* out, void* stream) {
-  FG_REQUIRE(state && token && state_w && state_b && token_w && token_b && out, "fg_chain_cell_norm: null pointer");
-  FG_REQUIRE(dtype == fg::kBF16 || dtype == fg::kF32, "fg_chain_cell_norm: dtype");
-  FG_REQUIRE(rows > 0 && rows <= 65535 && hidden > 0, "fg_chain_cell_norm: bad shape");
-  FG_REQUIRE(hidden % 8 == 0 && hidden <= 8 * 256 * kNormChunks, "fg_chain_cell_norm: hidden must be a multiple of 8, at most 8192");
-  FG_REQUIRE(ld_state >= hidden && ld_token >= hidden && ld_state % 8 == 0 && ld_token % 8 == 0,
-             "fg_chain_cell_norm: row strides must be multiples of 8, at least hidden");
-  const uintptr_t al = (uintptr_t)state | (uintptr_t)token | (uintptr_t)state_w | (uintptr_t)state_b |
-                       (uintptr_t)token_w | (uintptr_t)token_b | (uintptr_t)out;
-  FG_REQUIRE((al & 15) == 0, "fg_chain_cell_norm: 16-byte alignment");
-  const dim3 grid((unsigned)rows, 2);
-  hipStream_t s = (hipStream_t)stream;
-  if (dtype == fg::kBF16)
-    hipLaunchKernelGGL(chain_cell_norm_kernel<fg::kBF16>, grid, dim3(256), 0, s, state, ld_state, token, ld_token,
-                       state_w, state_b, token_w, token_b, hidden, eps, out);
-  else
-    hipLaunchKernelGGL(chain_cell_norm_kernel<fg::kF32>, grid, dim3(256), 0, s, state, ld_state, token, ld_token,
-                       state_w, state_b, token_w, token_b, hidden, eps, out);
-  return fg::check_launch("fg_chain_cell_norm");
+  return fg::chain_cell_norm(state, ld_state, dtype, token, ld_token, dtype, rows, hidden, state_w, state_b, token_w,
+                             token_b, eps, out, (hipStream_t)stream);
 }
 
 int fg_swiglu(const void* gate_up, void* out, int dtype, int rows, int inter, void* stream) {

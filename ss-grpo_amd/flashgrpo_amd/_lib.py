@@ -46,7 +46,7 @@ SIGNATURES = {
     "fg_copy_arrays": (_I, [_P, _P, _P, _I, _P]),
     "fg_chain_cell_norm": (_I, [_P, _I64, _P, _I64, _I, _I, _I, _P, _P, _P, _P, _F, _P, _P]),
     "fg_chain_cell_step_workspace": (_SZ, [_I, _I, _I]),
-    "fg_chain_cell_step": (_I, [_P, _I64, _P, _I64, _I, _I, _I, _P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
+    "fg_chain_cell_step": (_I, [_P, _I64, _P, _I64, _I, _I, _I, _I, _P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "fg_gate_up_swiglu": (_I, [_P, _I64, _P, _I64, _P, _I64, _I, _I, _I, _I, _P]),
     "fg_linear_parts": (_I, [_P, _I64, _P, _I64, _P, _I, _I, _I, _I, _I, _I, _I, _P]),
     "fg_residual_rmsnorm_parts": (_I, [_P, _I, _I, _I, _P, _I64, _P, _F, _P, _I64, _P]),

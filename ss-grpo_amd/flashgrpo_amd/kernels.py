@@ -438,8 +438,8 @@ def chain_cell_norm(state, token, state_w, state_b, token_w, token_b, eps, *, ou
 
 
 def chain_cell_step_ok(state, token, weights) -> bool:
-    """Whether fg_chain_cell_step takes this cell: everything fp32 on the GPU, hidden a multiple of 8
-    up to 8192, the bottleneck a multiple of 4, whole rows, 16-byte aligned. ``weights`` are the eight
+    """Whether fg_chain_cell_step takes this cell: everything fp32 on the GPU (the token rows bf16 too),
+    hidden a multiple of 8 up to 8192, the bottleneck a multiple of 4, whole rows, 16-byte aligned. ``weights`` are the eight
     tensors after (state, token) of :func:`chain_cell_step`, the gate aside."""
     out_w = weights[6]
     H, bott = out_w.shape
@@ -447,26 +447,27 @@ def chain_cell_step_ok(state, token, weights) -> bool:
     rows = lambda t: t.shape[-1] == H and t.numel() > 0 and t.is_contiguous()
     return (H % 8 == 0 and 0 < H <= 8192 and bott % 4 == 0 and bott > 0 and state.shape == token.shape
             and rows(state) and rows(token) and all(tuple(w.shape) == s for w, s in zip(weights, shapes))
+            and token.dtype in (torch.float32, torch.bfloat16) and token.is_cuda and token.data_ptr() % 16 == 0
             and all(t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
-                    for t in (state, token, *weights)))
+                    for t in (state, *weights)))
 
 
 def chain_cell_step(state, token, state_w, state_b, token_w, token_b, state_proj_w, token_proj_w, out_w, out_b, gate,
                     eps):
-    """One fp32 ChainDraftCell step (``fg_chain_cell_step``): state and token [rows, H] contiguous,
-    the projections [bottleneck, H], gate the sigmoid of the cell's gate (one element). Returns the
+    """One fp32 ChainDraftCell step (``fg_chain_cell_step``): state and token [rows, H] contiguous
+    (token fp32 or bf16), the projections [bottleneck, H], gate the sigmoid of the cell's gate (one element). Returns the
     new states [rows, H]."""
     weights = (state_w, state_b, token_w, token_b, state_proj_w, token_proj_w, out_w, out_b)
     _dev(state, token, *weights, gate)
     if state.ndim != 2 or not chain_cell_step_ok(state, token, weights) or gate.dtype != torch.float32 \
             or gate.numel() != 1:
-        raise ValueError("chain_cell_step: needs contiguous fp32 state and token [rows, H], projections [bottleneck, H], "
+        raise ValueError("chain_cell_step: needs contiguous fp32 state and fp32 or bf16 token [rows, H], projections [bottleneck, H], "
                          "out_w [H, bottleneck] with H % 8 == 0, bottleneck % 4 == 0, 16-byte aligned, and an fp32 gate")
     rows, H = state.shape
     bott = out_w.shape[1]
     out = torch.empty(rows, H, dtype=torch.float32, device=state.device)
     ws = torch.empty(_lib.load().fg_chain_cell_step_workspace(rows, H, bott), dtype=torch.uint8, device=state.device)
-    _call("fg_chain_cell_step", _ptr(state), H, _ptr(token), H, rows, H, bott, *[_ptr(t) for t in weights[:4]],
+    _call("fg_chain_cell_step", _ptr(state), H, _ptr(token), H, dtype_code(token), rows, H, bott, *[_ptr(t) for t in weights[:4]],
           float(eps), *[_ptr(t) for t in weights[4:]], _ptr(gate), _ptr(out), _ptr(ws), ws.numel(), _stream())
     return out
 

@@ -72,23 +72,25 @@ class ChainDraftCell(nn.Module):
         w = self._weights(dt, state.device)
         H = state.shape[-1]
         s = state.to(dt)
-        tok = token_embedding.to(dt)
         if s.is_cuda:
             # both LayerNorms in one launch, written side by side (fg_chain_cell_norm)
             from .. import kernels as K
 
             rows = lambda t: t.reshape(-1, H) if t.is_contiguous() else t.reshape(-1, H).contiguous()
-            r, t = rows(s), rows(tok)
+            # an fp32 cell reads bf16 embedding rows as they are
+            t = rows(token_embedding if (dt, token_embedding.dtype) == (torch.float32, torch.bfloat16)
+                     else token_embedding.to(dt))
+            r = rows(s)
             native = [w[k] for k in ("sn_w", "sn_b", "tn_w", "tn_b", "sp_w", "tp_w", "out_w", "out_b")]
             # the torch form stays where autograd follows the state and where autocast rounds the products
             if (w["gate"].dtype == torch.float32 and not (torch.is_grad_enabled() and s.requires_grad)
                     and not torch.is_autocast_enabled("cuda") and K.chain_cell_step_ok(r, t, native)):
                 return K.chain_cell_step(r, t, *native, w["gate"], w["eps"]).view(*s.shape)
-            x = K.chain_cell_norm(r, t, w["sn_w"], w["sn_b"], w["tn_w"], w["tn_b"], w["eps"])
+            x = K.chain_cell_norm(r, t.to(dt), w["sn_w"], w["sn_b"], w["tn_w"], w["tn_b"], w["eps"])
             xs, xt = x[:, :H].view(*s.shape), x[:, H:].view(*s.shape)
         else:
             xs = F.layer_norm(s, (H,), w["sn_w"], w["sn_b"], w["eps"])
-            xt = F.layer_norm(tok, (H,), w["tn_w"], w["tn_b"], w["eps"])
+            xt = F.layer_norm(token_embedding.to(dt), (H,), w["tn_w"], w["tn_b"], w["eps"])
         mixed = F.linear(xs, w["sp_w"]) + F.linear(xt, w["tp_w"])
         delta = F.linear(F.silu(mixed), w["out_w"], w["out_b"])
         return s + w["gate"] * delta
@@ -208,7 +210,8 @@ class MedusaHeads(nn.Module):
     def chain_next_state(self, state, token_ids, embedding_weight):
         """Next chain state from the parent state and the path token's embedding
         (``medusa_heads.py:279-286``), computed in the cell's parameter dtype."""
-        emb = embedding_weight.index_select(0, token_ids.to(embedding_weight.device).long())
+        ids = token_ids.to(embedding_weight.device)
+        emb = embedding_weight.index_select(0, ids if ids.dtype == torch.int32 else ids.long())
         return self.chain_cell.step(state, emb)
 
     # -------------------------------------------------------------- checkpoint I/O

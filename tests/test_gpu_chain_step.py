@@ -31,6 +31,9 @@ def test_chain_cell_step_matches_float64(rows, H, bott):
     bound = gate.double() * e_out + 2.0 ** -22 * (want.abs() + st.double().abs()) + 1e-6
     assert bool(((got.double() - want).abs() <= bound).all())
     assert torch.equal(got, K.chain_cell_step(*args))
+    # bf16 token rows (embeddings): the same as their widened copy
+    assert torch.equal(K.chain_cell_step(st, tk.bfloat16(), *args[2:]),
+                       K.chain_cell_step(st, tk.bfloat16().float(), *args[2:]))
 
 
 @pytest.mark.parametrize("B,H,heads", [(1, 64, 1), (65, 132, 2), (96, 1000, 3), (7, 4096, 1)])
