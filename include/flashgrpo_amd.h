@@ -253,8 +253,8 @@ int fg_chain_cell_step(const float* state, int64_t ld_state, const void* token, 
                        const float* out_w, const float* out_b, const float* gate, float* out, void* workspace,
                        size_t workspace_bytes, void* stream);
 
-/* Workspace (bytes) that lets fg_sample_tokens / fg_walk_step split each row of an
- * unrestricted (no top-k, no top-p) or greedy draw over several workgroups. */
+/* Workspace (bytes) that lets fg_sample_tokens / fg_walk_step split each row of a draw
+ * over several workgroups (rows that one workgroup holds in registers are not split). */
 size_t fg_sample_workspace(int rows);
 
 /* One supplied-noise draw per row (rule documented in csrc/sample.hip).
@@ -263,7 +263,7 @@ size_t fg_sample_workspace(int rows);
  * when noise != NULL, else counter noise (seed, step, seq_ids ? seq_ids[r] : r, draw).
  * greedy or temperature == 0: argmax (first maximum). top_k <= 0: off.
  * top_p_fixed = floor(top_p * 2^32), 0 = off. workspace (optional, >= fg_sample_workspace(rows)
- * bytes): unrestricted and greedy draws then run split over several workgroups per row;
+ * bytes): draws of long rows then run split over several workgroups per row;
  * results are identical either way (greedy, unrestricted, top-p and top-k up to 4096). */
 int fg_sample_tokens(const void* logits, int dtype, int64_t row_stride, int rows, int vocab,
                      const int32_t* row_index, const int32_t* forced, const uint32_t* noise, int noise_stride,

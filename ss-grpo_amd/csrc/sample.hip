@@ -17,8 +17,8 @@
 // row in registers (resident_sample). Longer rows with a workspace run over several workgroups:
 // unrestricted and greedy draws split over 16 chunks per
 // row (chunk maxima, then one draw launch; a walk step whose row maxima come from
-// the LM head's epilogue is the draw launch alone, see "split sampling"), top-p
-// draws without top-k over seven launches (see "split top-p"). Otherwise: one
+// the LM head's epilogue is the draw launch alone, see "split sampling"), top-k and top-p
+// draws over four launches or two (see "split top-k / top-p"). Otherwise: one
 // 1024-thread workgroup per sampled row. The row is split into 16
 // contiguous wave segments; a wave walks its segment 512 elements (8 per lane,
 // 16-byte loads) per step. Top-k / top-p use an MSB-first 4 x 8-bit radix
