@@ -87,14 +87,15 @@ FG_DEVICE float sanitize(float v) {
   return v;
 }
 
-// Running (max, sum of exp(x - max)) of a set of values.
+// Running (max, sum of exp(x - max)) of a set of values. The maximum ignores NaN, the sum does not:
+// a set without a finite value has the maximum -inf and the sum 0, or NaN where it holds a NaN.
 struct LseAcc {
   float m, s;
 };
 
 FG_DEVICE LseAcc lse_combine(LseAcc a, LseAcc b) {
   float m = fmaxf(a.m, b.m);
-  if (m == -INFINITY) return {m, 0.0f};
+  if (m == -INFINITY) return {m, a.s + b.s};
   return {m, a.s * __expf(a.m - m) + b.s * __expf(b.m - m)};
 }
 

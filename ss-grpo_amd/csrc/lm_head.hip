@@ -415,10 +415,11 @@ __global__ void __launch_bounds__(W * 64, 1) lm_stream_kernel(LmArgs a) {
               m8 = fmaxf(m8, v[j]);
             }
           const float mx = fmaxf(acc_l.m, m8);
-          float sm = (acc_l.m == -INFINITY) ? 0.0f : acc_l.s * __expf(acc_l.m - mx);
+          const float ref = mx == -INFINITY ? 0.0f : mx;  // -inf adds 0, NaN stays NaN
+          float sm = (acc_l.m == -INFINITY) ? acc_l.s : acc_l.s * __expf(acc_l.m - mx);
 #pragma unroll
           for (int j = 0; j < 8; ++j)
-            if (j < valid) sm += __expf(v[j] - mx);
+            if (j < valid) sm += __expf(v[j] - ref);
           acc_l = {mx, sm};
         }
       }
