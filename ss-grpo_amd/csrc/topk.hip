@@ -10,10 +10,12 @@
 // at least K disjoint groups of threads bound the pass's K-th element from below, so only the few
 // elements from the least of them on are listed in LDS as 64-bit rank keys and ranked by
 // comparing each with every other; the other elements cost a comparison each, and (optionally)
-// their part of the maximum and sum of exp. A chunk whose list overflows (long ties) keeps a
-// sorted top-K per thread instead, merged with the bitonic "max(A[i], B[K-1-i]) then sort" step.
+// their part of the maximum and sum of exp. A chunk whose list overflows (long ties)
+// and short chunks (sorted_chunks) keep a sorted top-K per thread, merged with the bitonic
+// "max(A[i], B[K-1-i]) then sort" step.
 // Bound by VALU and HBM about equally: the top-2 with sums of exp of 384 x 128,256 bf16 logits
-// (98 MB) 43.7 us inserting every element into such lists, 31.9 this way; the top-16 275 and 35.
+// (98 MB) 43.6 us inserting every element into such lists, 32.2 this way; the top-16 250 and 37.8. Equal
+// logits throughout overflow every list: the top-2 there 43 us that way, 106 this way.
 // Phase 2: one wave per row merges the chunk lists.
 //
 // With `sanitize` the values are first mapped as torch.nan_to_num(x.float(),
@@ -41,6 +43,85 @@ constexpr int kLoads = 5;                // groups of 8 elements per thread and 
 constexpr int kGroup = kThreads * 8;
 constexpr int kPass = kGroup * kLoads;   // elements per workgroup pass
 constexpr int kList = 256;               // listed candidates per chunk
+
+// The list's bound takes the maxima of bound_groups(K) groups of threads, so a chunk has to give each of
+// them an element; and in one load group a list of the top 1 or 2 costs more (its barriers) than the
+// sorted lists: 1 x 512 bf16 top-4 6.9 us sorted and 9.7 listed, 8 x 32,000 (chunks of 2,000) top-1 5.3
+// and 5.7, top-4 8.2 and 7.1.
+constexpr int bound_groups(int K) { return K > 4 ? K : 4; }
+constexpr bool sorted_chunks(int K, int chunk) {
+  return chunk <= kGroup && (K <= 2 || chunk <= kGroup - kGroup / bound_groups(K));
+}
+
+// Phase 1 of sorted_chunks: a sorted top-K per thread over its elements, then of the workgroup. Bound by
+// latency (a load, then the merges over lanes and waves).
+template <int DT, int K, bool STATS, bool SAN>
+__global__ void __launch_bounds__(kThreads) topk_phase1_sorted(const void* __restrict__ logits, int64_t row_stride,
+                                                               int vocab, int chunk, uint64_t* __restrict__ part_keys,
+                                                               float2* __restrict__ part_lse) {
+  const int row = blockIdx.x, c = blockIdx.y;
+  const char* rowp = (const char*)logits + (int64_t)row * row_stride * (DT == fg::kBF16 ? 2 : 4);
+  const int lo = c * chunk, hi = min(vocab, lo + chunk);
+  __shared__ uint64_t s_top[kThreads / 64][K];
+  __shared__ float2 s_lse[kThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint64_t top[K];
+#pragma unroll
+  for (int i = 0; i < K; ++i) top[i] = 0;
+  LseAcc acc{-INFINITY, 0.0f};
+  const int vec_hi = lo + ((hi - lo) & ~7);
+  for (int i = lo + tid * 8; i < vec_hi; i += kGroup) {
+    float v[8];
+    fg::load8<DT>(rowp, i, v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = sanitize<SAN>(v[j]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) insert_key<K>(top, fg::rank_key(v[j], (uint32_t)(i + j)));
+    if constexpr (STATS) {
+      float m8 = v[0];
+#pragma unroll
+      for (int j = 1; j < 8; ++j) m8 = fmaxf(m8, v[j]);
+      const float m = fmaxf(acc.m, m8), ref = m == -INFINITY ? 0.0f : m;  // -inf adds 0, NaN stays NaN
+      float s = acc.m == -INFINITY ? acc.s : acc.s * __expf(acc.m - m);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += __expf(v[j] - ref);
+      acc = {m, s};
+    }
+  }
+  for (int i = vec_hi + tid; i < hi; i += kThreads) {
+    const float v = sanitize<SAN>(fg::load_elem<DT>(rowp, i));
+    insert_key<K>(top, fg::rank_key(v, (uint32_t)i));
+    if constexpr (STATS) acc = lse_combine(acc, v != v ? LseAcc{-INFINITY, v} : LseAcc{v, v == -INFINITY ? 0.0f : 1.0f});
+  }
+  wave_merge<K>(top);
+  if constexpr (STATS) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      LseAcc other{__shfl_xor(acc.m, o, 64), __shfl_xor(acc.s, o, 64)};
+      acc = lse_combine(acc, other);
+    }
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) s_top[wave][i] = top[i];
+    if constexpr (STATS) s_lse[wave] = make_float2(acc.m, acc.s);
+  }
+  __syncthreads();
+  if (tid == 0) {
+#pragma unroll
+    for (int w = 1; w < kThreads / 64; ++w) {
+      uint64_t other[K];
+#pragma unroll
+      for (int i = 0; i < K; ++i) other[i] = s_top[w][i];
+      merge_desc<K>(top, other);
+      if constexpr (STATS) acc = lse_combine(acc, LseAcc{s_lse[w].x, s_lse[w].y});
+    }
+    const int64_t part = (int64_t)row * gridDim.y + c;
+#pragma unroll
+    for (int i = 0; i < K; ++i) part_keys[part * K + i] = top[i];
+    if constexpr (STATS) part_lse[part] = make_float2(acc.m, acc.s);
+  }
+}
 
 template <int DT, int K, bool STATS, bool SAN>
 __global__ void __launch_bounds__(kThreads) topk_phase1(const void* __restrict__ logits, int64_t row_stride,
@@ -94,7 +175,7 @@ __global__ void __launch_bounds__(kThreads) topk_phase1(const void* __restrict__
     }
     // bound: at least K of the 4 S groups of 64 / S threads have a maximum from it on, so the pass
     // has K elements there
-    constexpr int S = K > 4 ? K / 4 : 1;
+    constexpr int S = bound_groups(K) / 4;
     float gm = mx;
 #pragma unroll
     for (int o = 32 / S; o > 0; o >>= 1) gm = fmaxf(gm, __shfl_xor(gm, o, 64));
@@ -159,6 +240,8 @@ __global__ void __launch_bounds__(kThreads) topk_phase1(const void* __restrict__
     }
     if (tid >= n && tid < K) out[tid] = 0;
   } else {
+    // one element a step: the vector form of topk_phase1_sorted takes registers that cost every chunk
+    // its occupancy (the top-16 below 37.8 -> 51 us)
     __shared__ uint64_t s_top[kThreads / 64][K];
     uint64_t top[K];
 #pragma unroll
@@ -237,12 +320,11 @@ template <int DT, int K, bool STATS>
 void launch_topk(const void* logits, int64_t row_stride, int rows, int vocab, int chunks, int chunk, int kout,
                  uint64_t* part_keys, float2* part_lse, int32_t* tok, float* score, float* stats, bool san,
                  hipStream_t stream) {
-  if (san)
-    hipLaunchKernelGGL((topk_phase1<DT, K, STATS, true>), dim3(rows, chunks), dim3(kThreads), 0, stream, logits,
-                       row_stride, vocab, chunk, part_keys, part_lse);
-  else
-    hipLaunchKernelGGL((topk_phase1<DT, K, STATS, false>), dim3(rows, chunks), dim3(kThreads), 0, stream, logits, row_stride,
-                     vocab, chunk, part_keys, part_lse);
+  const bool sorted = sorted_chunks(K, chunk);
+  const auto phase1 = sorted ? (san ? topk_phase1_sorted<DT, K, STATS, true> : topk_phase1_sorted<DT, K, STATS, false>)
+                             : (san ? topk_phase1<DT, K, STATS, true> : topk_phase1<DT, K, STATS, false>);
+  hipLaunchKernelGGL(phase1, dim3(rows, chunks), dim3(kThreads), 0, stream, logits, row_stride, vocab, chunk, part_keys,
+                     part_lse);
   hipLaunchKernelGGL((topk_phase2<K, STATS>), dim3(rows), dim3(64), 0, stream, part_keys, part_lse, chunks, kout, tok,
                      score, stats);
 }
