@@ -34,10 +34,15 @@ constexpr int kThreads = 1024;
 constexpr int kWaves = kThreads / 64;
 constexpr int kStep = 512;  // elements per wave step
 
+// Histogram copies: lane l adds to copy l % kCopies of a bin, the copies of a bin side by side on
+// banks of their own, so that logits close to each other wait less for one word (the q-mass
+// pass of 64 x 152,064: 13.4 -> 12.2 us with 8 copies instead of one per wave).
+constexpr int kCopies = 8;
+
 struct Shared {
   uint64_t exp2[1024];  // kExp2Table
   uint64_t wsum[kWaves];
-  uint64_t hist[256];
+  uint64_t hist[256][kCopies];
   uint64_t wkey[kWaves];
   float wmax[kWaves];
   uint64_t u64b[2];
@@ -191,11 +196,11 @@ FG_DEVICE KeyCut radix_select(const Row<DT>& r, KeyCut within, uint64_t target, 
   for (int level = 0; level < 4; ++level) {
     const int shift = 24 - 8 * level;
     __syncthreads();
-    for (int d = threadIdx.x; d < 256; d += kThreads) sh.hist[d] = 0;
+    for (int d = threadIdx.x; d < 256 * kCopies; d += kThreads) (&sh.hist[0][0])[d] = 0;
     __syncthreads();
     for_wave_segment(r, [&](int i, float s, uint32_t key) {
       if (within(key, (uint32_t)i) && (key & pmask) == prefix)
-        atomicAdd((unsigned long long*)&sh.hist[(key >> shift) & 255u],
+        atomicAdd((unsigned long long*)&sh.hist[(key >> shift) & 255u][lane % kCopies],
                   (unsigned long long)(WEIGHTED ? r.weight(s) : 1ull));
     });
     __syncthreads();
@@ -204,7 +209,9 @@ FG_DEVICE KeyCut radix_select(const Row<DT>& r, KeyCut within, uint64_t target, 
       uint64_t h[4], mine = 0;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        h[j] = sh.hist[255 - 4 * lane - j];
+        h[j] = 0;
+#pragma unroll 1
+        for (int q = 0; q < kCopies; ++q) h[j] += sh.hist[255 - 4 * lane - j][q];
         mine += h[j];
       }
       uint64_t incl = fg::wave_incl_scan_u64(mine);
@@ -304,9 +311,10 @@ FG_DEVICE int block_sample(const void* rowp, int V, const SampleParams& sp, uint
 }
 
 // ------------------------------------------------------------------ selection by the fixed-point exponent
-// Bins of the exponent a (fg_common.h), 8 per octave below the row maximum: a never grows with
-// x, so the bins are runs of the candidate order. Elements of weight 0 are in no bin: they
-// cannot be drawn, and in the candidate order only NaN comes before one with weight.
+// Bins of the exponent a (fg_common.h), 8 per octave below the row maximum, or 256 (128 at least) over
+// the row's own range where that is narrower, so that a flat row's bins hold no more elements than
+// another's: a never grows with x, so the bins are runs of the candidate order. Elements of weight 0
+// are in no bin: they cannot be drawn, and in the candidate order only NaN comes before one with weight.
 constexpr int kSelBins = 256;
 constexpr int kSelBinShift = 17;             // 2^17 steps of a: 8 bins per octave
 constexpr uint32_t kSelAMax = 40u << 20;     // larger a weigh 0
@@ -317,18 +325,20 @@ FG_DEVICE uint32_t fixed_exponent(float m, float x, float kt) {
 #pragma clang fp contract(off)
   return (uint32_t)fminf((m - x) * kt, fg::kWeightZmax);
 }
-// Histogram copies: lane l adds to copy l % kCopies of a bin, the copies of a bin side by side on
-// banks of their own, so that logits close to each other wait less for one word (the q-mass
-// pass of 64 x 152,064: 13.4 -> 12.2 us with 8 copies instead of one per wave).
-constexpr int kCopies = 8;
-
 // The weight of weight_q40 from its exponent.
 FG_DEVICE uint64_t exponent_weight(uint32_t a, const uint64_t* tbl) {
   const uint64_t e = tbl[(a >> 10) & 1023u];
   const uint32_t w = (uint32_t)e - (__umul24((uint32_t)(e >> 32), a & 1023u) >> 10);
   return ((uint64_t)w << 32) >> ((a >> 20) + 23u);
 }
-FG_DEVICE int sel_bin(uint32_t a) { return min((int)(a >> kSelBinShift), kSelBins - 1); }
+// Steps of a (log2) of a bin in a row from `low` to m.
+FG_DEVICE int bin_shift(float m, float low, float kt) {
+  const uint32_t range = low <= m ? fixed_exponent(m, low, kt) : 0u;
+  return min(kSelBinShift, max(0, 24 - (int)__clz((int)(range | 1u))));
+}
+FG_DEVICE int sel_bin(uint32_t a, int shift) { return min((int)(a >> shift), kSelBins - 1); }
+FG_DEVICE float above_inf(float x) { return x > -INFINITY ? x : INFINITY; }  // for the least logit
+FG_DEVICE float wave_min(float v) { return -fg::wave_max(-v); }
 
 // Largest-first selection over the keys ck[0, n) >= cut (whole block of kThreads; the keys are
 // distinct): the key at which the running count, or the running q-mass of the logit that a key
@@ -569,6 +579,252 @@ FG_DEVICE int list_draw(const uint64_t* ck, int n, int64_t slots, uint32_t tp32,
   return (int)fg::rank_key_index(list_select<true, true>(ck, n, cut, fg::mulhi_u64_u32(total, u), m, kt, tbl, sel));
 }
 
+// Loads elements i0 .. i0 + 7 of a chunk ending at hi; past hi come -inf, whose weight is
+// 0 against any row maximum, so the weights need no per-element test.
+template <int DT>
+FG_DEVICE void split_load8(const char* p, int i0, int hi, float (&x)[8]) {
+  if (i0 + 8 <= hi) {
+    fg::load8<DT>(p, i0, x);
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x[j] = i0 + j < hi ? fg::load_elem<DT>(p, i0 + j) : -INFINITY;
+}
+
+// First index in [lo, hi) whose inclusive running mass w(x, index) exceeds target (the whole
+// block of THREADS; -1 if none), scanned in index order one group of THREADS x 8 elements at a
+// time (thread t holds 8 consecutive elements of a group), stopping at the group that holds
+// the target. The LOADS groups of a pass are loaded together. wsum: THREADS / 64 words.
+template <int DT, int THREADS, int LOADS, class W>
+FG_DEVICE int split_locate(const char* p, int lo, int hi, W&& weight, uint64_t target, uint64_t* wsum, int* found) {
+  constexpr int WAVES = THREADS / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (tid == 0) *found = -1;
+  uint64_t run = 0;  // block-uniform
+  bool done = false;
+  for (int base = lo; base < hi && !done; base += THREADS * 8 * LOADS) {
+    float x[LOADS][8];
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u)
+      if (base + u * THREADS * 8 < hi) split_load8<DT>(p, base + (u * THREADS + tid) * 8, hi, x[u]);
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u) {
+      if (base + u * THREADS * 8 >= hi) break;  // uniform
+      const int i0 = base + (u * THREADS + tid) * 8;
+      uint64_t mine = 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) mine += weight(x[u][j], i0 + j);
+      const uint64_t incl = fg::wave_incl_scan_u64(mine);
+      __syncthreads();  // wsum of the previous group has been read
+      if (lane == 63) wsum[wave] = incl;
+      __syncthreads();
+      uint64_t woff = 0, stot = 0;
+#pragma unroll 4
+      for (int w = 0; w < WAVES; ++w) {
+        if (w < wave) woff += wsum[w];
+        stot += wsum[w];
+      }
+      if (run + stot > target) {  // uniform: this group holds the target
+        uint64_t cum = run + woff + incl - mine;
+        if (cum <= target && target < cum + mine) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            cum += weight(x[u][j], i0 + j);
+            if (cum > target) {
+              *found = i0 + j;
+              break;
+            }
+          }
+        }
+        done = true;
+        break;
+      }
+      run += stot;
+    }
+  }
+  __syncthreads();
+  return *found;
+}
+
+// Where a cut lies: kept are the exponents below lo, and those in [lo, hi) whose rank key is at least cut.
+struct RowCut {
+  uint32_t lo, hi;
+  uint64_t cut;
+  uint64_t rest;  // q-mass (top-p) or count (top-k) before the cut within [lo, hi)
+  int n, nan;     // top-k: listed elements (all kept ones among them), NaN logits (they take slots)
+};
+FG_DEVICE RowCut bin_cut(int bin, int shift, uint64_t rest) {
+  return RowCut{(uint32_t)bin << shift, bin < kSelBins - 1 ? (uint32_t)(bin + 1) << shift : kSelAMax + 1, 0, rest, 0, 0};
+}
+
+struct NarrowShared {
+  uint64_t wred[kWaves];
+  uint32_t ones[kWaves], zeros[kWaves];
+  uint64_t before;
+  int digit, n, nan, found;
+};
+
+// f(x, i0) for every 8 elements from i0 on of a row, over the whole block; past V the logits are -inf.
+template <int DT, class F>
+FG_DEVICE void for_row8(const char* p, int V, F&& f) {
+  for (int base = 0; base < V; base += kThreads * 16) {
+    float x[2][8];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (base + u * kThreads * 8 < V) split_load8<DT>(p, base + (u * kThreads + threadIdx.x) * 8, V, x[u]);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (base + u * kThreads * 8 < V) f(x[u], base + (u * kThreads + (int)threadIdx.x) * 8);
+  }
+}
+
+// The cut of a row whose class [c.lo, c.hi) holds more elements than a list (flat rows, long ties), by one
+// workgroup: the class is cut into at most 256 parts by exponent and replaced by the one that holds the
+// cut, until its elements fit the list; a class of one value is cut by index. Top-k starts from all
+// exponents with c.rest = top_k. False where the row has no weight, NaN takes every slot, or more
+// distinct logits than a list share one exponent (2^-20 octaves).
+// Two passes over the row a step, as a rule one step. In place of block_sample, whose radix over the key
+// bits makes four passes a cut: top-k 50 of 64 equal rows of 152,064 bf16 logits 590 -> 170 us, top-k 1,000 of
+// rows with a standard deviation of 0.05 in units of the temperature 236 -> 48 (bins of the row's range too).
+template <int DT, bool COUNT>
+FG_DEVICE bool narrow_cut(const char* p, int V, float m, float kt, const uint64_t* tbl, uint64_t* ck, RowCut& c,
+                          NarrowShared& sh, SelectShared& sel, SmallShared& small) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  uint64_t* hist = ck;  // [kSelBins][kCopies], until the list takes its place
+  static_assert(kSelBins * kCopies <= kSelList, "the histogram fits the list");
+  const auto list = [&](auto&& take) {  // elements x at i with take(a, x, i) into ck; sh.n is 0
+    for_row8<DT>(p, V, [&](const float(&x)[8], int i0) {
+      uint32_t hit = 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (take(fixed_exponent(m, x[j], kt), x[j], i0 + j)) hit |= 1u << j;
+      if (!hit) return;
+      int at = atomicAdd(&sh.n, (int)__popc(hit));
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (hit >> j & 1u) {
+          if (at < kSelList) ck[at] = fg::rank_key(x[j], (uint32_t)(i0 + j));
+          ++at;
+        }
+    });
+    __syncthreads();
+  };
+  for (bool first = COUNT;; first = false) {
+    const uint32_t width = c.hi - c.lo;
+    const int shift = max(0, 24 - (int)__clz((int)(width - 1)));
+    __syncthreads();  // ck and sh are free
+    if (width == 1) {  // one exponent already
+      if (tid == 0) sh.n = 0;
+      __syncthreads();
+    } else {
+    for (int i = tid; i < kSelBins * kCopies; i += kThreads) hist[i] = 0;
+    if (tid == 0) {
+      sh.digit = -1;
+      sh.n = 0;
+      sh.nan = 0;
+    }
+    __syncthreads();
+    int nan = 0;
+    for_row8<DT>(p, V, [&](const float(&x)[8], int) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t a = fixed_exponent(m, x[j], kt);
+        if constexpr (COUNT) nan += x[j] != x[j];
+        if (a - c.lo < width)
+          atomicAdd((unsigned long long*)&hist[((a - c.lo) >> shift) * kCopies + lane % kCopies],
+                    (unsigned long long)(COUNT ? 1ull : exponent_weight(a, tbl)));
+      }
+    });
+    if (COUNT && first && nan) atomicAdd(&sh.nan, nan);
+    __syncthreads();
+    if (tid < 64) {  // the part of the cut: lane l owns parts 4 l .. 4 l + 3
+      uint64_t b[4], mine = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        b[j] = 0;
+#pragma unroll
+        for (int q = 0; q < kCopies; ++q) b[j] += hist[(4 * lane + j) * kCopies + q];
+        mine += b[j];
+      }
+      const uint64_t incl = fg::wave_incl_scan_u64(mine), total = fg::shfl_u64(incl, 63);
+      bool ok = total > 0;
+      uint64_t target = c.rest;
+      if (first) {
+        const uint64_t slots = (uint64_t)max((int)c.rest - sh.nan, 0);
+        ok &= slots > 0;
+        target = (total <= slots ? total : slots) - 1;
+      }
+      if (ok && incl - mine <= target && target < incl) {
+        uint64_t before = incl - mine;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (before + b[j] > target) {
+            sh.digit = 4 * lane + j;
+            sh.before = target - before;
+            break;
+          }
+          before += b[j];
+        }
+      }
+    }
+    __syncthreads();
+    if (sh.digit < 0) return false;
+    if (first) c.nan = sh.nan;
+    c.rest = sh.before;
+    c.lo += (uint32_t)sh.digit << shift;
+    c.hi = min(c.hi, c.lo + (1u << shift));
+    }
+    uint32_t ones = 0, zeros = 0;  // bits in which the keys of the class differ
+    list([&](uint32_t a, float x, int) {
+      const bool in = a - c.lo < c.hi - c.lo;
+      const uint32_t key = fg::sort_key32(x);
+      ones |= in ? key : 0u;
+      zeros |= in ? ~key : 0u;
+      return in || (COUNT && a < c.lo);
+    });
+    c.n = sh.n;
+    if (c.n <= kSelList) {
+      if constexpr (!COUNT)
+        c.cut = c.n <= kSmallList ? small_cut(ck, c.n, c.rest, m, kt, tbl, small)
+                                  : list_select<true, false>(ck, c.n, 0, c.rest, m, kt, tbl, sel);
+      return true;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      ones |= (uint32_t)__shfl_xor((int)ones, o, 64);
+      zeros |= (uint32_t)__shfl_xor((int)zeros, o, 64);
+    }
+    if (lane == 0) {
+      sh.ones[tid >> 6] = ones;
+      sh.zeros[tid >> 6] = zeros;
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int w = 0; w < kWaves; ++w) {
+      ones |= sh.ones[w];
+      zeros |= sh.zeros[w];
+    }
+    if ((ones & zeros) == 0) {  // one value: its first elements are kept, as many as rest reaches
+      const uint32_t key = ones;
+      const float v = fg::rank_key_value((uint64_t)key << 32);
+      const uint64_t w = COUNT ? 1ull : exponent_weight(fixed_exponent(m, v, kt), tbl);  // > 0: the class has mass
+      const int idx = split_locate<DT, kThreads, 2>(
+          p, 0, V, [&](float x, int) { return fg::sort_key32(x) == key ? 1ull : 0ull; }, c.rest / w, sh.wred, &sh.found);
+      c.cut = ((uint64_t)key << 32) | (uint64_t)(0xffffffffu - (uint32_t)idx);
+      if constexpr (COUNT) {  // at most top_k elements
+        if (tid == 0) sh.n = 0;
+        __syncthreads();
+        list([&](uint32_t a, float x, int i) {
+          return a < c.lo || (a < c.hi && fg::rank_key(x, (uint32_t)i) >= c.cut);
+        });
+        c.n = sh.n;
+      }
+      return true;
+    }
+    if (c.hi - c.lo == 1) return false;
+  }
+}
+
 // ------------------------------------------------------------------ one workgroup, the row in registers
 // A row of up to 8,192 G logits held by one workgroup, 8 G per thread (element 8 (1024 u + t) + j
 // of thread t): one memory pass and one launch for every kind of draw, by the rule of block_sample.
@@ -589,6 +845,7 @@ struct ResidentShared {
   SelectShared sel;
   SmallShared small;
   uint64_t before;
+  uint32_t least, most;
   int bin, n, nan, tok;
 };
 
@@ -659,8 +916,7 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
 #pragma unroll
   for (int w = 1; w < kWaves; ++w) m = fmaxf(m, sh.wmax[w]);
   const auto weight = [&](float v) { return fg::weight_q40(m, v, kt, sh.exp2); };
-  int bin = 0;  // elements in lower bins are kept, those in it from `cut` on
-  uint64_t cut = 0;
+  RowCut rc{};
   uint64_t hit = 0;  // bit 8 g + j: this thread's element j of group g is listed, later: is kept
   uint32_t e[CUTS ? G : 1][8];  // the exponents stand for the logits from here on
   if constexpr (CUTS) {
@@ -673,67 +929,111 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
       for (int j = 0; j < 8; ++j) {
         e[g][j] = fixed_exponent(m, x[g][j], kt);
         nan += x[g][j] != x[g][j];
-        if (e[g][j] <= kSelAMax)
-          atomicAdd((unsigned long long*)&h[sel_bin(e[g][j]) * kCopies],
-                    (unsigned long long)(count ? 1ull : exponent_weight(e[g][j], sh.exp2)));
       }
     }
     if (nan) atomicAdd(&rs.nan, nan);
-    __syncthreads();
-    if (wave == 0) {  // the bin of the cut: lane l owns bins 4 l .. 4 l + 3
-      uint64_t b[4], mine = 0;
+    const auto fresh_e = [&](int g) {
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        b[j] = 0;
+      for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(e[g][j]));
+    };
+    const auto index_of = [&](int bit) { return ((bit >> 3) * kThreads + tid) * 8 + (bit & 7); };
+    // all exponents in 8 bins an octave, then, while the cut's bin overflows the list, that bin's range in 256
+    uint32_t lo = 0, hi = kSelAMax + 1;
+    int shift = kSelBinShift, n;
+    for (bool first = true;; first = false) {
 #pragma unroll
-        for (int q = 0; q < kCopies; ++q) b[j] += rs.hist[4 * lane + j][q];
-        mine += b[j];
+      for (int g = 0; g < G; ++g) {
+        fresh_e(g);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (e[g][j] - lo < hi - lo)
+            atomicAdd((unsigned long long*)&h[sel_bin(e[g][j] - lo, shift) * kCopies],
+                      (unsigned long long)(count ? 1ull : exponent_weight(e[g][j], sh.exp2)));
       }
-      const uint64_t incl = fg::wave_incl_scan_u64(mine), total = fg::shfl_u64(incl, 63);
-      const uint64_t slots = (uint64_t)max(sp.top_k - rs.nan, 0);  // NaN ranks first and takes slots
-      // slow path (bin stays kSelBins): no weight, or every slot taken by NaN
-      const bool ok = total > 0 && (!count || slots > 0);
-      const uint64_t target = count ? (total <= slots ? total - 1 : slots - 1) : fg::mulhi_u64_u32(total, sp.tp32);
-      if (ok && incl - mine <= target && target < incl) {
-        uint64_t c = incl - mine;
+      __syncthreads();
+      if (wave == 0) {  // the bin of the cut: lane l owns bins 4 l .. 4 l + 3
+        uint64_t b[4], mine = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          if (c + b[j] > target) {
-            rs.bin = 4 * lane + j;
-            rs.before = target - (count ? 0ull : c);  // position of the cut within the list
-            break;
+          b[j] = 0;
+#pragma unroll
+          for (int q = 0; q < kCopies; ++q) b[j] += rs.hist[4 * lane + j][q];
+          mine += b[j];
+        }
+        const uint64_t incl = fg::wave_incl_scan_u64(mine), total = fg::shfl_u64(incl, 63);
+        const uint64_t slots = (uint64_t)max(sp.top_k - rs.nan, 0);  // NaN ranks first and takes slots
+        // block_sample (bin stays kSelBins): no weight, or every slot taken by NaN
+        const bool ok = total > 0 && (!count || slots > 0);
+        const uint64_t target = !first  ? rc.rest
+                                : count ? (total <= slots ? total : slots) - 1
+                                        : fg::mulhi_u64_u32(total, sp.tp32);
+        if (ok && incl - mine <= target && target < incl) {
+          uint64_t c = incl - mine;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if (c + b[j] > target) {
+              rs.bin = 4 * lane + j;
+              rs.before = target - c;  // position of the cut within the bin
+              break;
+            }
+            c += b[j];
           }
-          c += b[j];
         }
       }
-    }
-    __syncthreads();
-    bin = rs.bin;
-    if (bin == kSelBins) {
       __syncthreads();
-      return block_sample<DT>(rowp, V, sp, u, sh);
-    }
-    hit = 0;
+      n = -1;
+      if (rs.bin == kSelBins) break;
+      rc.lo = lo + ((uint32_t)rs.bin << shift);
+      rc.hi = rs.bin == kSelBins - 1 ? hi : min(hi, rc.lo + (1u << shift));
+      rc.rest = rs.before;
+      hit = 0;
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-      fresh(g);
+      for (int g = 0; g < G; ++g) {
+        fresh_e(g);
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (e[g][j] <= kSelAMax && (count ? sel_bin(e[g][j]) <= bin : sel_bin(e[g][j]) == bin))
-          hit |= 1ull << (8 * g + j);
-    }
-    const auto index_of = [&](int bit) { return ((bit >> 3) * kThreads + tid) * 8 + (bit & 7); };
-    if (hit) {
-      int at = atomicAdd(&rs.n, (int)__popcll(hit));
-      for (uint64_t rest = hit; rest; rest &= rest - 1) {
-        const int i = index_of(__builtin_ctzll(rest));
-        if (at < kSelList) rs.ck[at] = fg::rank_key(fg::load_elem<DT>(rowp, i), (uint32_t)i);
-        ++at;
+        for (int j = 0; j < 8; ++j)
+          if (e[g][j] < rc.hi && (count || e[g][j] >= rc.lo)) hit |= 1ull << (8 * g + j);
       }
+      if (hit) {
+        int at = atomicAdd(&rs.n, (int)__popcll(hit));
+        for (uint64_t rest = hit; rest; rest &= rest - 1) {
+          const int i = index_of(__builtin_ctzll(rest));
+          if (at < kSelList) rs.ck[at] = fg::rank_key(fg::load_elem<DT>(rowp, i), (uint32_t)i);
+          ++at;
+        }
+      }
+      __syncthreads();
+      n = rs.n;
+      if (G * 8 * kThreads <= kSelList || n <= kSelList) break;
+      uint32_t least = 0xffffffffu, most = 0;
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        fresh_e(g);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const bool in = e[g][j] >= rc.lo && e[g][j] < rc.hi;
+          least = min(least, in ? e[g][j] : 0xffffffffu);
+          most = max(most, in ? e[g][j] : 0u);
+        }
+      }
+      for (int i = tid; i < kCopies * kSelBins; i += kThreads) (&rs.hist[0][0])[i] = 0;
+      if (tid == 0) {
+        rs.least = 0xffffffffu;
+        rs.most = 0;
+      }
+      __syncthreads();  // rs.n and rs.bin have been read
+      atomicMin(&rs.least, least);
+      atomicMax(&rs.most, most);
+      if (tid == 0) rs.n = 0;
+      __syncthreads();
+      lo = rs.least;
+      hi = rs.most + 1;
+      n = -1;
+      if (hi - lo == 1) break;  // long ties
+      shift = max(0, 24 - (int)__clz((int)(hi - 1 - lo)));
     }
-    __syncthreads();
-    const int n = rs.n;
-    if (n > kSelList || sp.top_k > kSelTopK) {
+    if (n < 0) {
       __syncthreads();
       return block_sample<DT>(rowp, V, sp, u, sh);
     }
@@ -742,11 +1042,11 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
       __syncthreads();
       return tok;
     }
-    cut = n <= kSmallList ? small_cut(rs.ck, n, rs.before, m, kt, sh.exp2, rs.small)
-                          : list_select<true, false>(rs.ck, n, 0, rs.before, m, kt, sh.exp2, rs.sel);
+    rc.cut = n <= kSmallList ? small_cut(rs.ck, n, rc.rest, m, kt, sh.exp2, rs.small)
+                             : list_select<true, false>(rs.ck, n, 0, rc.rest, m, kt, sh.exp2, rs.sel);
     for (uint64_t rest = hit; rest; rest &= rest - 1) {
       const int i = index_of(__builtin_ctzll(rest));
-      if (fg::rank_key(fg::load_elem<DT>(rowp, i), (uint32_t)i) < cut) hit &= ~(rest & -rest);
+      if (fg::rank_key(fg::load_elem<DT>(rowp, i), (uint32_t)i) < rc.cut) hit &= ~(rest & -rest);
     }
   }
   // the draw among the kept elements, in vocabulary order: q-mass of each (group, wave)
@@ -763,7 +1063,7 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       if constexpr (CUTS) {
-        if (sel_bin(e[g][j]) < bin || ((hit >> (8 * g + j)) & 1)) w += exponent_weight(e[g][j], sh.exp2);
+        if (e[g][j] < rc.lo || ((hit >> (8 * g + j)) & 1)) w += exponent_weight(e[g][j], sh.exp2);
       } else {
         w += weight(x[g][j]);
       }
@@ -810,8 +1110,8 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
       const int i = (g * kThreads + tid) * 8 + j;
       w[j] = weight(v[j]);
       if constexpr (CUTS) {
-        const int b = sel_bin(fixed_exponent(m, v[j], kt));
-        if (b > bin || (b == bin && fg::rank_key(v[j], (uint32_t)i) < cut)) w[j] = 0;
+        const uint32_t a = fixed_exponent(m, v[j], kt);
+        if (a >= rc.hi || (a >= rc.lo && fg::rank_key(v[j], (uint32_t)i) < rc.cut)) w[j] = 0;
       }
       sum += w[j];
     }
@@ -1011,10 +1311,10 @@ struct SplitArgs {
   float* part_max;           // [rows, kSplitChunks]
   uint64_t* part_key;
   uint64_t* part_sum;
-  uint64_t* part_gsum;       // [rows, kSplitChunks, kSplitMaxGroups] q-mass per group of kSplitGroup
+  uint64_t* part_gsum;       // [rows, kSplitChunks, kSplitMaxGroups] q-mass per group of kSplitGroup (top-p: SelState)
   int groups;                // groups per chunk (group sums kept only up to kSplitMaxGroups)
   float* row_m;              // [rows] row maximum (sum launch -> pick launch)
-  uint64_t* row_best;        // [rows] first maximum's rank key
+  uint64_t* row_best;        // [rows] first maximum's rank key; restricted draws: bin_shift
   // row maxima parts read by the draw launch: [rows, src_stride], src_parts used
   const float* src_max;
   const uint64_t* src_key;
@@ -1058,19 +1358,8 @@ constexpr int kSplitMaxGroups = 16;
 // of 8,192 and one group of the second).
 FG_DEVICE bool split_group_live(int base, int u, int hi) { return base + u * kSplitThreads * 8 < hi; }
 
-// Loads elements i0 .. i0 + 7 of a chunk ending at hi; past hi come -inf, whose weight is
-// 0 against any row maximum, so the weights need no per-element test.
-template <int DT>
-FG_DEVICE void split_load8(const char* p, int i0, int hi, float (&x)[8]) {
-  if (i0 + 8 <= hi) {
-    fg::load8<DT>(p, i0, x);
-    return;
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) x[j] = i0 + j < hi ? fg::load_elem<DT>(p, i0 + j) : -INFINITY;
-}
-
-// Chunk maxima (raw maximum, NaN ignored, and with KEY the first-maximum rank key). Per pass a thread
+// Chunk maxima (raw maximum, NaN ignored, with KEY the first-maximum rank key, without it the least
+// logit of the whole groups of 8 in its place: bin_shift's range, which need not be exact). Per pass a thread
 // takes the maximum of its elements (NaN ignored) and then the first index holding it (the
 // first NaN when there is one, which ranks highest), and forms one rank key per pass instead
 // of one per element.
@@ -1082,7 +1371,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_max_kernel(SplitArgs a) {
   __shared__ uint64_t skey[kSplitWaves];
   const char* p = split_row<DT>(a, r);
   const int lo = c * a.chunk, hi = min(a.vocab, lo + a.chunk);
-  float mx = -INFINITY;
+  float mx = -INFINITY, low = INFINITY;
   uint64_t best = 0;
   for (int base = lo; base < hi; base += kSplitPass) {
     float x[kSplitLoads][8];
@@ -1096,11 +1385,14 @@ __global__ void __launch_bounds__(kSplitThreads) split_max_kernel(SplitArgs a) {
 #pragma unroll
     for (int u = 0; u < kSplitLoads; ++u) {
       if (!split_group_live(base, u, hi)) continue;
+      float low8 = INFINITY;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         pm = fmaxf(pm, x[u][j]);
-        nan |= x[u][j] != x[u][j];
+        if constexpr (KEY) nan |= x[u][j] != x[u][j];
+        else low8 = fminf(low8, x[u][j]);
       }
+      if (!KEY && base + (u * kSplitThreads + (int)threadIdx.x) * 8 + 8 <= hi) low = fminf(low, low8);
     }
     if constexpr (!KEY) {
       mx = fmaxf(mx, pm);
@@ -1124,6 +1416,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_max_kernel(SplitArgs a) {
   }
   mx = fg::wave_max(mx);
   if constexpr (KEY) best = fg::wave_max_u64(best);
+  else best = __float_as_uint(wave_min(low));
   const int wave = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
     smax[wave] = mx;
@@ -1134,10 +1427,11 @@ __global__ void __launch_bounds__(kSplitThreads) split_max_kernel(SplitArgs a) {
 #pragma unroll
     for (int w = 1; w < kSplitWaves; ++w) {
       mx = fmaxf(mx, smax[w]);
-      best = skey[w] > best ? skey[w] : best;
+      if constexpr (KEY) best = skey[w] > best ? skey[w] : best;
+      else best = __float_as_uint(fminf(__uint_as_float((uint32_t)best), __uint_as_float((uint32_t)skey[w])));
     }
     a.part_max[r * kSplitChunks + c] = fmaxf(smax[0], mx);
-    if constexpr (KEY) a.part_key[r * kSplitChunks + c] = skey[0] > best ? skey[0] : best;
+    a.part_key[r * kSplitChunks + c] = KEY && skey[0] > best ? skey[0] : best;
   }
 }
 
@@ -1231,61 +1525,6 @@ __global__ void __launch_bounds__(kSplitThreads) split_sum_kernel(SplitArgs a) {
       a.row_best[r] = best;
     }
   }
-}
-
-// First index in [lo, hi) whose inclusive running mass w(x, index) exceeds target (the whole
-// block of THREADS; -1 if none), scanned in index order one group of THREADS x 8 elements at a
-// time (thread t holds 8 consecutive elements of a group), stopping at the group that holds
-// the target. The LOADS groups of a pass are loaded together. wsum: THREADS / 64 words.
-template <int DT, int THREADS, int LOADS, class W>
-FG_DEVICE int split_locate(const char* p, int lo, int hi, W&& weight, uint64_t target, uint64_t* wsum, int* found) {
-  constexpr int WAVES = THREADS / 64;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (tid == 0) *found = -1;
-  uint64_t run = 0;  // block-uniform
-  bool done = false;
-  for (int base = lo; base < hi && !done; base += THREADS * 8 * LOADS) {
-    float x[LOADS][8];
-#pragma unroll
-    for (int u = 0; u < LOADS; ++u)
-      if (base + u * THREADS * 8 < hi) split_load8<DT>(p, base + (u * THREADS + tid) * 8, hi, x[u]);
-#pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
-      if (base + u * THREADS * 8 >= hi) break;  // uniform
-      const int i0 = base + (u * THREADS + tid) * 8;
-      uint64_t mine = 0;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) mine += weight(x[u][j], i0 + j);
-      const uint64_t incl = fg::wave_incl_scan_u64(mine);
-      __syncthreads();  // wsum of the previous group has been read
-      if (lane == 63) wsum[wave] = incl;
-      __syncthreads();
-      uint64_t woff = 0, stot = 0;
-#pragma unroll 4
-      for (int w = 0; w < WAVES; ++w) {
-        if (w < wave) woff += wsum[w];
-        stot += wsum[w];
-      }
-      if (run + stot > target) {  // uniform: this group holds the target
-        uint64_t cum = run + woff + incl - mine;
-        if (cum <= target && target < cum + mine) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            cum += weight(x[u][j], i0 + j);
-            if (cum > target) {
-              *found = i0 + j;
-              break;
-            }
-          }
-        }
-        done = true;
-        break;
-      }
-      run += stot;
-    }
-  }
-  __syncthreads();
-  return *found;
 }
 
 // Outputs of a draw: a token per row, or one step of the acceptance walk.
@@ -1408,8 +1647,8 @@ __global__ void __launch_bounds__(kSplitThreads) split_pick_kernel(SplitArgs a, 
 //  (4) one workgroup per row selects the cut exactly among the list (64-bit rank keys, so ties
 //      resolve in index order) and locates the draw: top-k among the list, top-p in the one
 //      chunk whose running kept mass crosses the target.
-// A row whose list overflows (flat rows), whose total is 0 or whose top-k slots are all taken by
-// NaN is drawn by block_sample in launch (4).
+// A row whose list overflows (flat rows) is narrowed further in launch (4) (narrow_cut); one whose total
+// is 0 or whose top-k slots are all taken by NaN is drawn by block_sample there.
 //
 // Bound by VALU and LDS issue of the two weighing passes. An 8-bit radix select over the key
 // bits needed four histogram launches instead of one: the first level's 256 bins are the sign
@@ -1421,10 +1660,10 @@ static_assert(kSelBins == kSplitThreads, "one histogram bin per thread");
 // Where the cut of one row lies (written by chunk 0 of launch 3).
 struct SelState {
   uint64_t rest;  // position of the cut within the list: q-mass (top-p) or count (top-k) before it
-  int32_t slow;   // the row is drawn by block_sample
+  int32_t slow;   // the row has no weight, or NaN takes every slot: block_sample draws it
   int32_t all;    // every listed element is kept (top-k with no more candidates than slots)
   int32_t bin;    // the cut's bin
-  int32_t pad;
+  int32_t crowded;  // part_gsum holds each chunk's least and largest listed key and their count
 };
 
 template <int DT, bool COUNT>
@@ -1435,7 +1674,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) 
   using AtomicBin = std::conditional_t<COUNT, unsigned int, unsigned long long>;
   __shared__ uint64_t tbl[COUNT ? 1 : 1024];
   __shared__ Bin h[kSelBins][kCopies];
-  __shared__ float smax[kSplitWaves];
+  __shared__ float smax[kSplitWaves], smin[kSplitWaves];
   __shared__ int s_nan;
   const char* p = split_row<DT>(a, r);
   const int lo = c * a.chunk, hi = min(a.vocab, lo + a.chunk);
@@ -1447,15 +1686,31 @@ __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) 
 #pragma unroll
   for (int q = 0; q < kCopies; ++q) (&h[0][0])[q * kSplitThreads + tid] = 0;
   if (tid == 0) s_nan = 0;
-  float mx = -INFINITY;  // row maximum from the parts
-  for (int q = tid; q < a.src_parts; q += kSplitThreads) mx = fmaxf(mx, a.src_max[r * a.src_stride + q]);
-  mx = fg::wave_max(mx);
-  if ((tid & 63) == 0) smax[tid >> 6] = mx;
+  const bool ranged = a.src_max == a.part_max;  // given maxima come without the least logit
+  float mx = -INFINITY, low = INFINITY;         // row maximum and least logit from the parts
+  for (int q = tid; q < a.src_parts; q += kSplitThreads) {
+    mx = fmaxf(mx, a.src_max[r * a.src_stride + q]);
+    if (ranged) low = fminf(low, __uint_as_float((uint32_t)a.src_key[r * a.src_stride + q]));
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    low = fminf(low, __shfl_xor(low, o, 64));
+  }
+  if ((tid & 63) == 0) {
+    smax[tid >> 6] = mx;
+    smin[tid >> 6] = low;
+  }
   __syncthreads();
   mx = smax[0];
+  low = smin[0];
 #pragma unroll
-  for (int w = 1; w < kSplitWaves; ++w) mx = fmaxf(mx, smax[w]);
+  for (int w = 1; w < kSplitWaves; ++w) {
+    mx = fmaxf(mx, smax[w]);
+    low = fminf(low, smin[w]);
+  }
   const float m = mx, kt = split_kt(a);
+  const int shift = ranged ? bin_shift(m, low, kt) : kSelBinShift;
   Bin* mine = &h[0][tid % kCopies];
   int nan = 0;
   for (int base = lo; base < hi; base += kSplitPass) {
@@ -1473,7 +1728,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) 
         if constexpr (COUNT) nan += x[u][j] != x[u][j];
         if (e <= kSelAMax) {
           const Bin w = COUNT ? (Bin)1 : (Bin)fg::weight_q40(m, x[u][j], kt, tbl);
-          atomicAdd((AtomicBin*)&mine[sel_bin(e) * kCopies], (AtomicBin)w);
+          atomicAdd((AtomicBin*)&mine[sel_bin(e, shift) * kCopies], (AtomicBin)w);
         }
       }
     }
@@ -1491,6 +1746,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) 
     if (c == 0) {
       a.list_n[r] = 0;
       a.row_m[r] = m;
+      a.row_best[r] = (uint64_t)shift;
     }
   }
 }
@@ -1518,7 +1774,8 @@ __global__ void __launch_bounds__(kSplitThreads) split_gather_kernel(SplitArgs a
   if (split_skip(a, r)) return;
   __shared__ uint64_t wsum[kSplitWaves];
   __shared__ int s_bin, s_base;
-  __shared__ uint64_t s_before;
+  __shared__ uint64_t s_before, s_mass;
+  __shared__ uint32_t s_least, s_most;
   const char* p = split_row<DT>(a, r);
   const int lo = c * a.chunk, hi = min(a.vocab, lo + a.chunk);
   float x[kSplitLoads][8];
@@ -1553,10 +1810,19 @@ __global__ void __launch_bounds__(kSplitThreads) split_gather_kernel(SplitArgs a
   if (incl - v <= target && target < incl) {  // one thread, unless the total is 0
     s_bin = tid;
     s_before = incl - v;
+    s_mass = v;
+  }
+  if (tid == 0) {
+    s_least = 0xffffffffu;
+    s_most = 0;
   }
   __syncthreads();
   const int bin = s_bin;
-  if (c == 0 && tid == 0) a.sel[r] = SelState{slow ? 0 : COUNT ? target : target - s_before, slow, all, bin, 0};
+  const RowCut rc = bin_cut(bin, (int)a.row_best[r], 0);
+  // top-p: half a list or more in the bin, by its q-mass: is it one value?
+  const bool crowded = !COUNT && !slow && s_mass > (uint64_t)(kSelList / 2) * exponent_weight(rc.lo, fg::kExp2Table);
+  if (c == 0 && tid == 0)
+    a.sel[r] = SelState{slow ? 0 : COUNT ? target : target - s_before, slow, all, bin, crowded};
   if (slow) return;
   if constexpr (!COUNT) {  // this chunk's q-mass above the cut's bin
     uint64_t above;
@@ -1565,9 +1831,11 @@ __global__ void __launch_bounds__(kSplitThreads) split_gather_kernel(SplitArgs a
   }
   const float m = a.row_m[r], kt = split_kt(a);
   uint32_t* list = a.list + (size_t)r * kSelList;
+  uint32_t least = 0xffffffffu, most = 0;  // keys listed here (crowded)
+  int listed_here = 0;
   const auto listed = [&](float xv) {
     const uint32_t e = fixed_exponent(m, xv, kt);
-    return e <= kSelAMax && (COUNT ? sel_bin(e) <= bin : sel_bin(e) == bin);
+    return e < rc.hi && (COUNT || e >= rc.lo);
   };
   for (int base = lo; base < hi; base += kSplitPass) {
     if (base != lo) {
@@ -1583,8 +1851,20 @@ __global__ void __launch_bounds__(kSplitThreads) split_gather_kernel(SplitArgs a
       for (int j = 0; j < 8; ++j)
         if (listed(x[u][j])) hit |= 1ull << (8 * u + j);
     }
+    if (crowded) {
+#pragma unroll
+      for (int u = 0; u < kSplitLoads; ++u)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (hit >> (8 * u + j) & 1) {
+            const uint32_t key = fg::sort_key32(x[u][j]);
+            least = min(least, key);
+            most = max(most, key);
+          }
+    }
     uint64_t count;
     const int at = (int)split_incl_scan((uint64_t)__popcll(hit), wsum, count) - __popcll(hit);
+    listed_here += (int)count;
     if (tid == 0 && count) s_base = atomicAdd(&a.list_n[r], (int)count);
     __syncthreads();
     int o = s_base + at;
@@ -1595,6 +1875,16 @@ __global__ void __launch_bounds__(kSplitThreads) split_gather_kernel(SplitArgs a
       ++o;
     }
   }
+  if (crowded) {
+    atomicMin(&s_least, least);
+    atomicMax(&s_most, most);
+    __syncthreads();
+    if (tid == 0) {
+      uint64_t* info = a.part_gsum + ((size_t)r * kSplitChunks + c) * kSplitMaxGroups;
+      info[0] = (uint64_t)s_least << 32 | s_most;
+      info[1] = (uint64_t)listed_here;
+    }
+  }
 }
 
 template <int DT, bool COUNT, bool WALK>
@@ -1602,6 +1892,7 @@ __global__ void __launch_bounds__(kThreads) split_select_kernel(SplitArgs a, Dra
   __shared__ Shared sh;
   __shared__ SelectShared sel;
   __shared__ SmallShared small;
+  __shared__ NarrowShared narrow;
   __shared__ uint64_t ck[kSelList];
   __shared__ uint64_t s_kept[kSplitChunks][kCopies];  // kept q-mass per chunk
   const int r = blockIdx.x, tid = threadIdx.x;
@@ -1620,30 +1911,92 @@ __global__ void __launch_bounds__(kThreads) split_select_kernel(SplitArgs a, Dra
   const SelState st = a.sel[r];
   const int n = a.list_n[r];
   const char* rowp = split_row<DT>(a, r);
-  int tok;
-  if (st.slow || n > kSelList) {
-    tok = block_sample<DT>(rowp, a.vocab, sp, u, sh);
-  } else {
-    const float m = a.row_m[r], kt = split_kt(a);
-    for (int i = tid; i < n; i += kThreads) {
-      const uint32_t idx = a.list[(size_t)r * kSelList + i];
-      ck[i] = fg::rank_key(fg::load_elem<DT>(rowp, idx), idx);
-    }
+  const float m = a.row_m[r], kt = split_kt(a);
+  const bool flat = n > kSelList;
+  bool ok = !st.slow;
+  int tok = -1;
+  if (ok) {
     fg::exp2_table_to_lds(sh.exp2);
     if (!COUNT && tid < kSplitChunks * kCopies)
-      s_kept[tid / kCopies][tid % kCopies] = tid % kCopies ? 0ull : a.part_a[r * kSplitChunks + tid / kCopies];
+      s_kept[tid / kCopies][tid % kCopies] = tid % kCopies || flat ? 0ull : a.part_a[r * kSplitChunks + tid / kCopies];
+  }
+  if constexpr (COUNT) {
+    int64_t slots = st.all ? (int64_t)n : (int64_t)st.rest + 1;
+    int listed = n;
+    if (ok && flat) {
+      RowCut c{0, kSelAMax + 1, 0, (uint64_t)a.top_k, 0, 0};
+      ok = narrow_cut<DT, true>(rowp, a.vocab, m, kt, sh.exp2, ck, c, narrow, sel, small);
+      slots = (int64_t)a.top_k - c.nan;
+      listed = c.n;
+    } else if (ok) {
+      for (int i = tid; i < n; i += kThreads) {
+        const uint32_t idx = a.list[(size_t)r * kSelList + i];
+        ck[i] = fg::rank_key(fg::load_elem<DT>(rowp, idx), idx);
+      }
+    }
     __syncthreads();
-    if constexpr (COUNT) {
-      tok = list_draw(ck, n, st.all ? (int64_t)n : (int64_t)st.rest + 1, sp.tp32, u, m, kt, sh.exp2, sel, small);
+    if (ok) tok = list_draw(ck, listed, slots, sp.tp32, u, m, kt, sh.exp2, sel, small);
+  } else if (ok) {
+    RowCut c = bin_cut(st.bin, (int)a.row_best[r], st.rest);
+    const auto kept_weight = [&](float x, int i) -> uint64_t {
+      const uint32_t e = fixed_exponent(m, x, kt);
+      return e < c.lo || (e < c.hi && fg::rank_key(x, (uint32_t)i) >= c.cut) ? exponent_weight(e, sh.exp2) : 0ull;
+    };
+    // a flat row whose bin holds one value is cut by index, from the chunks' counts of it
+    uint32_t least = 0xffffffffu, most = 0;
+    int ties = 0;  // lane l: chunk l's
+    if (flat && st.crowded) {
+      if ((tid & 63) < kSplitChunks) {
+        const uint64_t* info = a.part_gsum + ((size_t)r * kSplitChunks + (tid & 63)) * kSplitMaxGroups;
+        ties = (int)info[1];
+        if (ties) {
+          least = (uint32_t)(info[0] >> 32);
+          most = (uint32_t)info[0];
+        }
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        least = min(least, (uint32_t)__shfl_xor((int)least, o, 64));
+        most = max(most, (uint32_t)__shfl_xor((int)most, o, 64));
+      }
+    }
+    if (least == most) {
+      __syncthreads();  // sh.exp2
+      const float v = fg::rank_key_value((uint64_t)least << 32);
+      const uint64_t w = exponent_weight(fixed_exponent(m, v, kt), sh.exp2), last = c.rest / w;
+      const uint64_t upto = fg::wave_incl_scan_u64((uint64_t)ties);
+      const int c1 = (int)__builtin_ctzll(__ballot(last < upto));  // the chunk of the last kept one
+      const uint64_t in1 = last - fg::shfl_u64(upto - (uint64_t)ties, c1);
+      const int idx = split_locate<DT, kThreads, 2>(
+          rowp, c1 * a.chunk, min(a.vocab, (c1 + 1) * a.chunk),
+          [&](float x, int) { return fg::sort_key32(x) == least ? 1ull : 0ull; }, in1, sh.wsum, &sh.i32b[0]);
+      c.cut = ((uint64_t)least << 32) | (uint64_t)(0xffffffffu - (uint32_t)idx);
+      if (tid < kSplitChunks)
+        s_kept[tid][0] = a.part_a[r * kSplitChunks + tid] + w * (tid < c1 ? (uint64_t)ties : tid == c1 ? in1 + 1 : 0ull);
+    } else if (flat) {
+      ok = narrow_cut<DT, false>(rowp, a.vocab, m, kt, sh.exp2, ck, c, narrow, sel, small);
+      if (ok)
+        for_row8<DT>(rowp, a.vocab, [&](const float(&x)[8], int i0) {
+          uint64_t w = 0;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) w += kept_weight(x[j], i0 + j);
+          if (w) atomicAdd((unsigned long long*)&s_kept[i0 / a.chunk][tid % kCopies], (unsigned long long)w);
+        });
     } else {
-      const uint64_t cut = n <= kSmallList ? small_cut(ck, n, st.rest, m, kt, sh.exp2, small)
-                                           : list_select<true, false>(ck, n, 0, st.rest, m, kt, sh.exp2, sel);
-      const int bin = st.bin;
+      for (int i = tid; i < n; i += kThreads) {
+        const uint32_t idx = a.list[(size_t)r * kSelList + i];
+        ck[i] = fg::rank_key(fg::load_elem<DT>(rowp, idx), idx);
+      }
+      __syncthreads();
+      c.cut = n <= kSmallList ? small_cut(ck, n, c.rest, m, kt, sh.exp2, small)
+                              : list_select<true, false>(ck, n, 0, c.rest, m, kt, sh.exp2, sel);
       for (int i = tid; i < n; i += kThreads)
-        if (ck[i] >= cut)
+        if (ck[i] >= c.cut)
           atomicAdd((unsigned long long*)&s_kept[fg::rank_key_index(ck[i]) / (uint32_t)a.chunk][tid % kCopies],
                     (unsigned long long)fg::weight_q40(m, fg::rank_key_value(ck[i]), kt, sh.exp2));
-      __syncthreads();
+    }
+    __syncthreads();
+    if (ok) {
       // every wave: lane l holds chunk l's kept mass
       uint64_t kept = 0;
       if ((tid & 63) < kSplitChunks)
@@ -1652,14 +2005,13 @@ __global__ void __launch_bounds__(kThreads) split_select_kernel(SplitArgs a, Dra
       const uint64_t incl = fg::wave_incl_scan_u64(kept), target = fg::mulhi_u64_u32(fg::shfl_u64(incl, 63), u);
       const int c2 = (int)__builtin_ctzll(__ballot(target < incl));  // the total exceeds the target
       const uint64_t before = fg::shfl_u64(incl - kept, c2);
-      const auto kept_weight = [&](float x, int i) -> uint64_t {
-        const uint32_t e = fixed_exponent(m, x, kt);
-        const int b = sel_bin(e);
-        return b < bin || (b == bin && fg::rank_key(x, (uint32_t)i) >= cut) ? exponent_weight(e, sh.exp2) : 0ull;
-      };
       tok = split_locate<DT, kThreads, 2>(rowp, c2 * a.chunk, min(a.vocab, (c2 + 1) * a.chunk), kept_weight,
                                           target - before, sh.wsum, &sh.i32b[0]);
     }
+  }
+  if (!ok) {
+    __syncthreads();
+    tok = block_sample<DT>(rowp, a.vocab, sp, u, sh);
   }
   if constexpr (WALK) {
     if (tid < 64)
@@ -1678,8 +2030,8 @@ __global__ void __launch_bounds__(kThreads) split_select_kernel(SplitArgs a, Dra
 // lists, dropping first what lies below (a) some chunk's bound or (b) the least of the
 // chunks' bounds on their ceil(top_k / 16)-th elements: at least top_k elements of the row lie at
 // or above either. Elements 40 octaves below the chunk's maximum and -inf weigh 0 against any
-// row maximum and are not listed; NaN, which ranks first, always is. A chunk with more than
-// kTopkList candidates (long ties) sends the row to block_sample.
+// row maximum and are not listed; NaN, which ranks first, always is. A row with a chunk of more
+// than kTopkList candidates (flat rows, long ties) is cut by narrow_cut over the whole row.
 // Bound by launch and memory latency: top-k 50 at 32 x 151,936 bf16 took 207 us in one workgroup per
 // row, 47 with the four launches above, 25 with these two.
 constexpr int kTopkMax = 256;
@@ -1690,7 +2042,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_topk_kernel(SplitArgs a) 
   const int c = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, wave = tid >> 6;
   if (split_skip(a, r)) return;
   __shared__ uint32_t h[kSelBins];
-  __shared__ float smax[kSplitWaves], slow[2][kSplitWaves];
+  __shared__ float smax[kSplitWaves], smin[kSplitWaves], slow[2][kSplitWaves];
   __shared__ uint64_t wsum[kSplitWaves];
   __shared__ int s_bin[2];
   const char* p = split_row<DT>(a, r);
@@ -1708,19 +2060,27 @@ __global__ void __launch_bounds__(kSplitThreads) split_topk_kernel(SplitArgs a) 
 #pragma unroll
     for (int j = 0; j < 8; ++j) sm[j >> 2] = fmaxf(sm[j >> 2], x[u][j]);
   }
-  float m = fg::wave_max(fmaxf(sm[0], sm[1]));
-  if ((tid & 63) == 0) smax[wave] = m;
+  float m = fg::wave_max(fmaxf(sm[0], sm[1])), low = wave_min(fminf(above_inf(sm[0]), above_inf(sm[1])));
+  if ((tid & 63) == 0) {
+    smax[wave] = m;
+    smin[wave] = low;
+  }
   __syncthreads();
   m = smax[0];
+  low = smin[0];
 #pragma unroll
-  for (int w = 1; w < kSplitWaves; ++w) m = fmaxf(m, smax[w]);
+  for (int w = 1; w < kSplitWaves; ++w) {
+    m = fmaxf(m, smax[w]);
+    low = fminf(low, smin[w]);
+  }
   const float kt = split_kt(a);
+  const int shift = bin_shift(m, low, kt);
   // bin of a set's maximum, kSelBins for one that weighs 0 against any maximum from m on
   int sb[2];
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
     const uint32_t e = fixed_exponent(m, sm[q], kt);
-    sb[q] = e <= kSelAMax ? sel_bin(e) : kSelBins;
+    sb[q] = e <= kSelAMax ? sel_bin(e, shift) : kSelBins;
     if (sb[q] < kSelBins) atomicAdd(&h[sb[q]], 1u);
   }
   __syncthreads();
@@ -1781,6 +2141,7 @@ __global__ void __launch_bounds__(kThreads) split_topk_draw_kernel(SplitArgs a, 
   __shared__ Shared sh;
   __shared__ SelectShared sel;
   __shared__ SmallShared small;
+  __shared__ NarrowShared narrow;
   __shared__ uint64_t ck[kSelList];
   __shared__ int s_n;
   const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, c = tid >> 6;
@@ -1828,8 +2189,14 @@ __global__ void __launch_bounds__(kThreads) split_topk_draw_kernel(SplitArgs a, 
     }
   __syncthreads();
   int tok = -1;
-  if (!full && s_n > 0)
-    tok = list_draw(ck, s_n, sp.top_k, sp.tp32, u, m, split_kt(a), sh.exp2, sel, small);
+  int n = s_n;
+  int64_t slots = sp.top_k;
+  if (full) {
+    RowCut c2{0, kSelAMax + 1, 0, (uint64_t)sp.top_k, 0, 0};
+    n = narrow_cut<DT, true>(rowp, a.vocab, m, split_kt(a), sh.exp2, ck, c2, narrow, sel, small) ? c2.n : 0;
+    slots -= c2.nan;
+  }
+  if (n > 0) tok = list_draw(ck, n, slots, sp.tp32, u, m, split_kt(a), sh.exp2, sel, small);
   __syncthreads();
   if (tok < 0) tok = block_sample<DT>(rowp, a.vocab, sp, u, sh);
   if constexpr (WALK) {

@@ -79,3 +79,105 @@ def test_restricted_walk_step_with_given_maxima(kw):
     for other in res[1:]:
         for a, b in zip(res[0], other):
             assert np.array_equal(a, b)
+
+
+def _oracle(xs, noise, kw):
+    return OS.sample_rows(xs, noise, do_sample=not kw.get("greedy", False), temperature=kw.get("temperature", 1.0),
+                          top_p=kw.get("top_p", 1.0), top_k=kw.get("top_k"))
+
+
+def _flat_rows(V, seed):
+    """Rows whose logits crowd a few bins of the exponent, or one."""
+    g = np.random.default_rng(seed)
+    z = g.standard_normal((10, V)).astype(np.float32)
+    x = z * np.float32(0.3)
+    x[1] = z[1] * 0.05
+    x[2] = z[2] * 1e-3
+    x[3] = z[3] * 1e-6
+    x[4] = 7.25                                                            # one value
+    x[5] = np.where(g.random(V) < 0.7, 1.0, 1.5)                           # two
+    x[6] = torch.from_numpy(z[6] * 0.3 + 20).to(torch.bfloat16).float().numpy()  # a few values far from zero
+    x[7] = z[7] * 0.01
+    x[7, V // 5: V // 4] = -np.inf
+    x[8] = 0.5
+    x[8, :3] = np.nan
+    x[8, 5] = 9.0                                                          # one logit above long ties
+    x[9] = z[9] * 0.02
+    x[9, ::7] = -30.0                                                      # a crowd far below another
+    return torch.from_numpy(x)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [8200, 9000, 16384, 20003, 32768, 50304, 152064, 163848])
+def test_flat_rows_match_oracle(dtype, V):
+    """Cuts in bins with more logits than a list: sampled, and as walk steps that form the row maxima,
+    are given them, or have one workgroup per row."""
+    from flashgrpo_amd import kernels as K
+
+    x = _flat_rows(V, V).to(dtype)
+    R = x.shape[0]
+    xd, xs = x.to(DEV), x.float().numpy()
+    noise = np.random.default_rng(2).integers(0, 2 ** 32, (R, 1), dtype=np.uint32)
+    nd = torch.from_numpy(noise.view(np.int32)).to(DEV)
+    big = torch.nan_to_num(x.float(), nan=float("-inf"), neginf=float("-inf")).amax(1, keepdim=True).to(DEV)
+    parts = (big.contiguous(), torch.zeros(R, 1, dtype=torch.int64, device=DEV))  # a cut needs the maxima alone
+    tt = torch.full((R, 2), -5, dtype=torch.int32, device=DEV)
+    par = torch.tensor([[-1, 0]] * R, dtype=torch.int32, device=DEV)
+    nn = torch.full((R,), 2, dtype=torch.int32, device=DEV)
+    for kw in (dict(top_p=0.9), dict(top_p=0.4, temperature=0.8), dict(top_k=50), dict(top_k=1000, top_p=0.7),
+               dict(top_k=4096)):
+        want = _oracle(xs, noise, kw)
+        assert np.array_equal(K.sample_tokens(xd, noise=nd, **kw).cpu().numpy(), want), (V, dtype, kw)
+        for split, pt in ((True, None), (True, parts), (False, None)):
+            wk = K.walk_begin(tt, par, nn, acc_stride=2)
+            K.walk_rows(wk, 2)
+            K.walk_step(wk, xd, tt, par, nn, walk_step=0, noise=nd, split=split, parts=pt, **kw)
+            assert np.array_equal(wk["correction"].cpu().numpy(), want), (V, dtype, kw, split, pt is not None)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [163848, 200008])
+def test_chunks_of_two_passes_match_oracle(dtype, V):
+    """Rows whose 16 chunks are longer than a workgroup's pass (10,240 logits), with cuts and ties in the
+    second pass."""
+    from flashgrpo_amd import kernels as K
+
+    x = _rows(V, V)
+    chunk = (-(-V // 16) + 7) // 8 * 8
+    x[0, 10_240: chunk] += 8.0                      # the mass in the first chunk's second pass
+    x[1, 2 * chunk + 10_240: 3 * chunk] = 12.0      # a tie there
+    x[3, 5 * chunk + 10_000: 5 * chunk + 10_250] = 9.0   # a tie across the two passes
+    x = x.to(dtype)
+    noise = np.random.default_rng(3).integers(0, 2 ** 32, (12, 1), dtype=np.uint32)
+    nd = torch.from_numpy(noise.view(np.int32)).to(DEV)
+    for kw in (dict(top_p=0.95), dict(top_p=0.3), dict(top_k=5), dict(top_k=50, top_p=0.9), dict(top_k=256),
+               dict(top_k=1500)):
+        got = K.sample_tokens(x.to(DEV), noise=nd, **kw).cpu().numpy()
+        assert np.array_equal(got, _oracle(x.float().numpy(), noise, kw)), (V, dtype, kw)
+
+
+@pytest.mark.parametrize("kw", [dict(top_p=0.9), dict(top_k=1000)])
+def test_flat_rows_take_no_more_than_others(kw):
+    """A flat row costs about what any other does: it once went to a draw of many passes by one
+    workgroup (top-p 5.8 times as long, top-k 1,000 4.9)."""
+    from flashgrpo_amd import kernels as K
+
+    g = torch.Generator(device=DEV).manual_seed(1)
+    z = torch.randn(64, 152064, device=DEV, generator=g)
+
+    def best_us(x):
+        t = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                K.sample_tokens(x, seed=1, **kw)
+            b.record()
+            torch.cuda.synchronize()
+            t.append(a.elapsed_time(b) * 50)
+        return min(t)
+
+    broad = best_us((z * 2).to(torch.bfloat16))
+    for spread in (0.3, 0.05):
+        flat = best_us((z * spread).to(torch.bfloat16))
+        assert flat < 2.5 * broad, (spread, flat, broad)
