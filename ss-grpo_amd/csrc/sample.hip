@@ -277,6 +277,7 @@ struct SampleParams {
   int greedy;
   int top_k;      // 0 = off
   uint32_t tp32;  // 0 = off
+  bool cut() const { return !greedy && (top_k > 0 || tp32 != 0); }
 };
 
 // One draw from one row by the whole block. Returns the token (all threads).
@@ -837,10 +838,12 @@ FG_DEVICE bool narrow_cut(const char* p, int V, float m, float kt, const uint64_
 // barriers. Against the launches it replaces (three for an unrestricted draw, seven for top-p),
 // a draw of 8 x 32,000 bf16 rows took, us: unrestricted 16.6 -> 10.9, top-p 48.8 -> 31.1, top-k 50
 // 49.0 -> 15.7; of 512 rows 43.2 -> 19.9, 220.7 -> 63.4, 102.0 -> 32.0.
-template <bool CUTS>
+enum Cut : int { kNoCut, kTopP, kTopK };  // kTopK: with a top-p cut after it or not
+
+template <int CUT>
 struct ResidentShared {
-  uint64_t hist[CUTS ? kSelBins : 1][kCopies];
-  uint64_t ck[CUTS ? kSelList : 1];
+  uint64_t hist[CUT ? kSelBins : 1][kCopies];
+  uint64_t ck[CUT ? kSelList : 1];
   uint64_t wsum[kWaves * 8];   // [group][wave]
   SelectShared sel;
   SmallShared small;
@@ -849,9 +852,10 @@ struct ResidentShared {
   int bin, n, nan, tok;
 };
 
-template <int DT, int G, bool CUTS>
+template <int DT, int G, int CUT>
 FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, uint32_t u, Shared& sh,
-                              ResidentShared<CUTS>& rs) {
+                              ResidentShared<CUT>& rs) {
+  constexpr bool CUTS = CUT != kNoCut, count = CUT == kTopK;
   static_assert(G * kWaves <= kWaves * 8, "group sums");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const auto load_group = [&](int g, float(&v)[8]) {
@@ -873,29 +877,8 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
 #pragma unroll
     for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(x[g][j]));
   };
-  if (!CUTS && sp.greedy) {  // first maximum: value desc (NaN first), index asc
-    uint64_t best = 0;
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      fresh(g);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int i = (g * kThreads + tid) * 8 + j;
-        const uint64_t k = i < V ? fg::rank_key(x[g][j], (uint32_t)i) : 0ull;
-        best = k > best ? k : best;
-      }
-    }
-    best = fg::wave_max_u64(best);
-    if (lane == 0) sh.wkey[wave] = best;
-    __syncthreads();
-    best = 0;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) best = sh.wkey[w] > best ? sh.wkey[w] : best;
-    return (int)fg::rank_key_index(best);
-  }
   fg::exp2_table_to_lds(sh.exp2);
   const float kt = fg::weight_kt(sp.temperature > 0.0f && sp.temperature != 1.0f, sp.temperature);
-  const bool count = CUTS && sp.top_k > 0;
   if constexpr (CUTS) {
     for (int i = tid; i < kCopies * kSelBins; i += kThreads) (&rs.hist[0][0])[i] = 0;
     if (tid == 0) {
@@ -1037,7 +1020,7 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
       __syncthreads();
       return block_sample<DT>(rowp, V, sp, u, sh);
     }
-    if (count) {
+    if constexpr (count) {
       const int tok = list_draw(rs.ck, n, (int64_t)sp.top_k - rs.nan, sp.tp32, u, m, kt, sh.exp2, rs.sel, rs.small);
       __syncthreads();
       return tok;
@@ -1126,19 +1109,11 @@ FG_DEVICE int resident_sample(const void* rowp, int V, const SampleParams& sp, u
   return rs.tok;
 }
 
-// Groups of 8,192 logits a workgroup holds for a row of V: 0 when the row is too long.
-// One workgroup weighs 32,768 logits in about the time of a launch; twice as many still beat the
-// split launches without a cut (64 x 65,536 bf16: 14.3 against 17.1 us), but not with one, where
-// the weighing passes are two (64 x 65,536, top-p: 59.7 against 44.5 us split).
-constexpr int resident_groups(int vocab, bool cuts) {
-  return vocab <= 8192 * 4 ? 4 : vocab <= 8192 * 8 && !cuts ? 8 : 0;
-}
-
-template <int DT, int G, bool CUTS>
+template <int DT, int G, int CUT>
 FG_DEVICE int row_sample(const void* rowp, int V, const SampleParams& sp, uint32_t u, Shared& sh) {
   if constexpr (G > 0) {
-    __shared__ ResidentShared<CUTS> rs;
-    return resident_sample<DT, G, CUTS>(rowp, V, sp, u, sh, rs);
+    __shared__ ResidentShared<CUT> rs;
+    return resident_sample<DT, G, CUT>(rowp, V, sp, u, sh, rs);
   } else {
     return block_sample<DT>(rowp, V, sp, u, sh);
   }
@@ -1150,7 +1125,7 @@ FG_DEVICE uint32_t noise_value(const uint32_t* noise, int64_t noise_index, uint6
   return fg::counter_noise(seed, step, seq, draw);
 }
 
-template <int DT, int G, bool CUTS>
+template <int DT, int G, int CUT>
 __global__ void __launch_bounds__(kThreads) sample_rows_kernel(
     const void* __restrict__ logits, int64_t row_stride, int vocab, const int32_t* __restrict__ row_index,
     const int32_t* __restrict__ forced, const uint32_t* __restrict__ noise, int noise_stride, int noise_col,
@@ -1166,7 +1141,7 @@ __global__ void __launch_bounds__(kThreads) sample_rows_kernel(
   const char* rowp = (const char*)logits + (int64_t)src * row_stride * (DT == fg::kBF16 ? 2 : 4);
   uint32_t seq = seq_ids ? (uint32_t)seq_ids[rrow] : (uint32_t)rrow;
   uint32_t u = noise_value(noise, (int64_t)rrow * noise_stride + noise_col, seed, step, seq, (uint32_t)draw);
-  int tok = row_sample<DT, G, CUTS>(rowp, vocab, sp, u, sh);
+  int tok = row_sample<DT, G, CUT>(rowp, vocab, sp, u, sh);
   if (threadIdx.x == 0) out[rrow] = tok;
 }
 
@@ -1249,7 +1224,7 @@ FG_DEVICE void walk_apply(int b, int tok, int parent, const int32_t* tree_tokens
   }
 }
 
-template <int DT, int G, bool CUTS>
+template <int DT, int G, int CUT>
 __global__ void __launch_bounds__(kThreads) walk_step_kernel(
     const void* __restrict__ logits, int64_t row_stride, int vocab, const int32_t* __restrict__ slot_map,
     const int32_t* __restrict__ tree_tokens, const int32_t* __restrict__ parents, const int32_t* __restrict__ n_nodes,
@@ -1276,7 +1251,7 @@ __global__ void __launch_bounds__(kThreads) walk_step_kernel(
   uint32_t seq = seq_ids ? (uint32_t)seq_ids[b] : (uint32_t)b;
   uint32_t u = noise_value(noise, (int64_t)b * noise_stride + noise_col0 + walk_step, seed, step, seq,
                            (uint32_t)(draw0 + walk_step));
-  int tok = row_sample<DT, G, CUTS>(rowp, vocab, sp, u, sh);
+  int tok = row_sample<DT, G, CUT>(rowp, vocab, sp, u, sh);
   if (threadIdx.x < 64)
     walk_apply(b, tok, parent, tree_tokens, parents, n_nodes, nmax, batch, walk_step, acc_tokens, acc_nodes, acc_stride,
                acc_len, last_node, correction, state, err_flag, next_rows, next_active);
@@ -2292,7 +2267,7 @@ int scratch_for_current_device(void** out) {
 // draws need more than the others).
 bool split_setup(SplitArgs& a, void* workspace, size_t bytes, int rows, const void* logits, int64_t row_stride,
                  int vocab, float temperature, const SampleParams& sp) {
-  const bool cut = !sp.greedy && (sp.top_k > 0 || sp.tp32 != 0);
+  const bool cut = sp.cut();
   if (sp.top_k > kSelTopK && cut) return false;
   if (!workspace || bytes < (cut ? split_workspace_bytes(rows) : split_base_bytes(rows))) return false;
   char* w = (char*)(((uintptr_t)workspace + 15) & ~(uintptr_t)15);
@@ -2369,22 +2344,48 @@ SampleParams make_params(float temperature, int greedy, int top_k, int vocab, ui
   return sp;
 }
 
-// f(dtype, resident groups, whether the draw has a cut), each an integral constant, for the
-// one-workgroup-per-row kernels on rows of `vocab` logits.
+// Where a draw runs, the one rule: in one workgroup per row that holds `groups` x 8,192 logits in registers
+// (resident_sample), else over the split launches, which need the workspace, else in block_sample. `maxima`:
+// the row maxima parts are given. us on bf16 rows at each line:
+//  * greedy draws read each logit once and weigh none. Given maxima make them one launch that reads no logit
+//    (64 x 32,000: 2.5, resident 7.5). Otherwise split from 8,193 logits (8 x 32,000: 6.3, resident 8.1, block 8.7;
+//    64 x 512: split 7.0, block 5.2), up to 32,768 of them for at most 128 rows (256 x 32,000: 10.9 and 9.0).
+//  * a top_k over kSelTopK overfills the list: block_sample alone (8 x 32,000, top_k 5,000: 55, 70 after a
+//    resident histogram).
+//  * up to 8,192 logits one group, up to 16,384 two, up to 32,768 four: the padding is weighed too (64 x 512: one
+//    group 6.3, four 9.8, block_sample 7.6; top-p 11.4 and 16.1).
+//  * up to 65,536 without a cut eight from kLongRows rows on, or from kLongRowsMaxima with given maxima, when the
+//    split draw is two launches (65,536: 8 rows split 13.9 and resident 14.1, 64 rows 17.0 and 14.6, 512 59 and
+//    34; with maxima 64 rows 11.3 and 14.0, 256 25.8 and 16.5). With a cut the weighing passes are two and the
+//    split launches win (64 x 65,536, top-p: 59.7 and 41.6).
+struct DrawPath {
+  int groups;
+  bool split;
+};
+constexpr int kLongRows = 16, kLongRowsMaxima = 128;
+DrawPath draw_path(int vocab, const SampleParams& sp, int rows, bool workspace, bool maxima) {
+  if (sp.greedy) return {0, workspace && (maxima || vocab > 8192 * 4 || (vocab > 8192 && rows <= 128))};
+  if (sp.top_k > kSelTopK) return {0, false};
+  if (vocab <= 8192 * 4) return {vocab <= 8192 ? 1 : vocab <= 8192 * 2 ? 2 : 4, false};
+  const bool whole = vocab <= 8192 * 8 && !sp.cut() && (!workspace || rows >= (maxima ? kLongRowsMaxima : kLongRows));
+  return {whole ? 8 : 0, workspace && !whole};
+}
+
+// f(dtype, groups, Cut), each an integral constant, for the one-workgroup-per-row kernels.
 template <class F>
-void for_row_kernel(int dtype, int vocab, const SampleParams& sp, F&& f) {
-  const bool cuts = !sp.greedy && (sp.top_k || sp.tp32);
-  const auto groups = [&](auto dt, auto g) {
-    if constexpr (decltype(g)::value == 4) {
-      if (cuts) return f(dt, g, std::true_type{});
-    }
-    f(dt, g, std::false_type{});
-  };
+void for_row_kernel(int dtype, int path_groups, const SampleParams& sp, F&& f) {
   const auto types = [&](auto dt) {
-    switch (resident_groups(vocab, cuts)) {
-      case 4: groups(dt, std::integral_constant<int, 4>{}); break;
-      case 8: groups(dt, std::integral_constant<int, 8>{}); break;
-      default: f(dt, std::integral_constant<int, 0>{}, std::false_type{}); break;
+    const auto cuts = [&](auto g) {
+      if (!sp.cut()) f(dt, g, std::integral_constant<int, kNoCut>{});
+      else if (sp.top_k) f(dt, g, std::integral_constant<int, kTopK>{});
+      else f(dt, g, std::integral_constant<int, kTopP>{});
+    };
+    switch (path_groups) {
+      case 1: cuts(std::integral_constant<int, 1>{}); break;
+      case 2: cuts(std::integral_constant<int, 2>{}); break;
+      case 4: cuts(std::integral_constant<int, 4>{}); break;
+      case 8: f(dt, std::integral_constant<int, 8>{}, std::integral_constant<int, kNoCut>{}); break;
+      default: f(dt, std::integral_constant<int, 0>{}, std::integral_constant<int, kNoCut>{}); break;
     }
   };
   if (dtype == fg::kBF16) types(std::integral_constant<int, fg::kBF16>{});
@@ -2405,20 +2406,21 @@ int sample_tokens_impl(const char* who, const void* logits, int dtype, int64_t r
   SampleParams sp = make_params(temperature, greedy, top_k, vocab, top_p_fixed);
   hipStream_t s = (hipStream_t)stream;
   SplitArgs a;
-  if (!resident_groups(vocab, !sp.greedy && (sp.top_k || sp.tp32)) &&
-      split_setup(a, workspace, workspace_bytes, rows, logits, row_stride, vocab, temperature, sp)) {
+  const bool scratch = split_setup(a, workspace, workspace_bytes, rows, logits, row_stride, vocab, temperature, sp);
+  const DrawPath path = draw_path(vocab, sp, rows, scratch, false);
+  if (path.split) {
     a.row_index = row_index;
     a.forced = forced;
     DrawOut d{};
     d.noise = noise; d.noise_stride = noise_stride; d.noise_col = noise_col;
     d.seed = seed; d.step = step; d.seq_ids = seq_ids; d.draw = draw; d.out = out_tokens;
-    if (!sp.greedy && (sp.top_k || sp.tp32)) split_select<false>(dtype, a, d, sp, rows, true, s);
+    if (sp.cut()) split_select<false>(dtype, a, d, sp, rows, true, s);
     else if (dtype == fg::kBF16) split_draw<fg::kBF16, false>(a, d, rows, true, s);
     else split_draw<fg::kF32, false>(a, d, rows, true, s);
     return fg::check_launch(who);
   }
-  for_row_kernel(dtype, vocab, sp, [&](auto dt, auto g, auto cuts) {
-    hipLaunchKernelGGL((sample_rows_kernel<decltype(dt)::value, decltype(g)::value, decltype(cuts)::value>), dim3(rows), dim3(kThreads), 0, s,
+  for_row_kernel(dtype, path.groups, sp, [&](auto dt, auto g, auto cut) {
+    hipLaunchKernelGGL((sample_rows_kernel<decltype(dt)::value, decltype(g)::value, decltype(cut)::value>), dim3(rows), dim3(kThreads), 0, s,
                        logits, row_stride, vocab, row_index, forced, noise, noise_stride, noise_col, seed, step,
                        seq_ids, draw, sp, out_tokens);
   });
@@ -2477,8 +2479,8 @@ int fg_accept_walk(const void* tree_logits, int dtype, int64_t row_stride, int v
   hipLaunchKernelGGL(walk_init_kernel, dim3((batch + 63) / 64), dim3(64), 0, s, tree_tokens, parents, n_nodes, nmax,
                      batch, acc_tokens, acc_nodes, acc_stride, acc_len, last_node, correction, workspace);
   for (int t = 0; t < max_walk_steps; ++t) {
-    for_row_kernel(dtype, vocab, sp, [&](auto dt, auto g, auto cuts) {
-      hipLaunchKernelGGL((walk_step_kernel<decltype(dt)::value, decltype(g)::value, decltype(cuts)::value>), dim3(batch), dim3(kThreads), 0, s,
+    for_row_kernel(dtype, draw_path(vocab, sp, batch, false, false).groups, sp, [&](auto dt, auto g, auto cut) {
+      hipLaunchKernelGGL((walk_step_kernel<decltype(dt)::value, decltype(g)::value, decltype(cut)::value>), dim3(batch), dim3(kThreads), 0, s,
                          tree_logits, row_stride, vocab, slot_map, tree_tokens, parents, n_nodes, nmax, batch, t, 0,
                          noise, noise_stride, noise_col0, seed, step, seq_ids, draw0, sp, acc_tokens, acc_nodes,
                          acc_stride, acc_len, last_node, correction, workspace, err_flag, nullptr, nullptr);
@@ -2528,10 +2530,10 @@ int fg_walk_step(const void* step_logits, int dtype, int64_t row_stride, int voc
   SampleParams sp = make_params(temperature, greedy, top_k, vocab, top_p_fixed);
   hipStream_t s = (hipStream_t)stream;
   SplitArgs a;
-  if (!resident_groups(vocab, !sp.greedy && (sp.top_k || sp.tp32)) &&
-      split_setup(a, workspace, workspace_bytes, batch, step_logits, row_stride, vocab, temperature, sp)) {
+  const bool scratch = split_setup(a, workspace, workspace_bytes, batch, step_logits, row_stride, vocab, temperature, sp);
+  const DrawPath path = draw_path(vocab, sp, batch, scratch, part_max != nullptr);
+  if (path.split) {
     a.active = state + batch;
-    const bool cut = !sp.greedy && (sp.top_k || sp.tp32);
     const bool with_max = part_max == nullptr;
     if (!with_max) {
       a.src_max = part_max;
@@ -2547,13 +2549,13 @@ int fg_walk_step(const void* step_logits, int dtype, int64_t row_stride, int voc
     d.acc_tokens = acc_tokens; d.acc_nodes = acc_nodes; d.acc_stride = acc_stride; d.acc_len = acc_len;
     d.last_node = last_node; d.correction = correction; d.state = state; d.err_flag = err_flag;
     d.next_rows = next_row_index; d.next_active = next_row_active;
-    if (cut) split_select<true>(dtype, a, d, sp, batch, with_max, s);
+    if (sp.cut()) split_select<true>(dtype, a, d, sp, batch, with_max, s);
     else if (dtype == fg::kBF16) split_draw<fg::kBF16, true>(a, d, batch, with_max, s);
     else split_draw<fg::kF32, true>(a, d, batch, with_max, s);
     return fg::check_launch("fg_walk_step");
   }
-  for_row_kernel(dtype, vocab, sp, [&](auto dt, auto g, auto cuts) {
-    hipLaunchKernelGGL((walk_step_kernel<decltype(dt)::value, decltype(g)::value, decltype(cuts)::value>), dim3(batch), dim3(kThreads), 0, s,
+  for_row_kernel(dtype, path.groups, sp, [&](auto dt, auto g, auto cut) {
+    hipLaunchKernelGGL((walk_step_kernel<decltype(dt)::value, decltype(g)::value, decltype(cut)::value>), dim3(batch), dim3(kThreads), 0, s,
                        step_logits, row_stride, vocab, nullptr, tree_tokens, parents, n_nodes, nmax, batch, walk_step, 1,
                        noise, noise_stride, noise_col0, seed, step, seq_ids, draw0, sp, acc_tokens, acc_nodes,
                        acc_stride, acc_len, last_node, correction, state, err_flag, next_row_index, next_row_active);

@@ -156,6 +156,43 @@ def test_chunks_of_two_passes_match_oracle(dtype, V):
         assert np.array_equal(got, _oracle(x.float().numpy(), noise, kw)), (V, dtype, kw)
 
 
+@pytest.mark.parametrize("rows", [3, 15, 16, 130])
+@pytest.mark.parametrize("V", [8192, 8200, 16384, 16392, 32768, 32776, 65536, 65544])
+def test_draws_at_the_path_lines(V, rows):
+    """Every kind of draw on both sides of the sizes and row counts at which its path changes."""
+    from flashgrpo_amd import kernels as K
+
+    base = _rows(V, V)[[0, 1, 3, 6, 9]]
+    x = base[torch.arange(rows) % 5].to(torch.bfloat16)
+    n5 = np.random.default_rng(4).integers(0, 2 ** 32, (5, 1), dtype=np.uint32)
+    noise = n5[np.arange(rows) % 5]
+    nd = torch.from_numpy(noise.view(np.int32)).to(DEV)
+    xd, xs = x.to(DEV), base.to(torch.bfloat16).float().numpy()
+    for kw in (dict(), dict(temperature=0.6), dict(greedy=True), dict(top_p=0.9), dict(top_k=20)):
+        want = _oracle(xs, n5, kw)[np.arange(rows) % 5]
+        for split in (True, False):
+            got = K.sample_tokens(xd, noise=nd, split=split, **kw).cpu().numpy()
+            assert np.array_equal(got, want), (V, rows, kw, split)
+
+
+@pytest.mark.parametrize("V", [64, 8192, 32000, 65536, 70000])
+def test_greedy_walk_step_with_given_maxima_reads_no_logits(V):
+    """The first maxima that come with the logits are the greedy draw: the logits are not read again."""
+    from flashgrpo_amd import kernels as K
+
+    B = 6
+    tt = torch.full((B, 2), -5, dtype=torch.int32, device=DEV)
+    par = torch.tensor([[-1, 0]] * B, dtype=torch.int32, device=DEV)
+    nn = torch.full((B,), 2, dtype=torch.int32, device=DEV)
+    first = torch.arange(B, device=DEV) * 9 + 1
+    key = (torch.full((B,), 0xC0000000, dtype=torch.int64, device=DEV) << 32) | (0xffffffff - first)  # the value 2.0
+    parts = (torch.full((B, 1), 2.0, device=DEV), key[:, None].contiguous())
+    wk = K.walk_begin(tt, par, nn, acc_stride=2)
+    K.walk_rows(wk, 2)
+    K.walk_step(wk, torch.zeros(B, V, device=DEV), tt, par, nn, walk_step=0, greedy=True, parts=parts)
+    assert torch.equal(wk["correction"].long(), first)
+
+
 @pytest.mark.parametrize("kw", [dict(top_p=0.9), dict(top_k=1000)])
 def test_flat_rows_take_no_more_than_others(kw):
     """A flat row costs about what any other does: it once went to a draw of many passes by one
