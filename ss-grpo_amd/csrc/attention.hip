@@ -64,6 +64,8 @@ struct AttnArgs {
   int batch;
   float* o_part;
   float2* ml_part;
+  int group;           // units whose row tiles are dispatched side by side (a multiple of 8, or all)
+  bool longest_first;  // a unit's row tiles last to first
 };
 
 constexpr int kD = 128;            // head dim of the MFMA path
@@ -141,22 +143,18 @@ __global__ void __launch_bounds__(W * 64, 2) tree_attn_bf16_kernel(AttnArgs a, i
   constexpr int kRowsTile = rows_tile(W);
 
   // A unit is one (sequence, kv head, key part); its m_tiles row tiles read the same
-  // K/V tiles. Blocks are dispatched round-robin over the 8 XCDs, so the row tiles
-  // of a unit are placed 8 blocks apart: one XCD, dispatched together, the second
-  // read of each K/V tile served from that XCD's L2.
+  // K/V tiles. Blocks are dispatched round-robin over the 8 XCDs, so the row tiles of a
+  // unit are placed a.group blocks apart (a multiple of 8): one XCD, dispatched together,
+  // the second read of each K/V tile served from that XCD's L2 (chain_group).
   int unit = blockIdx.x, mt = 0;
   if (m_tiles > 1) {
     const int units8 = gridDim.x / m_tiles;  // units padded to whole groups of 8
-    if (a.anc) {
-      const int grp = blockIdx.x / (8 * m_tiles), rem = blockIdx.x % (8 * m_tiles);
-      mt = rem / 8;
-      unit = grp * 8 + rem % 8;
-    } else {
-      // A chain's later row tiles see more keys: they start first, so the last workgroups to
-      // finish are the short ones. A unit's tiles still meet on one XCD (units8 % 8 == 0).
-      mt = m_tiles - 1 - (int)blockIdx.x / units8;
-      unit = blockIdx.x % units8;
-    }
+    const int gs = min(a.group, units8);
+    const int g0 = (int)blockIdx.x / (gs * m_tiles) * gs, group = min(gs, units8 - g0);
+    const int rem = (int)blockIdx.x - g0 * m_tiles;
+    mt = rem / group;
+    if (a.longest_first) mt = m_tiles - 1 - mt;
+    unit = g0 + rem % group;
     if (unit >= a.batch * a.Hkv * a.splits) return;
   }
   const int sp = unit % a.splits;
@@ -572,10 +570,23 @@ size_t attn_workspace_bytes(int splits, int batch, int num_nodes, int q_heads) {
   return rows * (kD * sizeof(float) + sizeof(float2)) + 256;
 }
 
+// Units of a chain whose row tiles are dispatched side by side. The later tiles see more keys and
+// start first, so that the last workgroups to finish are short ones: over all units where there are
+// few (4 x 1024 after 1000, 32 units: 8 at a time 125.7 us, all 111.5), else over as many as an XCD's
+// 4 MB L2 keeps the K/V of, by the capacity, at most 4 per XCD (28 / 4 heads, 64 x 128 after 4096, 256 units:
+// 8 at a time 454 us, all 499; 32 / 8 heads, 64 x 256 alone: 8 at a time 162, 32 127, all 157).
+int chain_group(int units, int capacity) {
+  if (units < 64) return 1 << 20;
+  const int64_t unit_bytes = (int64_t)capacity * kD * 2 * 2;
+  return 8 * (int)std::max<int64_t>(1, std::min<int64_t>(4, (4 << 20) / unit_bytes));
+}
+
 template <int W>
-void launch_attn_bf16(const AttnArgs& a, int M, hipStream_t s) {
+void launch_attn_bf16(AttnArgs a, int M, hipStream_t s) {
   const int m_tiles = (M + rows_tile(W) - 1) / rows_tile(W);
   const int units = a.batch * a.Hkv * a.splits;
+  a.group = a.anc ? 8 : chain_group(units, a.capacity);
+  a.longest_first = !a.anc;
   const int blocks = m_tiles > 1 ? (units + 7) / 8 * 8 * m_tiles : units;
   hipLaunchKernelGGL(tree_attn_bf16_kernel<W>, dim3(blocks), dim3(W * 64), 0, s, a, m_tiles);
 }

@@ -75,3 +75,23 @@ def test_fp32_key_groups(d, prefix, chain):
     # fp32 scores of d terms and sums of at most 265 keys, each rounded to 2^-24
     err = (got.double() - want).abs().amax(-1) / want.abs().amax(-1)
     assert float(err.max()) < (d + 265) * 2.0 ** -24, float(err.max())
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,N,cap", [(9, 16, 8, 129, 700),      # 72 units: groups of 32, 32 and 8
+                                            (9, 16, 8, 129, 2400),     # groups of 24
+                                            (9, 8, 8, 300, 9000),      # groups of 8
+                                            (63, 2, 1, 200, 500),      # 63 units: one group
+                                            (65, 2, 1, 200, 500)])     # 65 units padded to 72
+def test_chain_tile_orders(B, Hq, Hkv, N, cap):
+    """Every row tile of every (sequence, kv head) is computed once, however they are grouped."""
+    from flashgrpo_amd import kernels as K
+
+    g = torch.Generator(device=DEV).manual_seed(cap)
+    d = 128
+    seq = torch.tensor([(41 * b) % 190 for b in range(B)], dtype=torch.int32, device=DEV)
+    q = torch.randn(B, N, Hq, d, device=DEV, generator=g).bfloat16()
+    k = torch.randn(B, Hkv, cap, d, device=DEV, generator=g, dtype=torch.bfloat16)
+    v = torch.randn(B, Hkv, cap, d, device=DEV, generator=g, dtype=torch.bfloat16)
+    got = K.tree_attention(q, k, v, seq_len=seq, anc=None, num_nodes=N, q_heads=Hq, kv_heads=Hkv, head_dim=d,
+                           out=torch.full_like(q, float("nan")))
+    _close(got, _want(q, k, v, seq, torch.tril(torch.ones(N, N, dtype=torch.bool, device=DEV))))
