@@ -53,6 +53,33 @@ constexpr int dist_for(int mi) { return mi >= 8 ? 2 : 3; }
 // asm-issued weight loads), so every row count runs 8 waves.
 constexpr int waves_for(int) { return 8; }
 
+// Whether a block round of kst k-steps has to end in a barrier. Its loop runs whole groups of `dist`
+// steps; the barrier of a step tells that every wave has read the steps before it, so after the loop only
+// the last step's stage may still be in use, if it is one that reads (a step past kst reads nothing), and
+// the next round refills stages 0 .. dist - 1 of dist + 1. Of the row counts up to 64 (dist 3) the
+// weights of 1,536, 3,584, 4,096 and 5,120 columns need none (a walk of four steps over 64 rows of 152,064 x
+// 3,584: 951.7 us with a barrier each round, 946.6 without).
+constexpr bool round_needs_barrier(int kst, int dist) {
+  const int steps = (kst + dist - 1) / dist * dist, last = steps - 1;
+  return last < kst && last % (dist + 1) != dist;
+}
+// The same by following the stages step by step.
+constexpr bool round_leaves_stage_in_use(int kst, int dist) {
+  int in_use = -1;  // stage that a wave behind the others may still read
+  for (int k0 = 0; k0 < kst; k0 += dist)
+    for (int s = k0; s < k0 + dist; ++s) in_use = s < kst ? s % (dist + 1) : -1;  // the step's barrier frees the last
+  for (int h = 0; h < dist; ++h)
+    if (h % (dist + 1) == in_use) return true;
+  return false;
+}
+constexpr bool rounds_agree() {
+  for (int dist = 2; dist <= 3; ++dist)
+    for (int kst = 1; kst <= 512; ++kst)
+      if (round_needs_barrier(kst, dist) != round_leaves_stage_in_use(kst, dist)) return false;
+  return true;
+}
+static_assert(rounds_agree(), "stage reuse between block rounds");
+
 template <int N>
 FG_DEVICE void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt");
@@ -205,6 +232,7 @@ __global__ void __launch_bounds__(W * 64, 1) lm_stream_kernel(LmArgs a) {
     pm_key[i] = 0;
   }
 
+  bool reused = false;  // the last round's last stage may be in use; the same in every wave
   for (int rd = 0; rd < rounds; ++rd) {
     // Every wave issues the same loads every k-step, so the waits below are static: a wave
     // without a block this round, and the k-steps past the last, re-read one cached line.
@@ -243,11 +271,12 @@ __global__ void __launch_bounds__(W * 64, 1) lm_stream_kernel(LmArgs a) {
 
     if constexpr (KT == 0) {
       // every wave is done with the last round's stages (with top-k its epilogue ends in a barrier)
-      if (rd > 0) {
+      if (reused) {
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
       }
+      reused = round_needs_barrier(kst, kDist);
     }
 #pragma unroll
     for (int h = 0; h < kDist; ++h) {
