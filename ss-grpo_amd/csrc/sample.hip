@@ -1334,7 +1334,7 @@ constexpr int kSplitMaxGroups = 16;
 FG_DEVICE bool split_group_live(int base, int u, int hi) { return base + u * kSplitThreads * 8 < hi; }
 
 // Chunk maxima (raw maximum, NaN ignored, with KEY the first-maximum rank key, without it the least
-// logit of the whole groups of 8 in its place: bin_shift's range, which need not be exact). Per pass a thread
+// logit of each pass's first load group beside it, which bounds bin_shift's range). Per pass a thread
 // takes the maximum of its elements (NaN ignored) and then the first index holding it (the
 // first NaN when there is one, which ranks highest), and forms one rank key per pass instead
 // of one per element.
@@ -1365,9 +1365,9 @@ __global__ void __launch_bounds__(kSplitThreads) split_max_kernel(SplitArgs a) {
       for (int j = 0; j < 8; ++j) {
         pm = fmaxf(pm, x[u][j]);
         if constexpr (KEY) nan |= x[u][j] != x[u][j];
-        else low8 = fminf(low8, x[u][j]);
+        else if (u == 0) low8 = fminf(low8, x[u][j]);
       }
-      if (!KEY && base + (u * kSplitThreads + (int)threadIdx.x) * 8 + 8 <= hi) low = fminf(low, low8);
+      if (!KEY && u == 0 && base + (int)threadIdx.x * 8 + 8 <= hi) low = fminf(low, low8);
     }
     if constexpr (!KEY) {
       mx = fmaxf(mx, pm);
@@ -1405,8 +1405,13 @@ __global__ void __launch_bounds__(kSplitThreads) split_max_kernel(SplitArgs a) {
       if constexpr (KEY) best = skey[w] > best ? skey[w] : best;
       else best = __float_as_uint(fminf(__uint_as_float((uint32_t)best), __uint_as_float((uint32_t)skey[w])));
     }
-    a.part_max[r * kSplitChunks + c] = fmaxf(smax[0], mx);
-    a.part_key[r * kSplitChunks + c] = KEY && skey[0] > best ? skey[0] : best;
+    mx = fmaxf(smax[0], mx);
+    if constexpr (KEY) {
+      a.part_max[r * kSplitChunks + c] = mx;
+      a.part_key[r * kSplitChunks + c] = skey[0] > best ? skey[0] : best;
+    } else {
+      a.part_key[r * kSplitChunks + c] = (uint64_t)__float_as_uint(mx) << 32 | (uint32_t)best;
+    }
   }
 }
 
@@ -1638,7 +1643,7 @@ struct SelState {
   int32_t slow;   // the row has no weight, or NaN takes every slot: block_sample draws it
   int32_t all;    // every listed element is kept (top-k with no more candidates than slots)
   int32_t bin;    // the cut's bin
-  int32_t crowded;  // part_gsum holds each chunk's least and largest listed key and their count
+  int32_t form;   // bin_shift << 1 | whether part_gsum holds each chunk's least and largest listed key and their count
 };
 
 template <int DT, bool COUNT>
@@ -1649,7 +1654,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) 
   using AtomicBin = std::conditional_t<COUNT, unsigned int, unsigned long long>;
   __shared__ uint64_t tbl[COUNT ? 1 : 1024];
   __shared__ Bin h[kSelBins][kCopies];
-  __shared__ float smax[kSplitWaves], smin[kSplitWaves];
+  __shared__ float smax[kSplitWaves];
   __shared__ int s_nan;
   const char* p = split_row<DT>(a, r);
   const int lo = c * a.chunk, hi = min(a.vocab, lo + a.chunk);
@@ -1661,31 +1666,32 @@ __global__ void __launch_bounds__(kSplitThreads) split_hist_kernel(SplitArgs a) 
 #pragma unroll
   for (int q = 0; q < kCopies; ++q) (&h[0][0])[q * kSplitThreads + tid] = 0;
   if (tid == 0) s_nan = 0;
-  const bool ranged = a.src_max == a.part_max;  // given maxima come without the least logit
-  float mx = -INFINITY, low = INFINITY;         // row maximum and least logit from the parts
-  for (int q = tid; q < a.src_parts; q += kSplitThreads) {
-    mx = fmaxf(mx, a.src_max[r * a.src_stride + q]);
-    if (ranged) low = fminf(low, __uint_as_float((uint32_t)a.src_key[r * a.src_stride + q]));
-  }
+  // row maximum and least logit: this path's own parts hold both, given maxima come without the least
+  static_assert(kSplitChunks == 16, "a part per lane of 16");
+  float m;
+  int shift = kSelBinShift;
+  const float kt = split_kt(a);
+  if (a.src_max == a.part_max) {
+    const uint64_t both = a.part_key[r * kSplitChunks + (tid & (kSplitChunks - 1))];
+    m = __uint_as_float((uint32_t)(both >> 32));
+    float low = __uint_as_float((uint32_t)both);
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    low = fminf(low, __shfl_xor(low, o, 64));
-  }
-  if ((tid & 63) == 0) {
-    smax[tid >> 6] = mx;
-    smin[tid >> 6] = low;
-  }
-  __syncthreads();
-  mx = smax[0];
-  low = smin[0];
+    for (int o = kSplitChunks / 2; o > 0; o >>= 1) {
+      m = fmaxf(m, __shfl_xor(m, o, 64));
+      low = fminf(low, __shfl_xor(low, o, 64));
+    }
+    shift = __builtin_amdgcn_readfirstlane(bin_shift(m, low, kt));
+    __syncthreads();
+  } else {
+    m = -INFINITY;
+    for (int q = tid; q < a.src_parts; q += kSplitThreads) m = fmaxf(m, a.src_max[r * a.src_stride + q]);
+    m = fg::wave_max(m);
+    if ((tid & 63) == 0) smax[tid >> 6] = m;
+    __syncthreads();
+    m = smax[0];
 #pragma unroll
-  for (int w = 1; w < kSplitWaves; ++w) {
-    mx = fmaxf(mx, smax[w]);
-    low = fminf(low, smin[w]);
+    for (int w = 1; w < kSplitWaves; ++w) m = fmaxf(m, smax[w]);
   }
-  const float m = mx, kt = split_kt(a);
-  const int shift = ranged ? bin_shift(m, low, kt) : kSelBinShift;
   Bin* mine = &h[0][tid % kCopies];
   int nan = 0;
   for (int base = lo; base < hi; base += kSplitPass) {
@@ -1757,6 +1763,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_gather_kernel(SplitArgs a
 #pragma unroll
   for (int u = 0; u < kSplitLoads; ++u)
     if (split_group_live(lo, u, hi)) split_load8<DT>(p, lo + (u * kSplitThreads + tid) * 8, hi, x[u]);
+  const int shift = (int)a.row_best[r];
   const uint64_t* hp = a.hist + (size_t)r * kSplitChunks * kSelBins;
   uint64_t v = 0, own = 0;
 #pragma unroll
@@ -1793,11 +1800,12 @@ __global__ void __launch_bounds__(kSplitThreads) split_gather_kernel(SplitArgs a
   }
   __syncthreads();
   const int bin = s_bin;
-  const RowCut rc = bin_cut(bin, (int)a.row_best[r], 0);
+  const RowCut rc = bin_cut(bin, shift, 0);
   // top-p: half a list or more in the bin, by its q-mass: is it one value?
-  const bool crowded = !COUNT && !slow && s_mass > (uint64_t)(kSelList / 2) * exponent_weight(rc.lo, fg::kExp2Table);
+  const bool crowded = !COUNT && !slow &&
+                       (float)s_mass > (float)(kSelList / 2) * __builtin_amdgcn_exp2f(40.0f - (float)rc.lo * 0x1p-20f);
   if (c == 0 && tid == 0)
-    a.sel[r] = SelState{slow ? 0 : COUNT ? target : target - s_before, slow, all, bin, crowded};
+    a.sel[r] = SelState{slow ? 0 : COUNT ? target : target - s_before, slow, all, bin, shift << 1 | (int)crowded};
   if (slow) return;
   if constexpr (!COUNT) {  // this chunk's q-mass above the cut's bin
     uint64_t above;
@@ -1912,7 +1920,7 @@ __global__ void __launch_bounds__(kThreads) split_select_kernel(SplitArgs a, Dra
     __syncthreads();
     if (ok) tok = list_draw(ck, listed, slots, sp.tp32, u, m, kt, sh.exp2, sel, small);
   } else if (ok) {
-    RowCut c = bin_cut(st.bin, (int)a.row_best[r], st.rest);
+    RowCut c = bin_cut(st.bin, st.form >> 1, st.rest);
     const auto kept_weight = [&](float x, int i) -> uint64_t {
       const uint32_t e = fixed_exponent(m, x, kt);
       return e < c.lo || (e < c.hi && fg::rank_key(x, (uint32_t)i) >= c.cut) ? exponent_weight(e, sh.exp2) : 0ull;
@@ -1920,7 +1928,7 @@ __global__ void __launch_bounds__(kThreads) split_select_kernel(SplitArgs a, Dra
     // a flat row whose bin holds one value is cut by index, from the chunks' counts of it
     uint32_t least = 0xffffffffu, most = 0;
     int ties = 0;  // lane l: chunk l's
-    if (flat && st.crowded) {
+    if (flat && (st.form & 1)) {
       if ((tid & 63) < kSplitChunks) {
         const uint64_t* info = a.part_gsum + ((size_t)r * kSplitChunks + (tid & 63)) * kSplitMaxGroups;
         ties = (int)info[1];
