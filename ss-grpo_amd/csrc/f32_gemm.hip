@@ -13,9 +13,10 @@
 // columns of one row.
 // Bound by the fp32 matrix rate (256 flop per clock and CU, 154 TFLOP/s in a loop of nothing else):
 // 45 KB of LDS leave three workgroups per CU, so a SIMD has three waves to fill its matrix core
-// from. 768 x 512 x 8192 in 67 us (96 TFLOP/s, the matrix cores busy 73% of a CU's time) and
-// 768 x 4096 x 512 with the cell's epilogue in 37 us; steps of 64 at two workgroups per CU took 79
-// and 52. Neither an order of the items that keeps 87% of the lines in an XCD's L2, nor two steps
+// from. In a loop of one launch 768 x 512 x 8192 takes 67 us (96 TFLOP/s, the matrix cores busy 73% of a
+// CU's time) and 768 x 4096 x 512 with the cell's epilogue 37 (steps of 64 at two workgroups per CU: 79 and
+// 52); in the proposal step, behind an LM head that has streamed 1 GB, 82.0 and 46.2 (79 and 70 TFLOP/s).
+// Neither an order of the items that keeps 87% of the lines in an XCD's L2, nor two steps
 // in flight, nor a start of K that differs between tiles moved it further. The fp32 Medusa block of
 // 96 x 4096 x 4096 with its norm and combine: 118 -> 54 us, of 4 heads 430 -> 186 (fmaf tiles before).
 #include "fg_f32.h"

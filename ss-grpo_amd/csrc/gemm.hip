@@ -754,7 +754,9 @@ void launch_f32_rows(const GemmArgs& g, hipStream_t s) {
   else hipLaunchKernelGGL((gemm_f32_rows_kernel<4, CDT>), grid, block, 0, s, g);
 }
 
-// Up to 64 rows without an epilogue, K a multiple of 128, 16-byte aligned rows.
+// Up to 64 rows, the four blocks of 16 whose sums a wave holds, without an epilogue, K a multiple of 128,
+// 16-byte aligned rows; other calls go to the fmaf tile. Against that tile, us: N = 32,000 by K = 512, 8 rows
+// 74.7 -> 14.7, 64 rows 78.9 -> 29.5 (65 rows on the tile: 103.8); K = 2,048, 64 rows 344.8 -> 89.7 (65: 421).
 bool f32_rows_ok(const GemmArgs& g, int epi, int batch) {
   return batch == 1 && epi == kEpiNone && g.M <= 64 && g.K % kF32Tile == 0 && g.lda % 4 == 0 && g.ldb % 4 == 0 &&
          ((uintptr_t)g.A & 15) == 0 && ((uintptr_t)g.B & 15) == 0;

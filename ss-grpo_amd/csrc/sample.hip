@@ -13,16 +13,15 @@
 //   order) whose inclusive q prefix exceeds target.
 // Integer sums make every result independent of reduction order.
 //
-// Rows of up to 65,536 logits are drawn in one launch by one workgroup per row that holds the
-// row in registers (resident_sample). Longer rows with a workspace run over several workgroups:
-// unrestricted and greedy draws split over 16 chunks per
-// row (chunk maxima, then one draw launch; a walk step whose row maxima come from
-// the LM head's epilogue is the draw launch alone, see "split sampling"), top-k and top-p
-// draws over four launches or two (see "split top-k / top-p"). Otherwise: one
-// 1024-thread workgroup per sampled row. The row is split into 16
-// contiguous wave segments; a wave walks its segment 512 elements (8 per lane,
-// 16-byte loads) per step. Top-k / top-p use an MSB-first 4 x 8-bit radix
-// select over the keys with count or q-weighted histograms in LDS.
+// draw_path chooses where a draw runs:
+//  * rows of up to 65,536 logits (32,768 with a cut), unless greedy: one launch of one workgroup per row
+//    that holds the row in registers (resident_sample);
+//  * longer rows with a workspace: over 16 chunks per row, unrestricted draws in three launches (two in a
+//    walk step whose row maxima come from the LM head's epilogue), greedy draws in two (one; see "split
+//    sampling"), top-k and top-p draws in four or two (see "split top-k / top-p");
+//  * otherwise (block_sample): one 1024-thread workgroup per row, the row split into 16 contiguous wave
+//    segments; a wave walks its segment 512 elements (8 per lane, 16-byte loads) per step. Top-k / top-p
+//    use an MSB-first 4 x 8-bit radix select over the keys with count or q-weighted histograms in LDS.
 #include <mutex>
 #include <type_traits>
 
@@ -397,7 +396,7 @@ FG_DEVICE uint64_t list_select(const uint64_t* ck, int n, uint64_t cut, uint64_t
     }
     __syncthreads();
 #pragma unroll 1
-  for (int i = tid; i < n; i += kThreads) {
+    for (int i = tid; i < n; i += kThreads) {
       const uint64_t k = ck[i], v = value(k);
       if (k >= cut && (v & fixed) == prefix) {
         const int d = (int)(v >> shift) & 255;
@@ -436,7 +435,7 @@ FG_DEVICE uint64_t list_select(const uint64_t* ck, int n, uint64_t cut, uint64_t
     fixed |= 255ull << shift;
     if (sh.cnt[sh.digit] == 1) {
 #pragma unroll 1
-  for (int i = tid; i < n; i += kThreads)
+      for (int i = tid; i < n; i += kThreads)
         if (ck[i] >= cut && (value(ck[i]) & fixed) == prefix) sh.found = value(ck[i]);
       __syncthreads();
       return sh.found;
@@ -718,62 +717,62 @@ FG_DEVICE bool narrow_cut(const char* p, int V, float m, float kt, const uint64_
       if (tid == 0) sh.n = 0;
       __syncthreads();
     } else {
-    for (int i = tid; i < kSelBins * kCopies; i += kThreads) hist[i] = 0;
-    if (tid == 0) {
-      sh.digit = -1;
-      sh.n = 0;
-      sh.nan = 0;
-    }
-    __syncthreads();
-    int nan = 0;
-    for_row8<DT>(p, V, [&](const float(&x)[8], int) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint32_t a = fixed_exponent(m, x[j], kt);
-        if constexpr (COUNT) nan += x[j] != x[j];
-        if (a - c.lo < width)
-          atomicAdd((unsigned long long*)&hist[((a - c.lo) >> shift) * kCopies + lane % kCopies],
-                    (unsigned long long)(COUNT ? 1ull : exponent_weight(a, tbl)));
+      for (int i = tid; i < kSelBins * kCopies; i += kThreads) hist[i] = 0;
+      if (tid == 0) {
+        sh.digit = -1;
+        sh.n = 0;
+        sh.nan = 0;
       }
-    });
-    if (COUNT && first && nan) atomicAdd(&sh.nan, nan);
-    __syncthreads();
-    if (tid < 64) {  // the part of the cut: lane l owns parts 4 l .. 4 l + 3
-      uint64_t b[4], mine = 0;
+      __syncthreads();
+      int nan = 0;
+      for_row8<DT>(p, V, [&](const float(&x)[8], int) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        b[j] = 0;
-#pragma unroll
-        for (int q = 0; q < kCopies; ++q) b[j] += hist[(4 * lane + j) * kCopies + q];
-        mine += b[j];
-      }
-      const uint64_t incl = fg::wave_incl_scan_u64(mine), total = fg::shfl_u64(incl, 63);
-      bool ok = total > 0;
-      uint64_t target = c.rest;
-      if (first) {
-        const uint64_t slots = (uint64_t)max((int)c.rest - sh.nan, 0);
-        ok &= slots > 0;
-        target = (total <= slots ? total : slots) - 1;
-      }
-      if (ok && incl - mine <= target && target < incl) {
-        uint64_t before = incl - mine;
+        for (int j = 0; j < 8; ++j) {
+          const uint32_t a = fixed_exponent(m, x[j], kt);
+          if constexpr (COUNT) nan += x[j] != x[j];
+          if (a - c.lo < width)
+            atomicAdd((unsigned long long*)&hist[((a - c.lo) >> shift) * kCopies + lane % kCopies],
+                      (unsigned long long)(COUNT ? 1ull : exponent_weight(a, tbl)));
+        }
+      });
+      if (COUNT && first && nan) atomicAdd(&sh.nan, nan);
+      __syncthreads();
+      if (tid < 64) {  // the part of the cut: lane l owns parts 4 l .. 4 l + 3
+        uint64_t b[4], mine = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          if (before + b[j] > target) {
-            sh.digit = 4 * lane + j;
-            sh.before = target - before;
-            break;
+          b[j] = 0;
+#pragma unroll
+          for (int q = 0; q < kCopies; ++q) b[j] += hist[(4 * lane + j) * kCopies + q];
+          mine += b[j];
+        }
+        const uint64_t incl = fg::wave_incl_scan_u64(mine), total = fg::shfl_u64(incl, 63);
+        bool ok = total > 0;
+        uint64_t target = c.rest;
+        if (first) {
+          const uint64_t slots = (uint64_t)max((int)c.rest - sh.nan, 0);
+          ok &= slots > 0;
+          target = (total <= slots ? total : slots) - 1;
+        }
+        if (ok && incl - mine <= target && target < incl) {
+          uint64_t before = incl - mine;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if (before + b[j] > target) {
+              sh.digit = 4 * lane + j;
+              sh.before = target - before;
+              break;
+            }
+            before += b[j];
           }
-          before += b[j];
         }
       }
-    }
-    __syncthreads();
-    if (sh.digit < 0) return false;
-    if (first) c.nan = sh.nan;
-    c.rest = sh.before;
-    c.lo += (uint32_t)sh.digit << shift;
-    c.hi = min(c.hi, c.lo + (1u << shift));
+      __syncthreads();
+      if (sh.digit < 0) return false;
+      if (first) c.nan = sh.nan;
+      c.rest = sh.before;
+      c.lo += (uint32_t)sh.digit << shift;
+      c.hi = min(c.hi, c.lo + (1u << shift));
     }
     uint32_t ones = 0, zeros = 0;  // bits in which the keys of the class differ
     list([&](uint32_t a, float x, int) {
@@ -828,7 +827,7 @@ FG_DEVICE bool narrow_cut(const char* p, int V, float m, float kt, const uint64_
 
 // ------------------------------------------------------------------ one workgroup, the row in registers
 // A row of up to 8,192 G logits held by one workgroup, 8 G per thread (element 8 (1024 u + t) + j
-// of thread t): one memory pass and one launch for every kind of draw, by the rule of block_sample.
+// of thread t): one memory pass and one launch for every draw but a greedy one, by the rule of block_sample.
 //  * the maximum;
 //  * top-k / top-p: a histogram over the bins above (counts / q-mass), the bin of the cut, a
 //    list of its elements (top-k: and of those above), the exact cut among them;
@@ -836,8 +835,8 @@ FG_DEVICE bool narrow_cut(const char* p, int V, float m, float kt, const uint64_
 //    target scans its lanes. Top-k draws among its list.
 // Bound by latency: one memory round trip and about 32 G weights per thread between some ten
 // barriers. Against the launches it replaces (three for an unrestricted draw, seven for top-p),
-// a draw of 8 x 32,000 bf16 rows took, us: unrestricted 16.6 -> 10.9, top-p 48.8 -> 31.1, top-k 50
-// 49.0 -> 15.7; of 512 rows 43.2 -> 19.9, 220.7 -> 63.4, 102.0 -> 32.0.
+// a draw of 8 x 32,000 bf16 rows took, us: unrestricted 16.6 -> 10.9, top-p 48.8 -> 30.4, top-k 50
+// 49.0 -> 14.7; of 512 rows 43.2 -> 19.9, 220.7 -> 63.4, 102.0 -> 32.0.
 enum Cut : int { kNoCut, kTopP, kTopK };  // kTopK: with a top-p cut after it or not
 
 template <int CUT>
@@ -1329,8 +1328,8 @@ constexpr int kSplitMaxGroups = 16;
 
 // Load group u of a pass starting at base (elements base + (u * kSplitThreads + t) * 8 ..
 // + 7 of thread t) holds an element before hi. Uniform over the workgroup: a group wholly
-// past the chunk end is neither loaded nor weighed (a 9,504-element chunk is one full pass
-// of 8,192 and one group of the second).
+// past the chunk end is neither loaded nor weighed (the chunk of a 128,256-logit row, 8,016
+// elements, reads four of the kSplitLoads groups).
 FG_DEVICE bool split_group_live(int base, int u, int hi) { return base + u * kSplitThreads * 8 < hi; }
 
 // Chunk maxima (raw maximum, NaN ignored, with KEY the first-maximum rank key, without it the least
@@ -1474,7 +1473,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_sum_kernel(SplitArgs a) {
   split_parts_max(a, r, smax, skey, mx, best);
   const float m = mx, kt = split_kt(a);
   // each group's q-mass: wave sums added into LDS (group g of the chunk = elements
-  // [lo + 2048 g, lo + 2048 (g + 1)) = load group u of pass g / 4)
+  // [lo + 2048 g, lo + 2048 (g + 1)) = load group g % kSplitLoads of pass g / kSplitLoads)
   const bool keep_groups = a.groups <= kSplitMaxGroups;
   int g = 0;
   for (int base = lo; base < hi; base += kSplitPass) {
@@ -2428,7 +2427,8 @@ int sample_tokens_impl(const char* who, const void* logits, int dtype, int64_t r
     return fg::check_launch(who);
   }
   for_row_kernel(dtype, path.groups, sp, [&](auto dt, auto g, auto cut) {
-    hipLaunchKernelGGL((sample_rows_kernel<decltype(dt)::value, decltype(g)::value, decltype(cut)::value>), dim3(rows), dim3(kThreads), 0, s,
+    hipLaunchKernelGGL((sample_rows_kernel<decltype(dt)::value, decltype(g)::value, decltype(cut)::value>),
+                       dim3(rows), dim3(kThreads), 0, s,
                        logits, row_stride, vocab, row_index, forced, noise, noise_stride, noise_col, seed, step,
                        seq_ids, draw, sp, out_tokens);
   });
@@ -2488,7 +2488,8 @@ int fg_accept_walk(const void* tree_logits, int dtype, int64_t row_stride, int v
                      batch, acc_tokens, acc_nodes, acc_stride, acc_len, last_node, correction, workspace);
   for (int t = 0; t < max_walk_steps; ++t) {
     for_row_kernel(dtype, draw_path(vocab, sp, batch, false, false).groups, sp, [&](auto dt, auto g, auto cut) {
-      hipLaunchKernelGGL((walk_step_kernel<decltype(dt)::value, decltype(g)::value, decltype(cut)::value>), dim3(batch), dim3(kThreads), 0, s,
+      hipLaunchKernelGGL((walk_step_kernel<decltype(dt)::value, decltype(g)::value, decltype(cut)::value>),
+                         dim3(batch), dim3(kThreads), 0, s,
                          tree_logits, row_stride, vocab, slot_map, tree_tokens, parents, n_nodes, nmax, batch, t, 0,
                          noise, noise_stride, noise_col0, seed, step, seq_ids, draw0, sp, acc_tokens, acc_nodes,
                          acc_stride, acc_len, last_node, correction, workspace, err_flag, nullptr, nullptr);
@@ -2563,7 +2564,8 @@ int fg_walk_step(const void* step_logits, int dtype, int64_t row_stride, int voc
     return fg::check_launch("fg_walk_step");
   }
   for_row_kernel(dtype, path.groups, sp, [&](auto dt, auto g, auto cut) {
-    hipLaunchKernelGGL((walk_step_kernel<decltype(dt)::value, decltype(g)::value, decltype(cut)::value>), dim3(batch), dim3(kThreads), 0, s,
+    hipLaunchKernelGGL((walk_step_kernel<decltype(dt)::value, decltype(g)::value, decltype(cut)::value>),
+                       dim3(batch), dim3(kThreads), 0, s,
                        step_logits, row_stride, vocab, nullptr, tree_tokens, parents, n_nodes, nmax, batch, walk_step, 1,
                        noise, noise_stride, noise_col0, seed, step, seq_ids, draw0, sp, acc_tokens, acc_nodes,
                        acc_stride, acc_len, last_node, correction, state, err_flag, next_row_index, next_row_active);

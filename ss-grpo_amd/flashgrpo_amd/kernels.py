@@ -690,7 +690,7 @@ def linear_rope_kv_write(x, w_pairs, bias_pairs, *, tile=(64, 64), stages=0, bat
 
 # ------------------------------------------------------------------ sampling / acceptance
 def sample_workspace(rows, device):
-    """Scratch that lets unrestricted / greedy draws run split over several workgroups per row."""
+    """Scratch that lets draws of long rows run split over several workgroups per row."""
     n = _lib.load().fg_sample_workspace(int(rows))
     return torch.empty(n, dtype=torch.uint8, device=device)
 
@@ -784,7 +784,7 @@ def walk_step(walk, step_logits, tree_tokens, parents, n_nodes, *, walk_step, no
     """One walk step: active row b draws from row b of step_logits.
 
     ``parts``: the (part_max, part_key) row maxima that ``lm_head_topk`` wrote with
-    step_logits (an unrestricted / greedy step then needs no chunk-maxima launch). ``next_rows``: also
+    step_logits (a step that splits its rows then needs no chunk-maxima launch). ``next_rows``: also
     fill walk['row_index'] / walk['row_active'] for the next step (as ``walk_rows``)."""
     _dev(step_logits, tree_tokens, parents, n_nodes, noise, seq_ids)
     if parts is not None:
